@@ -222,6 +222,7 @@ int ofx_ctx_destroy(ofx_ctx* c) {
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (void* p : c->allocs) (void)hipFree(p);
+    sweep_free(c);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return 0;

@@ -186,6 +186,8 @@ struct DevFields {
     double *zred = nullptr;     // [nz][RQ_N] per-zone reduced values (several zones only)
 };
 
+struct SweepSet;  // schedule of the pipelined LU-SGS sweeps (ofx_sweep.hip)
+
 }  // namespace ofx
 
 struct ofx_ctx {
@@ -203,6 +205,7 @@ struct ofx_ctx {
     ofx::Consts k{};
     ofx::DevMesh m;
     ofx::HostSched sched;
+    ofx::SweepSet* sweep = nullptr;  // null: the sweeps run level by level
     ofx::DevFields d;
     std::vector<void*> allocs;
     int par_dt = 0, par_lim = 0, par_fix = 0;  // parity of the reduction buffers in use
@@ -633,6 +636,11 @@ int sa_residual(ofx_ctx* c);
 int sa_residual_parts(ofx_ctx* c, unsigned parts);  // bits: gradient, face terms, cell terms
 int ns_lusgs(ofx_ctx* c, int lo_first = 0);
 int fusable_l0(const ofx_ctx* c);
+int sweep_build(ofx_ctx* c, const std::vector<int>& off, const std::vector<int>& nb, const std::vector<int>& id,
+                const std::vector<int>& lev, const std::vector<int>& levU);
+void sweep_free(ofx_ctx* c);
+int pipelined_lusgs_ns(ofx_ctx* c);
+int pipelined_lusgs_sa(ofx_ctx* c);
 int sa_lusgs(ofx_ctx* c, int lo_first = 0);
 int ns_update(ofx_ctx* c);
 int sa_update(ofx_ctx* c);

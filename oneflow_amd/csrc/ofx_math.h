@@ -136,4 +136,23 @@ OFX_HD double ofx_pow(double x, double y) {
     return exp_dd(zz.hi, zz.lo);
 }
 
+// a / b, correctly rounded, with y = div_reciprocal(b) at hand: one product and
+// two remainder steps in place of the compiler's division (Markstein: with y
+// the correctly rounded reciprocal and q within one ulp of a / b, fma(a - b q,
+// y, q) is the correctly rounded quotient; the first step brings q there).
+// Exact while no step can under- or overflow, which div_by_ok tells (b was
+// checked by div_reciprocal, 0 otherwise); a zero keeps its sign.
+constexpr double DIV_A = 4.149515568880993e180, DIV_B = 2.037035976334486e90;  // 2^600, 2^300
+OFX_HD double div_reciprocal(double b) { return (b > 1.0 / DIV_B && b < DIV_B) ? 1.0 / b : 0.0; }
+OFX_HD bool div_by_ok(double a, double y) {
+    const double m = fabs(a);
+    return y != 0.0 && ((m > 1.0 / DIV_A && m < DIV_A) || m == 0.0);
+}
+OFX_HD double div_by(double a, double b, double y) {
+    double q = a * y;
+    q = fma(fma(-b, q, a), y, q);
+    q = fma(fma(-b, q, a), y, q);
+    return a == 0.0 ? a : q;
+}
+
 }  // namespace ofxm

@@ -7,7 +7,7 @@
 // list in ascending face id, which is the order the reference's serial
 // scatter AddF2CField (codes/usolver/src/UCom.cpp:144-171) adds into a cell,
 // so the FP64 residual is the reference's bit for bit and no atomics are used.
-#include "ofx_physics.h"
+#include "ofx_lusgs.h"
 
 namespace ofx {
 
@@ -278,24 +278,6 @@ __global__ void __launch_bounds__(TB) k_ns_qext(DevMesh m, DevFields d, int par_
     else slot_reduce<10, true>(ext, d.slots, par_lim, RQ_N, RQ_QMIN);
 }
 
-
-// Time step after UTimeStep::ModifyTimeStep (codes/uns/src/UTimeStep.cpp:368-381)
-// and the LU-SGS diagonal of UNsSpectrum::CalcImplicitSpectrum
-// (codes/uns/src/UNsSpectrum.cpp:52-94, sp2 = 1), evaluated where consumed.
-__device__ __forceinline__ double clamped_dt(const DevFields& d, const Consts& k, int i, double mindt) {
-    double dt = d.timestep[i];
-    if (k.max_time_ratio > 0) {
-        double mp = k.max_time_ratio * mindt;
-        dt = (dt < mp) ? dt : mp;
-    }
-    return dt;
-}
-__device__ __forceinline__ double ns_impsr(const DevMesh& m, const DevFields& d, const Consts& k, int i, double mindt) {
-    double imp = (1.0 / clamped_dt(d, k, i, mindt)) * m.vol[i];
-    imp += d.invsr[i];
-    imp += d.vissr[i];
-    return imp;
-}
 
 // Materialise the clamped time step and the LU-SGS diagonal as fields
 // (for download; the solver evaluates them where they are consumed).
@@ -939,85 +921,6 @@ int fill_ghost_grad(ofx_ctx* c) {
 
 // ============================================================ LU-SGS
 
-// UNsLusgs::Solve for face f seen from cell i: GCom::SetGeometry orientation,
-// PrepareData/PrepareDataFacePrim, NsLusgs::GetStandardFluxIncrement(-1) with
-// CalcFaceEigenValue and CalcDH, then CalcViscousTerm and AddFluxIncrement
-// (codes/uns/src/UNsLusgs.cpp:189-335, codes/ns/src/NsLusgs.cpp:121-228,340-368).
-// The face term of UNsLusgs::Solve for cell i = l (after GCom::SetGeometry
-// has put i on the left): the split flux increment of the neighbour r and,
-// with viscosity, its viscous radius.  Own state (rl..pl) and neighbour data
-// are passed in, loaded by the caller.
-// VM: the viscous term of the face, 0 none (inviscid), 1 spectral-radius
-// model 1 (neighbour volume), 2 models 2 and 3 (centre distance) -- a
-// compile-time choice, so a face evaluates only its own model.
-template <int VM>
-__device__ __forceinline__ void ns_lusgs_face(const Consts& k, double xfn, double yfn, double zfn, double vfn,
-                                              double farea, double rl, double ul, double vl, double wl, double pl,
-                                              const double* pj, const double* dqj, double visl, double vist,
-                                              double volr, double dist, double* rhs0) {
-    double rr = pj[0], ur = pj[1], vr = pj[2], wr = pj[3], pr = pj[4];
-    double gl = k.gama, gr = k.gama;
-    double hl = gl / (gl - 1.0) * pl / rl + 0.5 * sqr3(ul, vl, wl);
-    double hr = gr / (gr - 1.0) * pr / rr + 0.5 * sqr3(ur, vr, wr);
-    double tmp0 = sqrt(rr / rl);
-    double tmp1 = 1.0 / (1.0 + tmp0);
-    double rm = sqrt(rr * rl);
-    double um = (ul + ur * tmp0) * tmp1;
-    double vm = (vl + vr * tmp0) * tmp1;
-    double wm = (wl + wr * tmp0) * tmp1;
-    double hm = (hl + hr * tmp0) * tmp1;
-    double pm = rm * (hm - 0.5 * sqr3(um, vm, wm)) * (gl - 1.0) / gl;
-    double gama = k.gama;
-    double c2f = dabs(gama * pm / rm);
-    double cmf = sqrt(c2f);
-    double vnf = xfn * um + yfn * vm + zfn * wm;
-    double lmdF = dabs(vnf - vfn) + cmf;
-    double c2 = dabs(gama * pj[4] / pj[0]);
-    double cm = sqrt(c2);
-    double vn_fluid = xfn * pj[1] + yfn * pj[2] + zfn * pj[3];
-    double vn_rel = vn_fluid - vfn;
-    double lmd1 = 0.5 * (vn_rel + -1.0 * lmdF);
-    double lmd2 = 0.5 * ((vn_rel + cm) + -1.0 * lmdF);
-    double lmd3 = 0.5 * ((vn_rel - cm) + -1.0 * lmdF);
-    double x1 = (lmd1 + lmd1 - lmd2 - lmd3) / (c2 + c2);
-    double x2 = (lmd2 - lmd3) / (cm + cm);
-    double dc = vn_fluid * dqj[0] - xfn * dqj[1] - yfn * dqj[2] - zfn * dqj[3];
-    double c2dc = c2 * dc;
-    double v2 = sqr3(pj[1], pj[2], pj[3]);
-    double ae = gama - 1.0;
-    double af = 0.5 * ae * v2;
-    double dh = -ae * (pj[1] * dqj[1] + pj[2] * dqj[2] + pj[3] * dqj[3] - dqj[4]);
-    double enth = (gama / (gama - 1.0)) * (pj[4] / pj[0]);
-    dh += af * dqj[0];
-    double hmj = enth + 0.5 * v2;
-    double term1 = dh * x1 + dc * x2;
-    double term2 = c2dc * x1 + dh * x2;
-    double dfj[5];
-    dfj[0] = lmd1 * dqj[0] - term1;
-    dfj[1] = lmd1 * dqj[1] - pj[1] * term1 + xfn * term2;
-    dfj[2] = lmd1 * dqj[2] - pj[2] * term1 + yfn * term2;
-    dfj[3] = lmd1 * dqj[3] - pj[3] * term1 + zfn * term2;
-    dfj[4] = lmd1 * dqj[4] - hmj * term1 + vn_fluid * term2;
-    for (int e = 0; e < 5; ++e) dfj[e] *= farea;
-    if (VM != 0) {
-        double visrad;
-        if (VM == 1) {
-            double density = 0.5 * (rl + rr);
-            double c1 = 4.0 / 3.0 * (visl + vist);
-            double cc2 = k.gama * (visl * k.oprl + vist * k.oprt);
-            double c3 = 2.0 * dmax(c1, cc2) / (k.reynolds * density);
-            visrad = (farea * farea) * c3 / volr;
-        } else {
-            double viscosity = visl + vist;
-            double density = 0.5 * (rl + rr);
-            double c1 = 2.0 * viscosity / (density * dist * k.reynolds + SMALL);
-            visrad = 0.5 * c1 * farea;
-        }
-        for (int e = 0; e < 5; ++e) rhs0[e] -= visrad * dqj[e];
-    }
-    for (int e = 0; e < 5; ++e) rhs0[e] += dfj[e];
-}
-
 // One cell of the lower (UPPER=false) or upper sweep.  Boundary faces are
 // skipped in both sweeps: their ghost increment is zero, so the reference's
 // upper-sweep contribution through them is exactly +0.  The cell's faces are
@@ -1095,21 +998,6 @@ __device__ __forceinline__ void ns_lusgs_cell(const DevMesh& m, const DevFields&
     }
 }
 
-// Whole sweep in one workgroup: levels in order, a workgroup barrier between
-// levels (every cell of a level depends only on earlier levels).
-template <bool UPPER, int MAXF, int VM, bool EN>
-__global__ void __launch_bounds__(1024) k_ns_sweep_1wg(DevMesh m, DevFields d, Consts k, int par) {
-    double mindt = slot_result<false>(d.slots, par, m.nz * RQ_N, RQ_DTMIN);
-    const int* off = UPPER ? m.upOff : m.loOff;
-    const int* ord = UPPER ? m.upOrder : m.loOrder;
-    int nl = UPPER ? m.nLevUp : m.nLevLo;
-    for (int L = 0; L < nl; ++L) {
-        for (int idx = off[L] + threadIdx.x; idx < off[L + 1]; idx += blockDim.x)
-            ns_lusgs_cell<UPPER, MAXF, VM, EN>(m, d, k, ord[idx], mindt);
-        __syncthreads();
-    }
-}
-
 // One level per launch (wide levels on large meshes).
 // base >= 0: the level's cells are base, base + 1, ... (no order lookup).
 template <bool UPPER, int MAXF, int VM, bool EN>
@@ -1127,37 +1015,24 @@ __global__ void __launch_bounds__(TB) k_ns_sweep_level(DevMesh m, DevFields d, C
     ns_lusgs_cell<UPPER, MAXF, VM, EN>(m, d, k, i, mindt, live);
 }
 
-// Launch policy: few wide levels (multicolour numbering) -> one grid-wide
-// launch per level; many narrow levels (natural numbering) -> one workgroup
-// walking all levels.
-bool use_level_launches(const std::vector<int>& off) {
-    int nl = (int)off.size() - 1;
-    return nl <= 64;
-}
-
 template <int MAXF, int VM, bool EN>
 static void launch_lusgs(ofx_ctx* c, int lo_first) {
     const DevMesh& m = c->m;
     for (int pass = 0; pass < 2; ++pass) {
         bool up = pass == 1;
         const std::vector<int>& off = up ? c->sched.upOff : c->sched.loOff;
-        if (!use_level_launches(off)) {
-            if (up) k_ns_sweep_1wg<true, MAXF, VM, EN><<<1, 1024, 0, c->stream>>>(m, c->d, c->k, c->par_dt);
-            else k_ns_sweep_1wg<false, MAXF, VM, EN><<<1, 1024, 0, c->stream>>>(m, c->d, c->k, c->par_dt);
-        } else {
-            const std::vector<int>& base = up ? c->sched.upBase : c->sched.loBase;
-            // upper level 0 holds the cells without a higher neighbour: their
-            // increment is dq += (-0)/D, which leaves dq unchanged bit for bit
-            for (size_t L = up ? 1 : (size_t)lo_first; L + 1 < off.size(); ++L) {
-                int b = off[L], e = off[L + 1];
-                if (e <= b) continue;
-                if (up)
-                    k_ns_sweep_level<true, MAXF, VM, EN><<<nblk(e - b), TB, 0, c->stream>>>(m, c->d, c->k, b, e, base[L],
-                                                                                       c->par_dt);
-                else
-                    k_ns_sweep_level<false, MAXF, VM, EN><<<nblk(e - b), TB, 0, c->stream>>>(m, c->d, c->k, b, e, base[L],
-                                                                                        c->par_dt);
-            }
+        const std::vector<int>& base = up ? c->sched.upBase : c->sched.loBase;
+        // upper level 0 holds the cells without a higher neighbour: their
+        // increment is dq += (-0)/D, which leaves dq unchanged bit for bit
+        for (size_t L = up ? 1 : (size_t)lo_first; L + 1 < off.size(); ++L) {
+            int b = off[L], e = off[L + 1];
+            if (e <= b) continue;
+            if (up)
+                k_ns_sweep_level<true, MAXF, VM, EN><<<nblk(e - b), TB, 0, c->stream>>>(m, c->d, c->k, b, e, base[L],
+                                                                                   c->par_dt);
+            else
+                k_ns_sweep_level<false, MAXF, VM, EN><<<nblk(e - b), TB, 0, c->stream>>>(m, c->d, c->k, b, e, base[L],
+                                                                                    c->par_dt);
         }
     }
 }
@@ -1179,11 +1054,12 @@ static void launch_lusgs_vm(ofx_ctx* c, int lo_first) {
 // per level.  Returns loOff[1], or 0.
 int fusable_l0(const ofx_ctx* c) {
     const HostSched& h = c->sched;
-    if (!use_level_launches(h.loOff) || h.loBase.empty() || h.loBase[0] != 0) return 0;
+    if (c->sweep || h.loBase.empty() || h.loBase[0] != 0) return 0;
     return h.loOff[1];
 }
 
 int ns_lusgs(ofx_ctx* c, int lo_first) {
+    if (c->sweep) return pipelined_lusgs_ns(c);
     int mf = c->m.maxFacesPerCell;
     if (mf <= 4) launch_lusgs_vm<4>(c, lo_first);
     else if (mf <= 6) launch_lusgs_vm<6>(c, lo_first);

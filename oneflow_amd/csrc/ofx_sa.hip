@@ -5,8 +5,6 @@
 
 namespace ofx {
 
-bool use_level_launches(const std::vector<int>& off);
-
 constexpr int TBS = 256;
 static inline int nblks(int n) { return (n + TBS - 1) / TBS; }
 
@@ -479,18 +477,6 @@ __device__ __forceinline__ void sa_lusgs_cell(const DevMesh& m, const DevFields&
 }
 
 template <bool UPPER, int MAXF>
-__global__ void __launch_bounds__(1024) k_sa_sweep_1wg(DevMesh m, DevFields d) {
-    const int* off = UPPER ? m.upOff : m.loOff;
-    const int* ord = UPPER ? m.upOrder : m.loOrder;
-    int nl = UPPER ? m.nLevUp : m.nLevLo;
-    for (int L = 0; L < nl; ++L) {
-        for (int idx = off[L] + threadIdx.x; idx < off[L + 1]; idx += blockDim.x)
-            sa_lusgs_cell<UPPER, MAXF>(m, d, ord[idx]);
-        __syncthreads();
-    }
-}
-
-template <bool UPPER, int MAXF>
 __global__ void __launch_bounds__(TBS) k_sa_sweep_level(DevMesh m, DevFields d, int b, int e, int base) {
     int idx = b + blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= e) return;
@@ -504,24 +490,20 @@ static void launch_sa_lusgs(ofx_ctx* c, int lo_first) {
     for (int pass = 0; pass < 2; ++pass) {
         bool up = pass == 1;
         const std::vector<int>& off = up ? c->sched.upOff : c->sched.loOff;
-        if (!use_level_launches(off)) {
-            if (up) k_sa_sweep_1wg<true, MAXF><<<1, 1024, 0, c->stream>>>(m, c->d);
-            else k_sa_sweep_1wg<false, MAXF><<<1, 1024, 0, c->stream>>>(m, c->d);
-        } else {
-            const std::vector<int>& base = up ? c->sched.upBase : c->sched.loBase;
-            // upper level 0: no higher neighbour, turbdq += (-0)/D changes nothing
-            for (size_t L = up ? 1 : (size_t)lo_first; L + 1 < off.size(); ++L) {
-                int b = off[L], e = off[L + 1];
-                if (e <= b) continue;
-                if (up) k_sa_sweep_level<true, MAXF><<<nblks(e - b), TBS, 0, c->stream>>>(m, c->d, b, e, base[L]);
-                else k_sa_sweep_level<false, MAXF><<<nblks(e - b), TBS, 0, c->stream>>>(m, c->d, b, e, base[L]);
-            }
+        const std::vector<int>& base = up ? c->sched.upBase : c->sched.loBase;
+        // upper level 0: no higher neighbour, turbdq += (-0)/D changes nothing
+        for (size_t L = up ? 1 : (size_t)lo_first; L + 1 < off.size(); ++L) {
+            int b = off[L], e = off[L + 1];
+            if (e <= b) continue;
+            if (up) k_sa_sweep_level<true, MAXF><<<nblks(e - b), TBS, 0, c->stream>>>(m, c->d, b, e, base[L]);
+            else k_sa_sweep_level<false, MAXF><<<nblks(e - b), TBS, 0, c->stream>>>(m, c->d, b, e, base[L]);
         }
     }
 }
 
 int sa_lusgs(ofx_ctx* c, int lo_first) {
     if (c->k.vismodel != 3) return 0;
+    if (c->sweep) return pipelined_lusgs_sa(c);
     int mf = c->m.maxFacesPerCell;
     if (mf <= 4) launch_sa_lusgs<4>(c, lo_first);
     else if (mf <= 6) launch_sa_lusgs<6>(c, lo_first);
