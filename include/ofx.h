@@ -286,33 +286,33 @@ int ofx_zones_norms(ofx_ctx* ctx, ofx_norms* out);
 int ofx_zones_aero(ofx_ctx* ctx, double* out);
 
 /* Face-kernel tile, the threads per block of the NS and SA face-flux kernels:
- * 64, 128, 256 (default) or 512.  Results do not depend on it (no
- * counterpart in the reference; a launch parameter). */
+ * 64, 128, 256 or 512 (default: 64 on grids of fewer than 131,072 faces, 256
+ * otherwise).  Results do not depend on it (no counterpart in the reference;
+ * a launch parameter). */
 int ofx_set_face_tile(ofx_ctx* ctx, int ns_tile, int sa_tile);
 
 /* Kernel variant (no counterpart in the reference; results do not depend on
  * it).  Kernels 0 and 1 both name the NS gradient kernel (it evaluates the
- * limiter in the same pass), kernel 5 the SA gradient: variant 0 (default)
+ * limiter in the same pass), kernel 5 the SA gradient: variant 0
  * reads the face terms (weights, normal, face centre offsets) by face id,
- * variant 1 reads the per-(cell, face) copies stored cell-major at mesh
+ * variant 1 (default) reads the per-(cell, face) copies stored cell-major at mesh
  * upload (64 bytes per cell face), contiguous per wave.  kernel 6, the NS
- * time step and LU-SGS sweeps: variant 0 (default) reads the faces' normals
+ * time step and LU-SGS sweeps: variant 0 reads the faces' normals
  * and areas by face id and evaluates the viscous radius's centre distance,
- * variant 1 reads per-(cell, face) copies of the normal, area, distance and
+ * variant 1 (default) reads per-(cell, face) copies of the normal, area, distance and
  * neighbour volume (48 bytes per cell face).  kernel 2, the residual
  * gather: variant 0 one lane per face of a cell, variant 1 (default) one
  * thread per cell.  kernel 3, the viscous FP64 NS face kernel: variant 0
  * (default) one thread per face, variant 1 two waves per 64 faces (inviscid
  * / viscous part).  kernel 4, the SA face kernel with the TEST diffusion
- * (iturb_visflux 2): variant 0 (default) reads the face's stored geometry
- * record, variant 1 evaluates it from the cell and face centres. */
+ * (iturb_visflux 2): variant 0 reads the face's stored geometry
+ * record, variant 1 (default) evaluates it from the cell and face centres. */
 int ofx_set_kernel_variant(ofx_ctx* ctx, int kernel, int variant);
 int ofx_get_kernel_variant(ofx_ctx* ctx, int kernel, int* variant);
 
 /* Autotuner (no counterpart in the reference): times the NS face kernel for
- * each face tile and split, the gather, both gradients and (LU-SGS runs)
- * the NS time step with the sweeps for each variant, and the SA residual for
- * each SA face tile and geometry variant on the current state (each the
+ * each face tile and split, the gather and both gradients for each variant,
+ * and the SA residual for each SA face tile and geometry variant on the current state (each the
  * median of five timings of `iters` launches), keeps the fastest, and
  * reports the face tiles in chosen2[0..1] (may be NULL).
  * Leaves res / turbres as one evaluation of the current state. */

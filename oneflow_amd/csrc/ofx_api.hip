@@ -705,20 +705,6 @@ int ofx_autotune(ofx_ctx* c, int iters, int* chosen2) {
         if (ms < best) { best = ms; pick = v; }
     }
     c->grad_variant = pick;
-    // the NS time step's and sweeps' face normals (parts 11 and 12, on the
-    // time step and residual of the current state)
-    if (c->cfg.time_integral == 0) {
-        best = 1e300;
-        pick = c->normal_variant;
-        for (int v = 0; v < 2; ++v) {
-            c->normal_variant = v;
-            double ms2 = 0;
-            OFX_TRY(median_ms(c, 11, iters, &ms));
-            OFX_TRY(median_ms(c, 12, iters, &ms2));
-            if (ms + ms2 < best) { best = ms + ms2; pick = v; }
-        }
-        c->normal_variant = pick;
-    }
     if (c->k.vismodel == 3) {
         // the same choice for the SA gradient (part 6)
         best = 1e300;
@@ -754,7 +740,7 @@ int ofx_autotune(ofx_ctx* c, int iters, int* chosen2) {
     OFX_TRY(ns_residual(c));
     if (c->k.vismodel == 3) OFX_TRY(sa_residual(c));
     OFX_HIP(hipStreamSynchronize(c->stream));
-    if (chosen2) { chosen2[0] = c->face_tb; chosen2[1] = c->saface_tb; }
+    if (chosen2) { chosen2[0] = c->face_tb; chosen2[1] = face_tile(c->saface_tb, c->m.F); }
     return 0;
 }
 

@@ -213,16 +213,25 @@ struct ofx_ctx {
     // its value when the limiter's grid extrema were last reduced (by the
     // time step or k_ns_qext), so a residual of the same state reuses them
     int qgen = 0, qext_gen = -1;
-    int face_tb = 256, saface_tb = 256;        // face-kernel tile (threads per block)
+    // Launch forms (results do not depend on them; ofx_set_kernel_variant,
+    // ofx_set_face_tile and ofx_autotune change them).  The defaults are the
+    // forms that won on every grid measured, 2-D of 11k-168k cells and 3-D of
+    // 148k-2.5M cells, in either numbering: per-entry copies of the face terms
+    // against reads by face id (us at 120,832 cells in 2-D and 2,524,160 in
+    // 3-D: gradient 15.8 -> 13.1 and 403 -> 310, SA gradient 5.3 -> 4.2 and 172
+    // -> 119, time step and sweeps 62.5 -> 57.9 and 1026 -> 917), one thread
+    // per cell in the gather (9.8 -> 5.5, 455 -> 173), the TEST geometry
+    // evaluated from the centres (9.6 -> 8.7, 306 -> 196).
+    int face_tb = 0, saface_tb = 0;            // face-kernel tile (threads per block), 0: face_tile's rule
     int gather_variant = 1;  // residual gather: 0 lanes per cell, 1 one thread per cell
-    int sa_geom_variant = 0;  // SA diffusion, TEST method: 0 stored face records, 1 evaluated from the centres
+    int sa_geom_variant = 1;  // SA diffusion, TEST method: 0 stored face records, 1 evaluated from the centres
     int face_split = 0;      // viscous NS face kernel: 1 inviscid and viscous parts on separate waves
     // cell gradients (NS gradient with limiter; SA gradient): 0 face terms
     // read by face id (fgg / frec / fz), 1 the per-entry copies (DevMesh::ellg)
-    int grad_variant = 0, sagrad_variant = 0;
+    int grad_variant = 1, sagrad_variant = 1;
     // NS time step and LU-SGS sweeps: 0 face normals and areas read by face
     // id, 1 the per-entry copies (DevMesh::ellg plane 2)
-    int normal_variant = 0;
+    int normal_variant = 1;
     int gen = 0;  // bumped whenever launch parameters change (mesh, config, tiles)
     bool dist_valid = false;  // wall distance computed for the current mesh / zones
     int fuse_l0 = 0;  // > 0 while a full step fuses the first lower-sweep level into the gathers
@@ -232,6 +241,13 @@ struct ofx_ctx {
     std::vector<ofx::ZoneK> zkh;
     std::vector<ofx_config> zcfg;
 };
+
+namespace ofx {
+// Threads per block of a face kernel over F faces.  256 unless that leaves
+// fewer than two blocks per CU: 64 then spreads the faces over all of them
+// (11,264 cells: 6.2 -> 5.1 us, 46,080: 9.0 -> 7.6; 120,832 and more: the same).
+inline int face_tile(int set, int F) { return set ? set : F < 2 * 256 * 256 ? 64 : 256; }
+}  // namespace ofx
 
 #define OFX_HIP(call)                                                              \
     do {                                                                           \

@@ -788,7 +788,7 @@ __global__ void __launch_bounds__(TB) k_ns_gather(DevMesh m, DevFields d) {
 
 template <int DIM, int LIM, bool SLAU2>
 static void launch_face(ofx_ctx* c, bool visc) {
-    const int tb = c->face_tb;  // face tile, chosen by ofx_autotune
+    const int tb = face_tile(c->face_tb, c->m.F);
     int nb = (c->m.F + tb - 1) / tb;
     if (visc && c->face_split && !c->k.flux_fp32) {
         k_ns_face<DIM, LIM, SLAU2, true, false, true><<<(c->m.F + 63) / 64, 128, 0, c->stream>>>(c->m, c->d, c->k, 64);

@@ -412,11 +412,11 @@ static void launch_sa(ofx_ctx* c, unsigned parts) {
         else k_sa_grad<DIM, MAXF><<<nblks(m.C), TBS, 0, c->stream>>>(m, c->d, c->k);
     }
     if (parts & 2u) {
-        const int nb = (m.F + c->saface_tb - 1) / c->saface_tb;
+        const int tb = face_tile(c->saface_tb, m.F), nb = (m.F + tb - 1) / tb;
         if (c->sa_geom_variant == 1 && c->k.iturb_visflux == 2)
-            k_sa_face<DIM, 1><<<nb, c->saface_tb, 0, c->stream>>>(m, c->d, c->k, c->saface_tb);
+            k_sa_face<DIM, 1><<<nb, tb, 0, c->stream>>>(m, c->d, c->k, tb);
         else
-            k_sa_face<DIM, 0><<<nb, c->saface_tb, 0, c->stream>>>(m, c->d, c->k, c->saface_tb);
+            k_sa_face<DIM, 0><<<nb, tb, 0, c->stream>>>(m, c->d, c->k, tb);
     }
     if (parts & 4u) k_sa_cell<MAXF><<<nblks(m.C), TBS, 0, c->stream>>>(m, c->d, c->k, c->par_dt, c->fuse_l0);
 }
