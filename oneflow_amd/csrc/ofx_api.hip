@@ -44,6 +44,23 @@ __global__ void k_fill_field(double* p, long n, double v) {
     if (i < n) p[i] = v;
 }
 
+// Room for the norms or forces of nz zones in pinned host memory.
+static int host_sums(ofx_ctx* c, int nz) {
+    if (nz <= c->hsum_n) return 0;
+    nz = std::max(nz, 64);  // (one page holds 85)
+    if (c->hsum) (void)hipHostFree(c->hsum);
+    c->hsum = nullptr;
+    c->hsum_n = 0;
+    void* p = nullptr;
+    if (hipHostMalloc(&p, sizeof(double) * 6 * (size_t)nz, hipHostMallocDefault) != hipSuccess) {
+        set_error("out of pinned host memory");
+        return OFX_ENOMEM;
+    }
+    c->hsum = static_cast<double*>(p);
+    c->hsum_n = nz;
+    return 0;
+}
+
 static int alloc_fields(ofx_ctx* c) {
     const size_t T = c->m.T, F = c->m.F, C = c->m.C;
     DevFields& d = c->d;
@@ -69,7 +86,8 @@ static int alloc_fields(ofx_ctx* c) {
     OFX_TRY(A(&d.visflux, 5 * F));
     OFX_TRY(A(&d.saface, 5 * F));
     OFX_TRY(A(&d.red, 16));
-    OFX_TRY(A(&d.norms, 8 + 6 * 512));
+    OFX_TRY(A(&d.norms, 6 * 512));
+    OFX_TRY(host_sums(c, 1));
     OFX_TRY(alloc_bytes(c, (void**)&d.slots, 2 * 12 * NSLOT * sizeof(unsigned long long)));
     // identity values in both parity buffers: min-reduced quantity 0 starts at LARGE, the others at +0
     for (int p = 0; p < 2; ++p)
@@ -223,6 +241,7 @@ int ofx_ctx_destroy(ofx_ctx* c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (void* p : c->allocs) (void)hipFree(p);
     sweep_free(c);
+    if (c->hsum) (void)hipHostFree(c->hsum);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return 0;
@@ -559,13 +578,13 @@ int ofx_wall_data(ofx_ctx* c, double* out) {
 int ofx_aero(ofx_ctx* c, double* out4) {
     CHECK_READY(c);
     if (!out4) { set_error("null out"); return OFX_EINVAL; }
-    return aero(c, out4);
+    return aero(c, 1, out4);
 }
 
 int ofx_aero_row(ofx_ctx* c, double* out12) {
     CHECK_READY(c);
     if (!out12) { set_error("null out"); return OFX_EINVAL; }
-    return aero_row_zone(c, 0, out12);
+    return aero_row(c, out12);
 }
 
 int ofx_time_kernel(ofx_ctx* c, int which, int iters, double* ms_out) {
@@ -802,6 +821,10 @@ int ofx_zones_set(ofx_ctx* c, int n, const int* cellStart, const int* bfaceStart
     OFX_TRY(upload(c, m.zface, zface.data(), sizeof(int) * F));
     OFX_TRY(upload(c, m.zwall, zwall.data(), sizeof(int) * (n + 1)));
     OFX_TRY(upload(c, zk, c->zkh.data(), sizeof(ZoneK) * n));
+    OFX_TRY(A((void**)&c->zcells, sizeof(int) * (n + 1)));
+    OFX_TRY(upload(c, c->zcells, cellStart, sizeof(int) * (n + 1)));
+    OFX_TRY(A((void**)&c->d.norms, sizeof(double) * 6 * 512 * (size_t)n));
+    OFX_TRY(host_sums(c, n));
     m.zk = zk;
     // per-zone reduction slots (both parities; the min quantity starts at LARGE) and results
     DevFields& d = c->d;
@@ -827,16 +850,13 @@ int ofx_zones_set(ofx_ctx* c, int n, const int* cellStart, const int* bfaceStart
 int ofx_zones_norms(ofx_ctx* c, ofx_norms* out) {
     CHECK_READY(c);
     if (!out) { set_error("null out"); return OFX_EINVAL; }
-    if (c->m.nz == 1) return norms(c, out);
-    for (int z = 0; z < c->m.nz; ++z) OFX_TRY(norms_range(c, c->zc[z], c->zc[z + 1], out + z));
-    return 0;
+    return norms(c, out, true);
 }
 
 int ofx_zones_aero(ofx_ctx* c, double* out) {
     CHECK_READY(c);
     if (!out) { set_error("null out"); return OFX_EINVAL; }
-    for (int z = 0; z < c->m.nz; ++z) OFX_TRY(aero_zone(c, z, out + 4 * z));
-    return 0;
+    return aero(c, c->m.nz, out);
 }
 
 // Bandwidth reference: one 16-byte load and store per thread.

@@ -181,7 +181,7 @@ struct DevFields {
     double *visflux = nullptr;  // [5][F]
     double *saface = nullptr;   // [5][F]: radius, matrix_l, matrix_r, conv flux, diff flux
     double *red = nullptr;      // reduction results (see RED_* in ofx_ns.hip)
-    double *norms = nullptr;    // [6] residual norm accumulators
+    double *norms = nullptr;    // [nz][6][512] residual norm partials
     unsigned long long *slots = nullptr;  // [2 parities][nz][RQ_N][NSLOT] grid-reduction slots
     double *zred = nullptr;     // [nz][RQ_N] per-zone reduced values (several zones only)
 };
@@ -208,6 +208,9 @@ struct ofx_ctx {
     ofx::SweepSet* sweep = nullptr;  // null: the sweeps run level by level
     ofx::DevFields d;
     std::vector<void*> allocs;
+    double* hsum = nullptr;  // pinned host memory the norm and force kernels write: [6 nz]
+    int hsum_n = 0;
+    int* zcells = nullptr;   // several zones: cell starts on the device (nz + 1)
     int par_dt = 0, par_lim = 0, par_fix = 0;  // parity of the reduction buffers in use
     // qgen counts host calls that may change the primitive state; qext_gen is
     // its value when the limiter's grid extrema were last reduced (by the
@@ -660,13 +663,11 @@ int pipelined_lusgs_sa(ofx_ctx* c);
 int sa_lusgs(ofx_ctx* c, int lo_first = 0);
 int ns_update(ofx_ctx* c);
 int sa_update(ofx_ctx* c);
-int norms(ofx_ctx* c, ofx_norms* out);
+int norms(ofx_ctx* c, ofx_norms* out, bool zones = false);
 int nan_stop(ofx_ctx* c);
 int wall_distance(ofx_ctx* c);
 inline int ensure_dist(ofx_ctx* c) { return c->dist_valid ? 0 : wall_distance(c); }
-int norms_range(ofx_ctx* c, int c0, int c1, ofx_norms* out);
-int aero_zone(ofx_ctx* c, int z, double* out4);
-int aero_row_zone(ofx_ctx* c, int z, double* out12);
+int aero_row(ofx_ctx* c, double* out12);
 int wall_data(ofx_ctx* c, double* host_out);
 int fill_ghost_grad(ofx_ctx* c);
 int materialize_timestep(ofx_ctx* c);
@@ -683,7 +684,7 @@ inline DevFields update_fields(const ofx_ctx* c) {
     if (c->cfg.time_integral == 1) { d.dq = d.res; d.turbdq = d.turbres; }
     return d;
 }
-int aero(ofx_ctx* c, double* out4);
+int aero(ofx_ctx* c, int nz, double* out);
 int init_freestream(ofx_ctx* c);
 
 }  // namespace ofx

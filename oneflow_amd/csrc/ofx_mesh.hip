@@ -752,11 +752,7 @@ int mesh_build(ofx_ctx* c, const double* x, const double* y, const double* z, co
     }
     k_face_vis_static<<<(F + TB - 1) / TB, TB, 0, c->stream>>>(m);
     OFX_HIP(hipGetLastError());
-    {
-        std::vector<int> ls(C), us(C);  // levels by storage cell
-        for (int sc = 0; sc < C; ++sc) { ls[sc] = lev[cinv[sc]]; us[sc] = levU[cinv[sc]]; }
-        OFX_TRY(sweep_build(c, off, c2n, cinv, ls, us));
-    }
+    OFX_TRY(sweep_build(c, off, c2n, cinv, lev, levU));
     // the wall distance is computed on first use (ensure_dist): a mesh that
     // is declared as several zones next searches each zone's walls only
     c->dist_valid = false;

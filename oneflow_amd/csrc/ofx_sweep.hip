@@ -607,11 +607,14 @@ int pipelined_lusgs_sa(ofx_ctx* c) {
 static bool use_pipeline(int C, int nlev) { return nlev > 8 && C / nlev < 3000; }
 
 // Build the pipelined schedule of a mesh that profits from it (at the mesh
-// upload; c->sweep stays empty otherwise and the level kernels run).
+// upload; c->sweep stays empty otherwise and the level kernels run).  id: grid
+// id of each storage cell; lev, levU: levels by grid id.
 int sweep_build(ofx_ctx* c, const std::vector<int>& off, const std::vector<int>& nb, const std::vector<int>& id,
                 const std::vector<int>& lev, const std::vector<int>& levU) {
     const int C = c->m.C;
     if (!use_pipeline(C, std::max(c->m.nLevLo, c->m.nLevUp)) || c->m.maxFacesPerCell > 16) return 0;
+    std::vector<int> level[2] = {std::vector<int>(C), std::vector<int>(C)};  // by storage cell
+    for (int sc = 0; sc < C; ++sc) { level[0][sc] = lev[id[sc]]; level[1][sc] = levU[id[sc]]; }
     // dependencies per cell in either direction, which size the ring
     int ne = 1;
     for (int sc = 0; sc < C; ++sc) {
@@ -628,7 +631,7 @@ int sweep_build(ofx_ctx* c, const std::vector<int>& off, const std::vector<int>&
     for (int k = 0; k < 2; ++k) {
         bool fits = false;
         for (int R = SW_RMAX; R >= SW_RMIN && !fits; R = R * 3 / 4) {
-            if (!build_sweep_plan(C, off, nb, id, k ? levU : lev, k == 1, R, SW_WIDTH, P[k])) return 0;
+            if (!build_sweep_plan(C, off, nb, id, level[k], k == 1, R, SW_WIDTH, P[k])) return 0;
             G[k][0] = sweep_groups(P[k], Shape<5>::CPG, Shape<5>::NW);
             G[k][1] = sweep_groups(P[k], Shape<1>::CPG, Shape<1>::NW);
             fits = Shape<5>::lds(P[k], G[k][0].max, NE) <= (size_t)SW_LDS &&
