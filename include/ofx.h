@@ -358,7 +358,7 @@ int ofx_mlp_set_params(ofx_mlp* net, const float* host);
 int ofx_mlp_forward(ofx_mlp* net, const float* x, int n, float* y);
 /* How ofx_mlp_forward and ofx_mlp_forward_noalloc evaluate the network (no
  * counterpart in the reference; results do not depend on it): variant 1
- * (default) all layers in one kernel, 128 samples per workgroup with the
+ * (default) all layers in one kernel, 16 to 64 samples per workgroup with the
  * hidden activations kept in LDS; variant 0 one GEMM kernel per layer, the
  * activations through device memory (the training pass's form). */
 int ofx_mlp_set_forward_variant(ofx_mlp* net, int variant);
@@ -367,10 +367,10 @@ int ofx_mlp_set_forward_variant(ofx_mlp* net, int variant);
  * capture, serving loops).  x_dev [n][9] and y_dev [n][5] are DEVICE pointers
  * owned by the caller; the work is launched on `stream` (a hipStream_t; NULL:
  * the network's own stream) with no host synchronisation, copy, memset or
- * allocation.  n <= 8192: the work arrays are one fixed 10.25 MiB device
- * array per GPU, held until the process ends and shared by every call on
- * that GPU, so calls that overlap on one GPU race.  Larger n is rejected
- * (OFX_EINVAL).  Results equal ofx_mlp_forward's bit for bit. */
+ * allocation.  n <= 8192; larger n is rejected (OFX_EINVAL).  Under
+ * forward variant 0 the work arrays are one fixed 10.25 MiB device array per
+ * GPU, held until the process ends and shared by every call on that GPU, so
+ * such calls that overlap on one GPU race; variant 1 needs no work array.  Results equal ofx_mlp_forward's bit for bit. */
 int ofx_mlp_forward_noalloc(ofx_mlp* net, const float* x_dev, int n, float* y_dev, void* stream);
 /* Mean-squared-error loss over the 5 outputs and its gradient with respect to
  * every parameter (same layout as the parameter vector); no update. */

@@ -24,6 +24,8 @@ namespace ofx {
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef __bf16 v4bf __attribute__((ext_vector_type(4)));
+typedef float v8f __attribute__((ext_vector_type(8)));
 typedef uint16_t bf16;
 
 constexpr int NIN = 9, NIN_P = 16, NHID = 256, NLAYER = 6, NOUT = 5, NOUT_P = 64;
@@ -148,116 +150,177 @@ __global__ void __launch_bounds__(256) k_gemm(const bf16* __restrict__ A, int ld
 
 // The network's weights and biases as the one-kernel forward pass reads them.
 struct MlpFwd {
-    const bf16* wt[NLAYER];  // transposed bf16 weights [kout][kin]
+    const bf16* wf[NLAYER];  // bf16 weights in MFMA operand order (frag_index)
     const float* b[NLAYER];
 };
 
-// The whole forward pass of 64 samples in one workgroup: the activations of
-// every hidden layer stay in LDS (64 x 256 bf16, 32 KiB), so HBM sees only the
-// packed inputs, the weights (from L2) and the outputs, and several
-// workgroups share a CU, so one's layer barriers do not idle the MFMA units.
-// Four waves; wave w computes all 64 rows and columns 64w..64w+63 of a
-// hidden layer (4 x 4 tiles of v_mfma_f32_16x16x32_bf16, operands as in
-// k_gemm: A from LDS, Bt straight from the weights), then all waves write
-// their tiles back over the layer's input once every wave has read it.  The
-// output layer needs its first 16 (of 64 padded) columns only: wave w
-// computes rows 16w..16w+15 of them.
+// Weights in operand order: lane l's 8 values of 16-column tile j and 32-wide
+// k step s are one 16-byte vector, 64 lanes contiguous, so that an operand load
+// is 1 KB of whole cache lines.  (From the transposed weights a load
+// touched half of 16 lines, the other half needed a step later: a forward pass
+// of 16 samples per workgroup took 17.1 us, 7.0 in this order.)  `steps`: k steps of the layer.
+__host__ __device__ constexpr int frag_steps(int l) { return l == 0 ? 1 : NHID / 32; }
+__host__ __device__ constexpr int frag_tiles(int l) { return l == NLAYER - 1 ? 1 : NHID / 16; }  // output: columns 0..15
+__device__ __forceinline__ size_t frag_index(int tile, int step, int steps, int lane) {
+    return ((size_t)(tile * steps + step) * 64 + lane) * 8;
+}
+struct MlpFrag {
+    const bf16* wb[NLAYER];
+    bf16* wf[NLAYER];
+};
+__global__ void __launch_bounds__(256) k_frag(MlpFrag P) {
+    int v = blockIdx.x * 256 + threadIdx.x;  // 16-byte vector over all layers
+#pragma unroll
+    for (int l = 0; l < NLAYER; ++l) {
+        const int steps = frag_steps(l), n = frag_tiles(l) * steps * 64;
+        if (v < n) {
+            const int lane = v & 63, st = (v >> 6) % steps, tile = (v >> 6) / steps;
+            const int kin = l == 0 ? NIN_P : NHID, kout = l == NLAYER - 1 ? NOUT_P : NHID;
+            const int k0 = 32 * st + 8 * (lane >> 4), col = 16 * tile + (lane & 15);
+            uint16_t o[8];
+            for (int e = 0; e < 8; ++e) o[e] = k0 + e < kin ? P.wb[l][(size_t)(k0 + e) * kout + col] : 0;
+            for (int e = 0; e < 8; ++e) P.wf[l][(size_t)v * 8 + e] = o[e];
+            return;
+        }
+        v -= n;
+    }
+}
+
+// The whole forward pass of BM = 16 RT samples in one workgroup of NW waves,
+// from the caller's fp32 inputs [n][9] to its fp32 outputs [n][5]: the
+// activations of every hidden layer stay in LDS (BM x 256 bf16), so HBM sees
+// the inputs, the outputs and (through L2) the weights.  Wave w computes columns
+// 16 CT w .. of every layer for all rows, as RT x CT tiles of
+// v_mfma_f32_16x16x32_bf16 with the weights as the first operand: lane l
+// supplies 8 k's of output column l % 16 and of row l % 16, and receives the
+// four consecutive columns 4 (l / 16) .. + 3 of row l % 16, so an epilogue
+// packs four activations into one 8-byte LDS write.  The weights are loaded
+// PF k steps ahead, across layer ends (they do not depend on the
+// activations), the activations one step ahead, into register rings indexed by
+// compile-time step numbers.  TWO: two activation buffers, one barrier per layer
+// instead of two.
 // Every product, sum order and epilogue is k_gemm's (the MFMA chain over k in
 // ascending 32-wide steps from zero, the 16-wide input layer through one MFMA
 // with k 16..31 zero), so the outputs are those of the layer-by-layer pass
 // bit for bit.  LDS rows are 512 bytes with no padding; the 16-byte vector v
 // of row r is stored at v ^ (r & 15), so the 16 rows an MFMA operand load
-// reads fall in different banks.  Mp is a multiple of 64; rows at or past it
-// would read zero inputs and not be stored.
+// reads fall in different banks.  Rows past n read zero inputs and are not
+// stored.
+// Shapes and what bounds them: see forward_fused.
 __device__ __forceinline__ int swz(int r, int k) { return (((k >> 3) ^ (r & 15)) << 3) | (k & 7); }
 
-__global__ void __launch_bounds__(256) k_mlp_forward(const bf16* __restrict__ x16, int Mp, MlpFwd P,
-                                                     float* __restrict__ y) {
-    constexpr int BM = 64;
-    __shared__ __align__(16) bf16 sH[BM][NHID];
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int m0 = blockIdx.x * BM;
-    const int r0 = 0, c0 = 64 * w;  // this wave's tile of a hidden layer
-    const int lr = lane & 15, lk = 8 * (lane >> 4);    // operand row within a 16-tile; k offset of the lane's 8
-    const v8bf zero8 = {};
-    v4f acc[4][4];
-    // bias + SiLU of this wave's tile into the activation rows
-    auto store_silu = [&](const float* bias) {
-        for (int j = 0; j < 4; ++j) {
-            const int col = c0 + 16 * j + lr;
-            const float bc = bias[col];
-            for (int i = 0; i < 4; ++i)
-                for (int r = 0; r < 4; ++r) {
-                    const int row = r0 + 16 * i + 4 * (lane >> 4) + r;
-                    sH[row][swz(row, col)] = f2bf(silu(acc[i][j][r] + bc));
-                }
-        }
-    };
-    // layer 0: k = 16 packed inputs, k 16..31 of the MFMA zero
-    for (int i = 0; i < 4; ++i)
-        for (int j = 0; j < 4; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-    {
-        v8bf b[4];
-        for (int j = 0; j < 4; ++j)
-            b[j] = lk < NIN_P ? *(const v8bf*)&P.wt[0][(size_t)(c0 + 16 * j + lr) * NIN_P + lk] : zero8;
-        for (int i = 0; i < 4; ++i) {
-            const int row = m0 + r0 + 16 * i + lr;
-            const v8bf a = (lk < NIN_P && row < Mp) ? *(const v8bf*)&x16[(size_t)row * NIN_P + lk] : zero8;
-            for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[j], acc[i][j], 0, 0, 0);
-        }
-    }
-    store_silu(P.b[0]);
-    __syncthreads();
-    // hidden layers 1..4: 256 -> 256, 8 k steps of 32 each.  The weights are
-    // loaded from L2 two steps ahead (across layer ends: they do not depend
-    // on the activations) and the activations from LDS one step ahead, into
-    // register rings indexed by compile-time step numbers (both loops
-    // unrolled).
-    v8bf B[3][4], Am[2][4];
-    auto load_b = [&](const bf16* wt, int ks, v8bf* dst) {
-        for (int j = 0; j < 4; ++j) dst[j] = *(const v8bf*)&wt[(size_t)(c0 + 16 * j + lr) * NHID + ks + lk];
-    };
-    auto load_a = [&](int ks, v8bf* dst) {
-        for (int i = 0; i < 4; ++i) {
-            const int row = r0 + 16 * i + lr;
-            dst[i] = *(const v8bf*)&sH[row][swz(row, ks + lk)];
-        }
-    };
+template <int RT, int NW, int PF, bool TWO>
+__global__ void __launch_bounds__(64 * NW) k_mlp_forward(const float* __restrict__ x, int n, MlpFwd P,
+                                                         float* __restrict__ y) {
+    constexpr int BM = 16 * RT, CT = 16 / NW;
     constexpr int NSTEP = NHID / 32, NHL = NLAYER - 2;  // k steps per layer, hidden 256 -> 256 layers
-    load_b(P.wt[1], 0, B[0]);
-    load_b(P.wt[1], 32, B[1]);
+    __shared__ __align__(16) bf16 sH[TWO ? 2 : 1][BM][NHID];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int m0 = blockIdx.x * BM, c0 = 16 * CT * w;
+    const int lr = lane & 15, q = lane >> 4, lk = 8 * q;
+    v4f acc[RT][CT];
+    v4f bias[CT];
+    auto load_bias = [&](int l) {
+#pragma unroll
+        for (int j = 0; j < CT; ++j) bias[j] = *(const v4f*)&P.b[l][c0 + 16 * j + 4 * q];
+    };
+    auto clear = [&]() {
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+            for (int j = 0; j < CT; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    };
+    // bias + SiLU of this wave's tile into the activation rows
+    auto store_silu = [&](bf16(*h)[NHID]) {
+#pragma unroll
+        for (int j = 0; j < CT; ++j)
+#pragma unroll
+            for (int i = 0; i < RT; ++i) {
+                const int row = 16 * i + lr, col = c0 + 16 * j + 4 * q;
+                const v4f v = acc[i][j] + bias[j];
+                const v4f s = {silu(v.x), silu(v.y), silu(v.z), silu(v.w)};
+                *(v4bf*)&h[row][swz(row, col)] = __builtin_convertvector(s, v4bf);
+            }
+    };
+    v8bf B[PF + 1][CT], Am[2][RT];
+    auto load_b = [&](int g) {  // weights of flat step g (layer 1 + g / NSTEP)
+        const bf16* wf = P.wf[1 + g / NSTEP];
+#pragma unroll
+        for (int j = 0; j < CT; ++j) B[g % (PF + 1)][j] = *(const v8bf*)&wf[frag_index(CT * w + j, g % NSTEP, NSTEP, lane)];
+    };
+    // layer 0: k = 16 packed inputs (9 used), k 16..31 of the MFMA zero
+    {
+        v8bf b[CT], a[RT];
+#pragma unroll
+        for (int j = 0; j < CT; ++j)
+            b[j] = *(const v8bf*)&P.wf[0][frag_index(CT * w + j, 0, 1, lane)];
+#pragma unroll
+        for (int i = 0; i < RT; ++i) {
+            const int row = m0 + 16 * i + lr;
+            v8f f = {};
+            if (row < n && q < 2) {
+                const float* xr = x + (size_t)row * NIN + lk;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) f[k] = (k == 0 || q == 0) ? xr[k * (q == 0)] : 0.f;
+            }
+            a[i] = __builtin_convertvector(f, v8bf);
+        }
+        load_bias(0);
+#pragma unroll
+        for (int g = 0; g < PF; ++g) load_b(g);
+        clear();
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+            for (int j = 0; j < CT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
+    }
+    store_silu(sH[0]);
+    __syncthreads();
 #pragma unroll
     for (int h = 0; h < NHL; ++h) {
-        for (int i = 0; i < 4; ++i)
-            for (int j = 0; j < 4; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+        bf16(*src)[NHID] = sH[TWO ? h & 1 : 0];
+        auto load_a = [&](int ks, v8bf* dst) {
+#pragma unroll
+            for (int i = 0; i < RT; ++i) {
+                const int row = 16 * i + lr;
+                dst[i] = *(const v8bf*)&src[row][swz(row, ks + lk)];
+            }
+        };
+        load_bias(1 + h);
+        clear();
         load_a(0, Am[0]);
 #pragma unroll
         for (int st = 0; st < NSTEP; ++st) {
-            const int g = h * NSTEP + st, g2 = g + 2;
-            if (g2 < NHL * NSTEP) load_b(P.wt[1 + g2 / NSTEP], 32 * (g2 % NSTEP), B[g2 % 3]);
+            const int g = h * NSTEP + st;
+            if (g + PF < NHL * NSTEP) load_b(g + PF);
             if (st + 1 < NSTEP) load_a(32 * (st + 1), Am[(st + 1) & 1]);
-            for (int i = 0; i < 4; ++i)
-                for (int j = 0; j < 4; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Am[st & 1][i], B[g % 3][j], acc[i][j], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < RT; ++i)
+#pragma unroll
+                for (int j = 0; j < CT; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(B[g % (PF + 1)][j], Am[st & 1][i], acc[i][j], 0, 0, 0);
         }
-        __syncthreads();  // every wave has read this layer's input
-        store_silu(P.b[1 + h]);
+        if (!TWO) __syncthreads();  // every wave has read this layer's input
+        store_silu(sH[TWO ? (h + 1) & 1 : 0]);
         __syncthreads();
     }
-    // output layer: columns 0..15 of the padded 64, rows 16w..16w+15
-    {
-        const int L = NLAYER - 1;
+    // output layer: the first 16 of the padded 64 columns, row tiles dealt to the waves
+    const bf16(*src)[NHID] = sH[TWO ? NHL & 1 : 0];
+    const v4f bo = *(const v4f*)&P.b[NLAYER - 1][4 * q];
+    for (int i = w; i < RT; i += NW) {
         v4f o = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
         for (int ks = 0; ks < NHID; ks += 32) {
-            const v8bf b = *(const v8bf*)&P.wt[L][(size_t)lr * NHID + ks + lk];
-            const int row = 16 * w + lr;
-            const v8bf a = *(const v8bf*)&sH[row][swz(row, ks + lk)];
-            o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, o, 0, 0, 0);
+            const v8bf b = *(const v8bf*)&P.wf[NLAYER - 1][frag_index(0, ks / 32, NSTEP, lane)];
+            const v8bf a = *(const v8bf*)&src[16 * i + lr][swz(16 * i + lr, ks + lk)];
+            o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a, o, 0, 0, 0);
         }
-        const float bc = P.b[L][lr];
-        for (int r = 0; r < 4; ++r) {
-            const int row = m0 + 16 * w + 4 * (lane >> 4) + r;
-            if (row < Mp) y[(size_t)row * NOUT_P + lr] = o[r] + bc;
+        o += bo;
+        const int row = m0 + 16 * i + lr;
+        if (row < n) {
+            float* yr = y + (size_t)row * NOUT;
+            if (q == 0) { yr[0] = o.x; yr[1] = o.y; yr[2] = o.z; yr[3] = o.w; }
+            if (q == 1) yr[4] = o.x;
         }
     }
 }
@@ -415,6 +478,7 @@ struct ofx_mlp {
     int kin[NLAYER], kout[NLAYER];        // padded shapes of each layer
     float *w[NLAYER], *b[NLAYER];          // fp32 master
     bf16 *wb[NLAYER], *wt[NLAYER];         // bf16 copy and its transpose
+    bf16* wf[NLAYER];                      // bf16 copy in MFMA operand order (frag_index)
     float *mw[NLAYER], *vw[NLAYER], *mb[NLAYER], *vb[NLAYER];
     float *gw[NLAYER], *gb[NLAYER];        // gradients
     int step = 0;
@@ -429,6 +493,8 @@ struct ofx_mlp {
     float *dyf = nullptr, *gz = nullptr;  // fp32 gradient of the current layer's pre-activation
     bf16 *gzb = nullptr, *gzb2 = nullptr;
     float *part = nullptr, *lpart = nullptr, *loss = nullptr, *cpart = nullptr;
+    float *io_x = nullptr, *io_y = nullptr;  // device copies of a one-kernel forward's inputs and outputs
+    int io_cap = 0;
     int fwd_variant = 1;  // inference forward pass: 0 layer by layer, 1 one kernel (k_mlp_forward)
     std::vector<void*> allocs;
 };
@@ -472,6 +538,23 @@ int mlp_reserve(ofx_mlp* n, int samples) {
     OFX_TRY(A((void**)&n->loss, sizeof(float) * 4));
     OFX_TRY(A((void**)&n->cpart, sizeof(float) * ((size_t)Mp / COLSUM_ROWS * NHID + NHID)));
     n->cap = Mp;
+    return 0;
+}
+
+// Device buffers of a one-kernel forward of `samples` samples.
+int io_reserve(ofx_mlp* n, int samples) {
+    if (samples <= n->io_cap) return 0;
+    OFX_HIP(hipStreamSynchronize(n->stream));
+    if (n->io_x) (void)hipFree(n->io_x);
+    n->io_x = nullptr;
+    n->io_cap = 0;
+    if (hipMalloc((void**)&n->io_x, sizeof(float) * (size_t)samples * (NIN + NOUT)) != hipSuccess) {
+        n->io_x = nullptr;
+        set_error("mlp: out of device memory");
+        return OFX_ENOMEM;
+    }
+    n->io_y = n->io_x + (size_t)samples * NIN;
+    n->io_cap = samples;
     return 0;
 }
 
@@ -546,19 +629,34 @@ int colsum(ofx_mlp* n, const float* g, int M, int N, float* out) {
     return 0;
 }
 
-// All layers in one kernel (k_mlp_forward): packed inputs x16 [Mp][16] ->
-// padded outputs y [Mp][64] (columns 0..15 written).
-int forward_fused(const ofx_mlp* n, hipStream_t st, const bf16* x16, int Mp, float* y) {
+// All layers in one kernel (k_mlp_forward): fp32 inputs x [n][9] -> fp32 outputs
+// y [n][5].
+template <int RT, int NW, int PF, bool TWO>
+int forward_shape(const ofx_mlp* n, hipStream_t st, const float* x, int nsamp, float* y) {
     MlpFwd P;
-    for (int l = 0; l < NLAYER; ++l) { P.wt[l] = n->wt[l]; P.b[l] = n->b[l]; }
-    k_mlp_forward<<<(Mp + 63) / 64, 256, 0, st>>>(x16, Mp, P, y);
+    for (int l = 0; l < NLAYER; ++l) { P.wf[l] = n->wf[l]; P.b[l] = n->b[l]; }
+    k_mlp_forward<RT, NW, PF, TWO><<<(nsamp + 16 * RT - 1) / (16 * RT), 64 * NW, 0, st>>>(x, nsamp, P, y);
     OFX_HIP(hipGetLastError());
     return 0;
+}
+// Rows per workgroup by sample count.  Up to one workgroup per CU the pass is
+// bound by one workgroup's chain (five layers of weights through one CU, ~1 us
+// each), shortest with the fewest rows; beyond, by the SiLU epilogues, the
+// matrix units and the weights' L2 traffic, which more rows share.  us for 16 /
+// 32 / 64 rows: 500 samples 7.2 / 9.2 / 12.9, 4096 8.3 / 9.6 / 13.2, 8192 13.5 /
+// 10.2 / 13.5, 16384 24 / 17 / 15, 1,000,003 1186 / 803 / 627 (0.89 PFLOP/s).
+// 128 rows: 710; four waves of 64 columns instead of eight of 32: 643.  With the
+// weights' transposed rows as operands, activations packed and written one
+// by one, and separate kernels packing inputs and outputs, 500 samples took
+// 37 us and 1,000,003 took 1333.
+int forward_fused(const ofx_mlp* n, hipStream_t st, const float* x, int nsamp, float* y) {
+    if (nsamp <= 16 * 256) return forward_shape<1, 8, 8, true>(n, st, x, nsamp, y);
+    if (nsamp <= 32 * 256) return forward_shape<2, 8, 8, true>(n, st, x, nsamp, y);
+    return forward_shape<4, 8, 4, true>(n, st, x, nsamp, y);
 }
 
 // keep_z: store the pre-activations (a backward pass follows).
 int forward(ofx_mlp* n, int Mp, bool keep_z) {
-    if (!keep_z && n->fwd_variant == 1) return forward_fused(n, n->stream, n->h[0], Mp, n->y);
     for (int l = 0; l < NLAYER - 1; ++l)
         OFX_TRY(gemm<EPI_BIAS_SILU>(n, n->h[l], n->kin[l], n->wt[l], n->kin[l], Mp, n->kout[l], n->kin[l], 1, nullptr,
                                     n->h[l + 1], n->kout[l], n->b[l], nullptr, keep_z ? n->z[l] : nullptr));
@@ -568,9 +666,21 @@ int forward(ofx_mlp* n, int Mp, bool keep_z) {
     return 0;
 }
 
-// The transposed bf16 weights [kout][kin] that the forward products read,
-// refreshed whenever the bf16 weights change.
-int refresh_wt(ofx_mlp* n) {
+// The operand-ordered weights of the one-kernel forward.
+int refresh_frag(ofx_mlp* n) {
+    MlpFrag P;
+    int vec = 0;
+    for (int l = 0; l < NLAYER; ++l) { P.wb[l] = n->wb[l]; P.wf[l] = n->wf[l]; vec += 64 * frag_tiles(l) * frag_steps(l); }
+    k_frag<<<(vec + 255) / 256, 256, 0, n->stream>>>(P);
+    OFX_HIP(hipGetLastError());
+    return 0;
+}
+
+// The transposed bf16 weights [kout][kin] that the layered forward products
+// read, refreshed whenever the bf16 weights change (and the operand-ordered
+// ones, for training at its end only).
+int refresh_wt(ofx_mlp* n, bool frag = true) {
+    if (frag) OFX_TRY(refresh_frag(n));
     for (int l = 0; l < NLAYER; ++l) OFX_TRY(transpose(n, n->wb[l], n->kin[l], n->kout[l], n->wt[l], n->kout[l]));
     return 0;
 }
@@ -700,8 +810,8 @@ int ofx_mlp_create(ofx_mlp** out, int device, unsigned long long seed) {
         if (!rc) { rc = mlp_alloc(n, &p, sizeof(float) * n->kout[l]); n->vb[l] = (float*)p; }
         if (!rc) { rc = mlp_alloc(n, &p, sizeof(float) * nw); n->gw[l] = (float*)p; }
         if (!rc) { rc = mlp_alloc(n, &p, sizeof(float) * n->kout[l]); n->gb[l] = (float*)p; }
-        if (!rc) { rc = mlp_alloc(n, &p, 16); }  // spare slots keep the count at 12 per layer
-        if (!rc) { rc = mlp_alloc(n, &p, 16); }
+        if (!rc) { rc = mlp_alloc(n, &p, sizeof(bf16) * 512 * frag_tiles(l) * frag_steps(l)); n->wf[l] = (bf16*)p; }
+        if (!rc) { rc = mlp_alloc(n, &p, 16); }  // a spare slot keeps the count at 12 per layer
         if (!rc && hipMemcpyAsync(n->w[l], hw.data(), sizeof(float) * nw, hipMemcpyHostToDevice, n->stream) != hipSuccess)
             rc = OFX_EHIP;
         if (!rc) {
@@ -724,6 +834,7 @@ int ofx_mlp_destroy(ofx_mlp* n) {
     (void)hipSetDevice(n->device);
     if (n->stream) (void)hipStreamSynchronize(n->stream);
     for (void* p : n->allocs) (void)hipFree(p);
+    if (n->io_x) (void)hipFree(n->io_x);
     if (n->stream) (void)hipStreamDestroy(n->stream);
     delete n;
     return 0;
@@ -774,14 +885,20 @@ int ofx_mlp_set_params(ofx_mlp* n, const float* host) {
 int ofx_mlp_forward(ofx_mlp* n, const float* x, int nsamp, float* y) {
     if (!n || !x || !y || nsamp < 1 || nsamp > MLP_MAXN) { set_error("mlp_forward: bad arguments"); return OFX_EINVAL; }
     OFX_HIP(hipSetDevice(n->device));
-    OFX_TRY(load_batch(n, x, nullptr, nsamp, false));
-    int Mp = (nsamp + 63) / 64 * 64;
-    OFX_TRY(forward(n, Mp, false));
-    // tgt (Mp x NOUT floats) is free in a forward-only call: pack there, copy once
-    size_t cnt = (size_t)nsamp * NOUT;
-    k_pack_outputs<<<(unsigned)((cnt + 255) / 256), 256, 0, n->stream>>>(n->y, nsamp, n->tgt);
-    OFX_HIP(hipGetLastError());
-    OFX_HIP(hipMemcpyAsync(y, n->tgt, sizeof(float) * cnt, hipMemcpyDeviceToHost, n->stream));
+    const size_t cnt = (size_t)nsamp * NOUT;
+    if (n->fwd_variant == 1) {
+        OFX_TRY(io_reserve(n, nsamp));
+        OFX_HIP(hipMemcpyAsync(n->io_x, x, sizeof(float) * (size_t)nsamp * NIN, hipMemcpyHostToDevice, n->stream));
+        OFX_TRY(forward_fused(n, n->stream, n->io_x, nsamp, n->io_y));
+        OFX_HIP(hipMemcpyAsync(y, n->io_y, sizeof(float) * cnt, hipMemcpyDeviceToHost, n->stream));
+    } else {
+        OFX_TRY(load_batch(n, x, nullptr, nsamp, false));
+        OFX_TRY(forward(n, (nsamp + 63) / 64 * 64, false));
+        // tgt (Mp x NOUT floats) is free in a forward-only call: pack there, copy once
+        k_pack_outputs<<<(unsigned)((cnt + 255) / 256), 256, 0, n->stream>>>(n->y, nsamp, n->tgt);
+        OFX_HIP(hipGetLastError());
+        OFX_HIP(hipMemcpyAsync(y, n->tgt, sizeof(float) * cnt, hipMemcpyDeviceToHost, n->stream));
+    }
     OFX_HIP(hipStreamSynchronize(n->stream));
     return 0;
 }
@@ -793,28 +910,25 @@ int ofx_mlp_forward_noalloc(ofx_mlp* n, const float* x_dev, int nsamp, float* y_
         return OFX_EINVAL;
     }
     OFX_HIP(hipSetDevice(n->device));
+    hipStream_t st = stream ? static_cast<hipStream_t>(stream) : n->stream;
+    if (n->fwd_variant == 1) return forward_fused(n, st, x_dev, nsamp, y_dev);
     unsigned char* base = nullptr;
     OFX_TRY(scratch_address(n->device, &base));
-    hipStream_t st = stream ? static_cast<hipStream_t>(stream) : n->stream;
     bf16* in = reinterpret_cast<bf16*>(base);
     bf16* act[2] = {reinterpret_cast<bf16*>(base + NOALLOC_IN), reinterpret_cast<bf16*>(base + NOALLOC_IN + NOALLOC_ACT)};
     float* yp = reinterpret_cast<float*>(base + NOALLOC_IN + 2 * NOALLOC_ACT);
     const int Mp = (nsamp + 63) / 64 * 64;
     k_pack_inputs<<<(Mp * NIN_P + 255) / 256, 256, 0, st>>>(x_dev, nsamp, Mp, in);
     OFX_HIP(hipGetLastError());
-    if (n->fwd_variant == 1) {
-        OFX_TRY(forward_fused(n, st, in, Mp, yp));
-    } else {
-        const bf16* h = in;
-        for (int l = 0; l < NLAYER - 1; ++l) {
-            OFX_TRY(gemm_on<EPI_BIAS_SILU>(st, h, n->kin[l], n->wt[l], n->kin[l], Mp, n->kout[l], n->kin[l], 1,
-                                           nullptr, act[l & 1], n->kout[l], n->b[l], nullptr, nullptr));
-            h = act[l & 1];
-        }
-        const int L = NLAYER - 1;
-        OFX_TRY(gemm_on<EPI_BIAS>(st, h, n->kin[L], n->wt[L], n->kin[L], Mp, n->kout[L], n->kin[L], 1, yp, nullptr,
-                                  n->kout[L], n->b[L], nullptr, nullptr));
+    const bf16* h = in;
+    for (int l = 0; l < NLAYER - 1; ++l) {
+        OFX_TRY(gemm_on<EPI_BIAS_SILU>(st, h, n->kin[l], n->wt[l], n->kin[l], Mp, n->kout[l], n->kin[l], 1, nullptr,
+                                       act[l & 1], n->kout[l], n->b[l], nullptr, nullptr));
+        h = act[l & 1];
     }
+    const int L = NLAYER - 1;
+    OFX_TRY(gemm_on<EPI_BIAS>(st, h, n->kin[L], n->wt[L], n->kin[L], Mp, n->kout[L], n->kin[L], 1, yp, nullptr,
+                              n->kout[L], n->b[L], nullptr, nullptr));
     size_t cnt = (size_t)nsamp * NOUT;
     k_pack_outputs<<<(unsigned)((cnt + 255) / 256), 256, 0, st>>>(yp, nsamp, y_dev);
     OFX_HIP(hipGetLastError());
@@ -856,7 +970,7 @@ static int train_step(ofx_mlp* n, int nsamp, float lr) {
                                                                (size_t)n->kout[l], lr, b1, b2, eps, c1, c2);
     }
     OFX_HIP(hipGetLastError());
-    return refresh_wt(n);
+    return refresh_wt(n, false);
 }
 
 int ofx_mlp_train(ofx_mlp* n, const float* x, const float* t, int nsamp, int batch, int steps, float lr,
@@ -908,6 +1022,7 @@ int ofx_mlp_train(ofx_mlp* n, const float* x, const float* t, int nsamp, int bat
         rc = train_step(n, bsz, lr);
         if (!rc) k_copy1<<<1, 64, 0, n->stream>>>(n->loss, dl + st);
     }
+    if (const int r2 = refresh_frag(n)) rc = rc ? rc : r2;
     if (!rc && hipStreamSynchronize(n->stream) != hipSuccess) rc = OFX_EHIP;
     if (!rc && loss_out && hipMemcpy(loss_out, dl, sizeof(float) * (size_t)steps, hipMemcpyDeviceToHost) != hipSuccess)
         rc = OFX_EHIP;

@@ -85,3 +85,18 @@ def test_training_reduces_loss():
     first, last = float(losses[:5].mean()), float(losses[-20:].mean())
     print(f"\n[mlp] training loss {first:.4e} -> {last:.4e}", flush=True)
     assert np.all(np.isfinite(losses)) and last < 0.1 * first, (first, last)
+
+
+@pytest.mark.parametrize("n", [1, 15, 17, 4095, 4096, 4097, 8192, 8193, 8255])
+def test_one_kernel_forward_shapes(n):
+    """Every workgroup shape of the one-kernel forward at its edges, against
+    the layered pass: the same bits, an infinite and a NaN input included."""
+    rng = np.random.default_rng(n)
+    x = rng.normal(0, 1, (n, NIN)).astype(np.float32)
+    x[0, 3], x[n // 2, 8] = np.inf, np.nan
+    m = net(random_params(rng, scale=1.0).astype(np.float32))
+    m.set_forward_variant(0)
+    y0 = m.forward(x)
+    m.set_forward_variant(1)
+    y1 = m.forward(x)
+    assert np.array_equal(y0, y1, equal_nan=True)
