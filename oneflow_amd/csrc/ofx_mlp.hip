@@ -26,6 +26,7 @@ typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef __bf16 v4bf __attribute__((ext_vector_type(4)));
 typedef float v8f __attribute__((ext_vector_type(8)));
+typedef uint16_t v8us __attribute__((ext_vector_type(8)));
 typedef uint16_t bf16;
 
 constexpr int NIN = 9, NIN_P = 16, NHID = 256, NLAYER = 6, NOUT = 5, NOUT_P = 64;
@@ -49,13 +50,12 @@ __device__ __forceinline__ float dsilu(float z) {
     return s * (1.0f + z * (1.0f - s));
 }
 
-enum { EPI_PARTIAL = 0, EPI_BIAS_SILU = 1, EPI_BIAS = 2, EPI_DSILU = 3 };
+enum { EPI_BIAS_SILU = 0, EPI_BIAS = 1 };
 
 // C[M x N] = A[M x K] Bt[N x K]^T: both operands bf16 with k contiguous
 // (row strides lda, ldb), so every global and LDS access moves 8 elements
 // (16 bytes) at a time.  BM x BN block tile (64 or 128 each; M and N
-// multiples of them); blockIdx.z selects the K range [z*kchunk,
-// (z+1)*kchunk), a multiple of 16 (an 8-element vector at or past its end is
+// multiples of them); K a multiple of 16 (an 8-element vector at or past its end is
 // zero-filled, so K = 16 runs through the 32-deep MFMA with zero products
 // added).  256 threads: wave w owns rows (BM/2)*(w>>1).. and columns
 // (BN/2)*(w&1).. as (BM/32) x (BN/32) tiles of gfx950's
@@ -68,9 +68,8 @@ enum { EPI_PARTIAL = 0, EPI_BIAS_SILU = 1, EPI_BIAS = 2, EPI_DSILU = 3 };
 // tiles re-read each operand from L2 fewer times (the forward of many samples).
 template <int EPI, int KC, int BM, int BN>
 __global__ void __launch_bounds__(256) k_gemm(const bf16* __restrict__ A, int lda, const bf16* __restrict__ Bt, int ldb,
-                                              int kchunk, int M, float* __restrict__ Cf, bf16* __restrict__ Cb, int ldc,
-                                              const float* __restrict__ bias, const float* __restrict__ zin,
-                                              float* __restrict__ zout) {
+                                              int ke, float* __restrict__ Cf, bf16* __restrict__ Cb, int ldc,
+                                              const float* __restrict__ bias) {
     constexpr int PAD = 8;              // bf16 elements of row padding (LDS bank spread)
     constexpr int VR = KC / 8;          // 8-element vectors per tile row
     constexpr int NVA = BM * VR / 256;  // vectors per thread of the A tile
@@ -82,7 +81,6 @@ __global__ void __launch_bounds__(256) k_gemm(const bf16* __restrict__ A, int ld
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
     const int wm = (BM / 2) * (w >> 1), wn = (BN / 2) * (w & 1);
-    const int kb = blockIdx.z * kchunk, ke = kb + kchunk;
     v4f acc[MT][NT];
     for (int i = 0; i < MT; ++i)
         for (int j = 0; j < NT; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
@@ -100,8 +98,8 @@ __global__ void __launch_bounds__(256) k_gemm(const bf16* __restrict__ A, int ld
             rb[u] = (k0 + kv < ke) ? *(const v4u*)&Bt[(size_t)(n0 + r) * ldb + k0 + kv] : v4u{0u, 0u, 0u, 0u};
         }
     };
-    gload(kb);
-    for (int k0 = kb; k0 < ke; k0 += KC) {
+    gload(0);
+    for (int k0 = 0; k0 < ke; k0 += KC) {
         __syncthreads();  // the previous chunk's MFMAs have read LDS
 #pragma unroll
         for (int u = 0; u < NVA; ++u) {
@@ -132,19 +130,8 @@ __global__ void __launch_bounds__(256) k_gemm(const bf16* __restrict__ A, int ld
                 int col = n0 + wn + 16 * j + (lane & 15);
                 size_t o = (size_t)row * ldc + col;
                 float v = acc[i][j][r];
-                if (EPI == EPI_PARTIAL) {
-                    Cf[(size_t)blockIdx.z * M * ldc + o] = v;
-                } else if (EPI == EPI_BIAS_SILU) {
-                    float z = v + bias[col];
-                    if (zout) zout[o] = z;  // pre-activations kept for a backward pass only
-                    Cb[o] = f2bf(silu(z));
-                } else if (EPI == EPI_BIAS) {
-                    Cf[o] = v + bias[col];
-                } else {  // EPI_DSILU: gradient through the activation
-                    float g = v * dsilu(zin[o]);
-                    Cf[o] = g;
-                    Cb[o] = f2bf(g);
-                }
+                if (EPI == EPI_BIAS_SILU) Cb[o] = f2bf(silu(v + bias[col]));
+                else Cf[o] = v + bias[col];
             }
 }
 
@@ -164,25 +151,34 @@ __host__ __device__ constexpr int frag_tiles(int l) { return l == NLAYER - 1 ? 1
 __device__ __forceinline__ size_t frag_index(int tile, int step, int steps, int lane) {
     return ((size_t)(tile * steps + step) * 64 + lane) * 8;
 }
+// The backward products' order is that of W itself (a step covers 32 output
+// columns; the output layer's first 32 of 64).
 struct MlpFrag {
     const bf16* wb[NLAYER];
-    bf16* wf[NLAYER];
+    bf16 *wf[NLAYER], *wb_frag[NLAYER];
 };
 __global__ void __launch_bounds__(256) k_frag(MlpFrag P) {
     int v = blockIdx.x * 256 + threadIdx.x;  // 16-byte vector over all layers
 #pragma unroll
     for (int l = 0; l < NLAYER; ++l) {
+        const int kin = l == 0 ? NIN_P : NHID, kout = l == NLAYER - 1 ? NOUT_P : NHID;
         const int steps = frag_steps(l), n = frag_tiles(l) * steps * 64;
+        const int bsteps = l == NLAYER - 1 ? 1 : NHID / 32, nb = l == 0 ? 0 : NHID / 16 * bsteps * 64;
+        const int lane = v & 63;
         if (v < n) {
-            const int lane = v & 63, st = (v >> 6) % steps, tile = (v >> 6) / steps;
-            const int kin = l == 0 ? NIN_P : NHID, kout = l == NLAYER - 1 ? NOUT_P : NHID;
+            const int st = (v >> 6) % steps, tile = (v >> 6) / steps;
             const int k0 = 32 * st + 8 * (lane >> 4), col = 16 * tile + (lane & 15);
-            uint16_t o[8];
-            for (int e = 0; e < 8; ++e) o[e] = k0 + e < kin ? P.wb[l][(size_t)(k0 + e) * kout + col] : 0;
-            for (int e = 0; e < 8; ++e) P.wf[l][(size_t)v * 8 + e] = o[e];
+            for (int e = 0; e < 8; ++e) P.wf[l][(size_t)v * 8 + e] = k0 + e < kin ? P.wb[l][(size_t)(k0 + e) * kout + col] : 0;
             return;
         }
         v -= n;
+        if (v < nb) {
+            const int st = (v >> 6) % bsteps, tile = (v >> 6) / bsteps;
+            for (int e = 0; e < 8; ++e)
+                P.wb_frag[l][(size_t)v * 8 + e] = P.wb[l][(size_t)(16 * tile + (lane & 15)) * kout + 32 * st + 8 * (lane >> 4) + e];
+            return;
+        }
+        v -= nb;
     }
 }
 
@@ -341,47 +337,6 @@ __global__ void k_transpose(const bf16* in, int R, int Cc, bf16* out, int Cp) {
     }
 }
 
-// Sum of the split-K partials in split order.
-__global__ void k_splitk_sum(const float* part, int nsplit, size_t n, float* out) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float s = 0.f;
-    for (int z = 0; z < nsplit; ++z) s += part[(size_t)z * n + i];
-    out[i] = s;
-}
-
-// Column sums of an M x N fp32 matrix (bias gradients), two stages in a fixed
-// order: block (x, y) sums columns 64x..64x+63 over rows COLSUM_ROWS*y ..
-// (4 row lanes of COLSUM_ROWS/4 rows, then the 4 lanes in order) into
-// part[y][N]; then one block per 64 columns adds the row-chunk partials: row
-// lane r takes chunks r, r+4, r+8, ... in order, then the 4 lanes in order.
-constexpr int COLSUM_ROWS = 64;
-__global__ void __launch_bounds__(256) k_colsum_part(const float* g, int M, int N, float* part) {
-    __shared__ float sm[4][64];
-    int c = blockIdx.x * 64 + (threadIdx.x & 63), lane4 = threadIdx.x >> 6;
-    int r0 = blockIdx.y * COLSUM_ROWS + lane4 * (COLSUM_ROWS / 4);
-    float s = 0.f;
-    if (c < N)
-#pragma unroll
-        for (int r = r0; r < r0 + COLSUM_ROWS / 4; ++r)
-            if (r < M) s += g[(size_t)r * N + c];
-    sm[lane4][threadIdx.x & 63] = s;
-    __syncthreads();
-    if (threadIdx.x < 64 && c < N)
-        part[(size_t)blockIdx.y * N + c] = ((sm[0][threadIdx.x] + sm[1][threadIdx.x]) + sm[2][threadIdx.x]) + sm[3][threadIdx.x];
-}
-__global__ void __launch_bounds__(256) k_colsum_final(const float* part, int chunks, int N, float* out) {
-    __shared__ float sm[4][64];
-    int c = blockIdx.x * 64 + (threadIdx.x & 63), lane4 = threadIdx.x >> 6;
-    float s = 0.f;
-    if (c < N)
-        for (int k = lane4; k < chunks; k += 4) s += part[(size_t)k * N + c];
-    sm[lane4][threadIdx.x & 63] = s;
-    __syncthreads();
-    if (threadIdx.x < 64 && c < N)
-        out[c] = ((sm[0][threadIdx.x] + sm[1][threadIdx.x]) + sm[2][threadIdx.x]) + sm[3][threadIdx.x];
-}
-
 // Inputs fp32 [n][NIN] -> bf16 [Mp][NIN_P] (zero padded).
 __global__ void k_pack_inputs(const float* x, int n, int Mp, bf16* out) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -390,71 +345,393 @@ __global__ void k_pack_inputs(const float* x, int n, int Mp, bf16* out) {
     out[i] = (r < n && c < NIN) ? f2bf(x[(size_t)r * NIN + c]) : (bf16)0;
 }
 
-// MSE over the real outputs: loss partials and the bf16 / fp32 output gradient.
-__global__ void k_mse(const float* y, const float* tgt, int n, int Mp, bf16* dyb, float* dyf, float* lpart) {
-    __shared__ float sm[256];
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    float l = 0.f;
-    if (i < Mp * NOUT_P) {
-        int r = i / NOUT_P, c = i % NOUT_P;
-        float g = 0.f;
-        if (r < n && c < NOUT) {
-            float d = y[i] - tgt[(size_t)r * NOUT + c];
-            l = d * d;
-            g = 2.0f * d / (float)(n * NOUT);
+// ---- training: three kernels per step (gradients, weight products, update)
+
+// Layer l's increment in the parameter vector's layout (W[kin][kout], b[kout], ...).
+__host__ __device__ constexpr int lay_kin(int l) { return l == 0 ? NIN_P : NHID; }
+__host__ __device__ constexpr int lay_kout(int l) { return l == NLAYER - 1 ? NOUT_P : NHID; }
+__host__ __device__ constexpr int lay_off(int l) {
+    int o = 0;
+    for (int k = 0; k < l; ++k) o += lay_kin(k) * lay_kout(k) + lay_kout(k);
+    return o;
+}
+// Columns of a layer's pre-activation gradient that are kept (the output
+// layer's padding columns are zero beyond the first 16).
+__host__ __device__ constexpr int lay_gcols(int l) { return l == NLAYER - 1 ? 16 : NHID; }
+
+struct MlpTrain {
+    const bf16 *wf[NLAYER], *wb_frag[NLAYER];  // weights in operand order, forward and backward products
+    const float* b[NLAYER];
+    bf16 *hT[NLAYER], *gT[NLAYER];  // layer inputs and pre-activation gradients, [feature][sample]
+    float* cs[NLAYER];              // column sums of the fp32 gradients over 16 samples: [Mp / 16][lay_gcols]
+    float* lpart;                   // squared errors of 4 samples each
+    const float *x, *t;             // samples [..][9], targets [..][5]
+    const int* idx;                 // sample of each row (null: the row)
+    int n, Mp;                      // samples, and rounded up to 64 (the rest zero rows without loss)
+};
+
+// Forward and backward of BM = 16 RT samples in one workgroup: the forward pass
+// as k_mlp_forward, the pre-activations staying in registers (a lane holds the
+// same tile of every layer, so SiLU' of the backward pass finds them in place),
+// then from the output error down g_{l-1} = (g_l W_l^T) silu'(z_{l-1}), the
+// gradients through LDS like the activations.  HBM sees the samples, the weights
+// (L2), and what the weight products need: both factors transposed (sample
+// contiguous), in 32-byte pieces written from LDS.
+// Bound by the chain of 11 products in a workgroup, each step of which waits for
+// its weights from L2 and for the LDS exchange between layers.  Shapes measured
+// (us per training step, all three kernels, at 64 / 1024 / 4096 / 8192 samples):
+// <1,8,8> 32 / 42 / 49 / 78, <2,8,3> 39 / 50 / 54 / 68, <2,8,8> (weights further
+// ahead, but 50 registers spilled) 44 / 53 / 62 / 77, <2,16,4> 43 / 52 / 59 / 73,
+// <1,4,4> 37 / 48 / 57 / 95.  So 16 samples a workgroup while those are no more
+// than the 256 CUs, and 32 beyond.  A step of separate kernels for every product,
+// transpose, column sum and update (75 launches) took 404 us at 8192 samples.
+// The arithmetic is that of separate products: MFMA chains over k in ascending
+// 32-wide steps, fp32 epilogues, column sums of 16 samples in order.
+template <int RT, int NW, int PF>
+__global__ void __launch_bounds__(64 * NW) k_mlp_grad(MlpTrain P) {
+    constexpr int BM = 16 * RT, CT = 16 / NW;
+    constexpr int NSTEP = NHID / 32, NHL = NLAYER - 2, NF = NHL * NSTEP;  // forward steps 0..NF-1, backward NF..2NF-1
+    constexpr int GP = NHID + 4;  // fp32 gradient row, padded
+    static_assert(NW * 64 >= NHID * RT, "a thread per column and 16 samples");
+    __shared__ __align__(16) bf16 sH[2][BM][NHID];
+    __shared__ __align__(16) float sG[2][BM][GP];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int m0 = blockIdx.x * BM, c0 = 16 * CT * w;
+    const int lr = lane & 15, q = lane >> 4, lk = 8 * q;
+    v4f z[NLAYER - 1][RT][CT];
+    v8bf B[PF + 1][CT], Am[2][RT];
+    auto load_b = [&](int g) {  // weights of flat step g
+        const bf16* wf = g < NF ? P.wf[1 + g / NSTEP] : P.wb_frag[NHL - (g - NF) / NSTEP];
+#pragma unroll
+        for (int j = 0; j < CT; ++j) B[g % (PF + 1)][j] = *(const v8bf*)&wf[frag_index(CT * w + j, g % NSTEP, NSTEP, lane)];
+    };
+    // eight k steps against the activations (or gradients) in src, from flat step g0
+    auto product = [&](v4f(*acc)[CT], bf16(*src)[NHID], int g0) {
+        auto load_a = [&](int ks, v8bf* dst) {
+#pragma unroll
+            for (int i = 0; i < RT; ++i) dst[i] = *(const v8bf*)&src[16 * i + lr][swz(16 * i + lr, ks + lk)];
+        };
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+            for (int j = 0; j < CT; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+        load_a(0, Am[0]);
+#pragma unroll
+        for (int st = 0; st < NSTEP; ++st) {
+            const int g = g0 + st;
+            if (g + PF < 2 * NF) load_b(g + PF);
+            if (st + 1 < NSTEP) load_a(32 * (st + 1), Am[(st + 1) & 1]);
+#pragma unroll
+            for (int i = 0; i < RT; ++i)
+#pragma unroll
+                for (int j = 0; j < CT; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(B[g % (PF + 1)][j], Am[st & 1][i], acc[i][j], 0, 0, 0);
         }
-        dyb[i] = f2bf(g);
-        dyf[i] = g;
+    };
+    // column t % 256, samples 16 (t / 256) .. + 15 of an LDS tile, to [feature][sample]
+    const int tg = t / NHID, tc = NW * 64 == NHID * RT || tg < RT ? t & (NHID - 1) : NHID;
+    auto put16 = [&](bf16* dst, const v8bf& a, const v8bf& b) {
+        v8bf* o = reinterpret_cast<v8bf*>(dst + m0 + 16 * tg);
+        o[0] = a;
+        o[1] = b;
+    };
+    auto store_hT = [&](bf16(*h)[NHID], bf16* dst) {
+        if (tc >= NHID) return;
+        v8us a, b;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            a[k] = h[16 * tg + k][swz(16 * tg + k, tc)];
+            b[k] = h[16 * tg + 8 + k][swz(16 * tg + 8 + k, tc)];
+        }
+        put16(dst + (size_t)tc * P.Mp, __builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b));
+    };
+    auto store_gT = [&](float(*g)[GP], int l, int cols) {
+        if (tc >= cols) return;
+        v8f a, b;
+        float s = 0.f;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) { a[k] = g[16 * tg + k][tc]; s += a[k]; }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) { b[k] = g[16 * tg + 8 + k][tc]; s += b[k]; }
+        P.cs[l][(size_t)(m0 / 16 + tg) * cols + tc] = s;
+        put16(P.gT[l] + (size_t)tc * P.Mp, __builtin_convertvector(a, v8bf), __builtin_convertvector(b, v8bf));
+    };
+    // ---- forward.  Layer 0: k = 16 packed inputs (9 used), k 16..31 of the MFMA zero
+    {
+        v8bf a[RT];
+#pragma unroll
+        for (int i = 0; i < RT; ++i) {
+            const int row = m0 + 16 * i + lr;
+            v8f f = {};
+            if (row < P.n && q < 2) {
+                const float* xr = P.x + (size_t)(P.idx ? P.idx[row] : row) * NIN + lk;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) f[k] = (k == 0 || q == 0) ? xr[k * (q == 0)] : 0.f;
+            }
+            a[i] = __builtin_convertvector(f, v8bf);
+            if (w == 0 && q < 2) *(v8bf*)&sH[1][16 * i + lr][swz(16 * i + lr, lk)] = a[i];
+        }
+#pragma unroll
+        for (int g = 0; g < PF; ++g) load_b(g);
+#pragma unroll
+        for (int j = 0; j < CT; ++j) {
+            const v8bf b = *(const v8bf*)&P.wf[0][frag_index(CT * w + j, 0, 1, lane)];
+#pragma unroll
+            for (int i = 0; i < RT; ++i)
+                z[0][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a[i], v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        }
     }
-    sm[threadIdx.x] = l;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (threadIdx.x < s) sm[threadIdx.x] += sm[threadIdx.x + s];
+#pragma unroll
+    for (int l = 0; l < NLAYER - 1; ++l) {
+        if (l > 0) product(z[l], sH[(l - 1) & 1], (l - 1) * NSTEP);
+        // (layer 0's packed inputs lie in buffer 1 until layer 1 has been computed)
+#pragma unroll
+        for (int j = 0; j < CT; ++j) {
+            const v4f bias = *(const v4f*)&P.b[l][c0 + 16 * j + 4 * q];
+#pragma unroll
+            for (int i = 0; i < RT; ++i) {
+                const int row = 16 * i + lr, col = c0 + 16 * j + 4 * q;
+                const v4f v = z[l][i][j] + bias;
+                z[l][i][j] = v;
+                const v4f h = {silu(v.x), silu(v.y), silu(v.z), silu(v.w)};
+                *(v4bf*)&sH[l & 1][row][swz(row, col)] = __builtin_convertvector(h, v4bf);
+            }
+        }
         __syncthreads();
+        if (l == 0 && tc < NIN_P) store_hT(sH[1], P.hT[0]);
+        store_hT(sH[l & 1], P.hT[l + 1]);
+        if (l == 0) __syncthreads();  // the inputs are out before layer 1 overwrites them
     }
-    if (threadIdx.x == 0) lpart[blockIdx.x] = sm[0];
+    // output layer (first 16 columns), error and loss: wave i takes row tile i
+    constexpr int LB = (NLAYER - 2) & 1;  // buffer of the last activations
+    if (w < RT) {
+        const int i = w, row = m0 + 16 * i + lr;
+        v4f o = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < NHID; ks += 32) {
+            const v8bf b = *(const v8bf*)&P.wf[NLAYER - 1][frag_index(0, ks / 32, NSTEP, lane)];
+            const v8bf a = *(const v8bf*)&sH[LB][16 * i + lr][swz(16 * i + lr, ks + lk)];
+            o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a, o, 0, 0, 0);
+        }
+        o += *(const v4f*)&P.b[NLAYER - 1][4 * q];
+        v4f g = {}, e2 = {};
+        if (row < P.n) {
+            const float* tr = P.t + (size_t)(P.idx ? P.idx[row] : row) * NOUT;
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (4 * q + c < NOUT) {
+                    const float d = o[c] - tr[4 * q + c];
+                    e2[c] = d * d;
+                    g[c] = 2.0f * d / (float)(P.n * NOUT);
+                }
+        }
+        // loss of rows 4k .. 4k + 3: per column (0 + 2) + (1 + 3), then ((c0 + c4) + c2) + (c1 + c3)
+        v4f r;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const float u = e2[c] + __shfl_xor(e2[c], 2);
+            r[c] = u + __shfl_xor(u, 1);
+        }
+        const float r4 = __shfl(r.x, (lane & 15) + 16);  // column 4
+        if (q == 0 && (lr & 3) == 0) P.lpart[row / 4] = ((r.x + r4) + r.z) + (r.y + r.w);
+        *(v4f*)&sG[0][16 * i + lr][4 * q] = g;
+        *(v4bf*)&sH[1 - LB][16 * i + lr][swz(16 * i + lr, 4 * q)] = __builtin_convertvector(g, v4bf);
+        *(v4bf*)&sH[1 - LB][16 * i + lr][swz(16 * i + lr, 16 + 4 * q)] = v4bf{};  // k 16..31 of the one step below
+    }
+    __syncthreads();
+    // ---- backward: g of layer l - 1 from that of layer l
+    store_gT(sG[0], NLAYER - 1, 16);
+#pragma unroll
+    for (int l = NLAYER - 1; l >= 1; --l) {
+        const int src = (NLAYER - 1 - l + 1 - LB) & 1, dst = 1 - src, gb = (NLAYER - l) & 1;
+        v4f acc[RT][CT];
+        if (l == NLAYER - 1) {  // 16 of the 64 padded columns are not zero: one step
+#pragma unroll
+            for (int j = 0; j < CT; ++j) {
+                const v8bf b = *(const v8bf*)&P.wb_frag[l][frag_index(CT * w + j, 0, 1, lane)];
+#pragma unroll
+                for (int i = 0; i < RT; ++i) {
+                    const v8bf a = *(const v8bf*)&sH[src][16 * i + lr][swz(16 * i + lr, lk)];
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a, v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                }
+            }
+        } else {
+            product(acc, sH[src], NF + (NHL - l) * NSTEP);
+        }
+#pragma unroll
+        for (int j = 0; j < CT; ++j)
+#pragma unroll
+            for (int i = 0; i < RT; ++i) {
+                const int row = 16 * i + lr, col = c0 + 16 * j + 4 * q;
+                const v4f v = acc[i][j], zz = z[l - 1][i][j];
+                const v4f g = {v.x * dsilu(zz.x), v.y * dsilu(zz.y), v.z * dsilu(zz.z), v.w * dsilu(zz.w)};
+                *(v4f*)&sG[gb][row][col] = g;
+                if (l > 1) *(v4bf*)&sH[dst][row][swz(row, col)] = __builtin_convertvector(g, v4bf);
+            }
+        __syncthreads();
+        store_gT(sG[gb], l - 1, NHID);
+    }
 }
 
-// Sum of n partials by one block (strided, then a tree in LDS; fixed order).
-__global__ void __launch_bounds__(256) k_sum_partials(const float* p, int n, float scale, float* out) {
+// Weight gradients dW_l = H_l^T G_l of layers [l0, l1), split over the samples:
+// one workgroup per 64 x 64 tile and split (blockIdx.y), all layers in one
+// launch so that their tiles fill the GPU together (72 tiles x 8 splits at 8192
+// samples: 19 us).  Bound by the operands from HBM/L2 (42 MB written just before).  Both factors lie with the sample contiguous; a chunk of 64 samples
+// goes through LDS, the next one's loads under way.  The MFMA chain runs over
+// the split's samples in ascending 32-wide steps.  part: layer l's
+// [nsplit][lay_kin][lay_gcols] at its offset.
+struct MlpWgrad {
+    const bf16 *hT[NLAYER], *gT[NLAYER];
+    float* part[NLAYER];
+    int Mp, ks;  // samples, and per split (a multiple of 16)
+};
+__host__ __device__ constexpr int wg_tm(int l) { return l == 0 ? 1 : NHID / 64; }
+__host__ __device__ constexpr int wg_tn(int l) { return l == NLAYER - 1 ? 1 : NHID / 64; }
+__global__ void __launch_bounds__(256) k_wgrad(MlpWgrad P, int l0, int l1) {
+    constexpr int KC = 64, PAD = 8, VR = KC / 8;
+    __shared__ __align__(16) bf16 sA[64][KC + PAD];
+    __shared__ __align__(16) bf16 sB[64][KC + PAD];
+    int l = l0, tile = blockIdx.x;
+    while (l + 1 < l1 && tile >= wg_tm(l) * wg_tn(l)) { tile -= wg_tm(l) * wg_tn(l); ++l; }
+    const int m0 = 64 * (tile / wg_tn(l)), n0 = 64 * (tile % wg_tn(l));
+    const int rows = lay_kin(l), cols = lay_gcols(l);
+    const bf16 *A = P.hT[l], *Bt = P.gT[l];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int wm = 32 * (w >> 1), wn = 32 * (w & 1);
+    const int kb = blockIdx.y * P.ks, ke = kb + P.ks;
+    v4f acc[2][2];
+    for (int i = 0; i < 2; ++i)
+        for (int j = 0; j < 2; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    v4u ra[2], rb[2];
+    auto gload = [&](int k0) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int e = u * 256 + t, r = e / VR, kv = k0 + 8 * (e % VR);
+            ra[u] = kv < ke && m0 + r < rows ? *(const v4u*)&A[(size_t)(m0 + r) * P.Mp + kv] : v4u{0u, 0u, 0u, 0u};
+            rb[u] = kv < ke && n0 + r < cols ? *(const v4u*)&Bt[(size_t)(n0 + r) * P.Mp + kv] : v4u{0u, 0u, 0u, 0u};
+        }
+    };
+    gload(kb);
+    for (int k0 = kb; k0 < ke; k0 += KC) {
+        __syncthreads();  // the previous chunk's MFMAs have read LDS
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int e = u * 256 + t, r = e / VR, kv = 8 * (e % VR);
+            *(v4u*)&sA[r][kv] = ra[u];
+            *(v4u*)&sB[r][kv] = rb[u];
+        }
+        __syncthreads();
+        if (k0 + KC < ke) gload(k0 + KC);
+#pragma unroll
+        for (int ks = 0; ks < KC; ks += 32) {
+            v8bf a[2], b[2];
+            for (int i = 0; i < 2; ++i) a[i] = *(const v8bf*)&sA[wm + 16 * i + (lane & 15)][ks + 8 * (lane >> 4)];
+            for (int j = 0; j < 2; ++j) b[j] = *(const v8bf*)&sB[wn + 16 * j + (lane & 15)][ks + 8 * (lane >> 4)];
+            for (int i = 0; i < 2; ++i)
+                for (int j = 0; j < 2; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+    }
+    float* out = P.part[l] + (size_t)blockIdx.y * rows * cols;
+    for (int i = 0; i < 2; ++i)
+        for (int j = 0; j < 2; ++j)
+            for (int r = 0; r < 4; ++r) {
+                const int row = m0 + wm + 16 * i + 4 * (lane >> 4) + r, col = n0 + wn + 16 * j + (lane & 15);
+                if (row < rows && col < cols) out[(size_t)row * cols + col] = acc[i][j][r];
+            }
+}
+
+// The end of a step for layers [l0, l1): the splits' partials added in order,
+// then Adam on the fp32 weights with the bf16 copies refreshed (ADAM), or the
+// gradient vector written.  A thread owns 8 columns of a weight row; further
+// blocks own 64 bias columns each (the 16-sample sums of a 64-sample chunk in
+// order, four lanes of every fourth chunk, then those in order) and the last one
+// the loss (l0 = 0 only).  Bound by the partials (8.7 MB) and the optimiser state
+// (10 MB with the bf16 copies) at 8192 samples: 14 us.
+struct MlpUpdate {
+    float *w[NLAYER], *m[NLAYER], *v[NLAYER], *b[NLAYER], *mb[NLAYER], *vb[NLAYER];
+    bf16 *wb[NLAYER], *wf[NLAYER], *wb_frag[NLAYER];
+    const float *part[NLAYER], *cs[NLAYER];
+    const float* lpart;
+    float *grad, *loss;
+    int nsplit, Mp, n;
+    float lr, b1, b2, eps, c1, c2;
+};
+__device__ __forceinline__ float adam(float w, float g, float* m, float* v, const MlpUpdate& P) {
+    const float mi = P.b1 * *m + (1.f - P.b1) * g;
+    const float vi = P.b2 * *v + (1.f - P.b2) * g * g;
+    *m = mi;
+    *v = vi;
+    return w - P.lr * (mi * P.c1) / (sqrtf(vi * P.c2) + P.eps);
+}
+__host__ __device__ constexpr int upd_wblocks(int l) { return lay_kin(l) * lay_gcols(l) / 8 / 256 + (lay_kin(l) * lay_gcols(l) / 8 % 256 != 0); }
+__host__ __device__ constexpr int upd_bblocks(int l) { return (lay_gcols(l) + 63) / 64; }
+template <bool ADAM>
+__global__ void __launch_bounds__(256) k_update(MlpUpdate P, int l0, int l1) {
     __shared__ double sm[256];
+    int blk = blockIdx.x;
+    const int t = threadIdx.x;
+    for (int l = l0; l < l1; ++l) {
+        const int cols = lay_gcols(l), kout = lay_kout(l);
+        if (blk < upd_wblocks(l)) {
+            const int e = blk * 256 + t, nv = lay_kin(l) * cols / 8;
+            if (e >= nv) return;
+            const int k = e / (cols / 8), c = 8 * (e % (cols / 8));
+            const size_t n = (size_t)lay_kin(l) * cols, o = (size_t)k * cols + c, wo = (size_t)k * kout + c;
+            v8f g = {};
+            for (int s = 0; s < P.nsplit; ++s) g += *(const v8f*)&P.part[l][(size_t)s * n + o];
+            if (!ADAM) {
+                for (int u = 0; u < 8; ++u) P.grad[lay_off(l) + wo + u] = g[u];
+                return;
+            }
+            v8f w = *(const v8f*)&P.w[l][wo], m = *(const v8f*)&P.m[l][wo], v = *(const v8f*)&P.v[l][wo];
+            for (int u = 0; u < 8; ++u) {
+                float mu = m[u], vu = v[u];
+                w[u] = adam(w[u], g[u], &mu, &vu, P);
+                m[u] = mu;
+                v[u] = vu;
+            }
+            *(v8f*)&P.w[l][wo] = w;
+            *(v8f*)&P.m[l][wo] = m;
+            *(v8f*)&P.v[l][wo] = v;
+            const v8bf h = __builtin_convertvector(w, v8bf);
+            *(v8bf*)&P.wb[l][wo] = h;
+            if (l > 0)  // backward operand: row k of tile k / 16, columns c .. c + 7 of step c / 32
+                *(v8bf*)&P.wb_frag[l][frag_index(k / 16, c / 32, l == NLAYER - 1 ? 1 : NHID / 32, k % 16 + 16 * (c % 32 / 8))] = h;
+            for (int u = 0; u < 8; ++u)  // forward operand: column c + u, k within step k / 32
+                *(__bf16*)&P.wf[l][frag_index((c + u) / 16, k / 32, frag_steps(l), (c + u) % 16 + 16 * (k % 32 / 8)) + k % 8] = h[u];
+            return;
+        }
+        blk -= upd_wblocks(l);
+        if (blk < upd_bblocks(l)) {
+            const int c = blk * 64 + (t & 63), r = t >> 6, chunks = P.Mp / 64;
+            float s = 0.f;
+            if (c < cols)
+                for (int k = r; k < chunks; k += 4) {
+                    const float* p = P.cs[l] + (size_t)4 * k * cols + c;
+                    s += ((p[0] + p[cols]) + p[2 * (size_t)cols]) + p[3 * (size_t)cols];
+                }
+            float* sf = reinterpret_cast<float*>(sm);
+            sf[t] = s;
+            __syncthreads();
+            if (r == 0 && c < cols) {
+                const float g = ((sf[t] + sf[64 + t]) + sf[128 + t]) + sf[192 + t];
+                if (ADAM) P.b[l][c] = adam(P.b[l][c], g, &P.mb[l][c], &P.vb[l][c], P);
+                else P.grad[lay_off(l) + lay_kin(l) * kout + c] = g;
+            }
+            return;
+        }
+        blk -= upd_bblocks(l);
+    }
     double s = 0.0;
-    for (int i = threadIdx.x; i < n; i += 256) s += p[i];
-    sm[threadIdx.x] = s;
+    for (int i = t; i < P.Mp / 4; i += 256) s += P.lpart[i];
+    sm[t] = s;
     __syncthreads();
     for (int k = 128; k > 0; k >>= 1) {
-        if (threadIdx.x < k) sm[threadIdx.x] += sm[threadIdx.x + k];
+        if (t < k) sm[t] += sm[t + k];
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[0] = (float)(sm[0] * scale);
-}
-
-// Adam on fp32 master weights, bf16 copy refreshed.
-__global__ void k_adam(float* w, const float* g, float* m, float* v, bf16* wb, size_t n, float lr, float b1, float b2,
-                       float eps, float c1, float c2) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float gi = g[i];
-    float mi = b1 * m[i] + (1.f - b1) * gi;
-    float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    float wi = w[i] - lr * (mi * c1) / (sqrtf(vi * c2) + eps);
-    w[i] = wi;
-    if (wb) wb[i] = f2bf(wi);
-}
-
-// Mini-batch rows idx[0..b) of the device training set into the input/target buffers.
-__global__ void k_gather_batch(const float* x, const float* t, const int* idx, int b, float* xo, float* to) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= b) return;
-    int r = idx[i];
-    for (int c = 0; c < NIN; ++c) xo[(size_t)i * NIN + c] = x[(size_t)r * NIN + c];
-    for (int c = 0; c < NOUT; ++c) to[(size_t)i * NOUT + c] = t[(size_t)r * NOUT + c];
-}
-
-__global__ void k_copy1(const float* a, float* b) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) b[0] = a[0];
+    if (t == 0) *P.loss = (float)(sm[0] * (1.0f / (float)(P.n * NOUT)));
 }
 
 // y[i][0..NOUT) of the padded output rows, packed densely for one host copy
@@ -478,21 +755,21 @@ struct ofx_mlp {
     int kin[NLAYER], kout[NLAYER];        // padded shapes of each layer
     float *w[NLAYER], *b[NLAYER];          // fp32 master
     bf16 *wb[NLAYER], *wt[NLAYER];         // bf16 copy and its transpose
-    bf16* wf[NLAYER];                      // bf16 copy in MFMA operand order (frag_index)
+    bf16 *wf[NLAYER], *wb_frag[NLAYER];    // bf16 copies in MFMA operand order (frag_index)
     float *mw[NLAYER], *vw[NLAYER], *mb[NLAYER], *vb[NLAYER];
-    float *gw[NLAYER], *gb[NLAYER];        // gradients
+    float* grad = nullptr;                 // gradient vector, in the parameters' layout
     int step = 0;
-    // per-call buffers, sized for `cap` samples
-    int cap = 0, max_split = 1;
-    bf16* h[NLAYER];   // layer inputs: h[0] = packed inputs, h[l] = silu(z[l-1])
-    float* z[NLAYER - 1];
-    float* y = nullptr;
-    float* tgt = nullptr;
+    // layered forward pass, sized for `cap` samples
+    int cap = 0;
+    bf16* h[NLAYER];                       // layer inputs: h[0] = packed inputs
+    float *y = nullptr, *yd = nullptr;     // padded and dense outputs
     float* xin = nullptr;
-    bf16 *dyb = nullptr, *ht = nullptr, *gt = nullptr;  // ht, gt: transposed factors of a weight gradient
-    float *dyf = nullptr, *gz = nullptr;  // fp32 gradient of the current layer's pre-activation
-    bf16 *gzb = nullptr, *gzb2 = nullptr;
-    float *part = nullptr, *lpart = nullptr, *loss = nullptr, *cpart = nullptr;
+    std::vector<void*> fwd_allocs;
+    // gradients, sized for `tcap` samples: one block (MlpTrain, MlpWgrad)
+    int tcap = 0;
+    char* tbuf = nullptr;
+    bf16 *hT[NLAYER], *gT[NLAYER];
+    float *cs[NLAYER], *lpart = nullptr, *part = nullptr, *loss = nullptr, *tx = nullptr, *tt = nullptr;
     float *io_x = nullptr, *io_y = nullptr;  // device copies of a one-kernel forward's inputs and outputs
     int io_cap = 0;
     int fwd_variant = 1;  // inference forward pass: 0 layer by layer, 1 one kernel (k_mlp_forward)
@@ -509,35 +786,81 @@ int mlp_alloc(ofx_mlp* n, void** p, size_t bytes) {
     return 0;
 }
 
-int mlp_reserve(ofx_mlp* n, int samples) {
-    int Mp = (samples + 63) / 64 * 64;
+// Buffers of a layered forward pass.
+int layered_reserve(ofx_mlp* n, int samples) {
+    const int Mp = (samples + 63) / 64 * 64;
     if (Mp <= n->cap) return 0;
-    // grow: drop the old per-call buffers (parameters are the first allocations)
     OFX_HIP(hipStreamSynchronize(n->stream));
-    size_t keep = NLAYER * 12;
-    for (size_t i = keep; i < n->allocs.size(); ++i) (void)hipFree(n->allocs[i]);
-    n->allocs.resize(std::min(keep, n->allocs.size()));
-    auto A = [&](void** p, size_t bytes) { return mlp_alloc(n, p, bytes); };
+    for (void* p : n->fwd_allocs) (void)hipFree(p);
+    n->fwd_allocs.clear();
+    n->cap = 0;
+    auto A = [&](void** p, size_t bytes) -> int {
+        if (hipMalloc(p, bytes) != hipSuccess) { set_error("mlp: out of device memory"); return OFX_ENOMEM; }
+        n->fwd_allocs.push_back(*p);
+        return 0;
+    };
     for (int l = 0; l < NLAYER; ++l) OFX_TRY(A((void**)&n->h[l], sizeof(bf16) * (size_t)Mp * n->kin[l]));
-    for (int l = 0; l < NLAYER - 1; ++l) OFX_TRY(A((void**)&n->z[l], sizeof(float) * (size_t)Mp * NHID));
     OFX_TRY(A((void**)&n->y, sizeof(float) * (size_t)Mp * NOUT_P));
-    OFX_TRY(A((void**)&n->tgt, sizeof(float) * (size_t)Mp * NOUT));
+    OFX_TRY(A((void**)&n->yd, sizeof(float) * (size_t)Mp * NOUT));
     OFX_TRY(A((void**)&n->xin, sizeof(float) * (size_t)Mp * NIN));
-    OFX_TRY(A((void**)&n->dyb, sizeof(bf16) * (size_t)Mp * NOUT_P));
-    OFX_TRY(A((void**)&n->dyf, sizeof(float) * (size_t)Mp * NOUT_P));
-    OFX_TRY(A((void**)&n->ht, sizeof(bf16) * (size_t)Mp * NHID));
-    OFX_TRY(A((void**)&n->gt, sizeof(bf16) * (size_t)Mp * NHID));
-    OFX_TRY(A((void**)&n->gz, sizeof(float) * (size_t)Mp * NHID));
-    OFX_TRY(A((void**)&n->gzb, sizeof(bf16) * (size_t)Mp * NHID));
-    OFX_TRY(A((void**)&n->gzb2, sizeof(bf16) * (size_t)Mp * NHID));
-    // weight_grad doubles the split count while a split exceeds SPLITK_CHUNK
-    // samples, so it stays below 2 Mp / SPLITK_CHUNK; one more slot holds the sum
-    n->max_split = 2 * (Mp / SPLITK_CHUNK) + 1;
-    OFX_TRY(A((void**)&n->part, sizeof(float) * (size_t)(n->max_split + 1) * NHID * NHID));
-    OFX_TRY(A((void**)&n->lpart, sizeof(float) * ((size_t)Mp * NOUT_P / 256 + 1)));
-    OFX_TRY(A((void**)&n->loss, sizeof(float) * 4));
-    OFX_TRY(A((void**)&n->cpart, sizeof(float) * ((size_t)Mp / COLSUM_ROWS * NHID + NHID)));
     n->cap = Mp;
+    return 0;
+}
+
+// Splits of a weight gradient over Mp samples: at most SPLITK_CHUNK samples each
+// while Mp divides into multiples of 16.
+int wgrad_splits(int Mp) {
+    int ns = 1;
+    while (Mp / ns > SPLITK_CHUNK && Mp % (ns * 2) == 0 && (Mp / (ns * 2)) % 16 == 0) ns *= 2;
+    return ns;
+}
+// All layers' partials together up to this many splits, one layer's beyond
+// (64: 70 MB; 128 more layers' tiles in flight would not fill the GPU any better).
+constexpr int SPLITS_TOGETHER = 64;
+constexpr int wgrad_elems(int l) { return lay_kin(l) * lay_gcols(l); }
+
+// Buffers of the gradients of `samples` samples (every element a kernel reads is
+// written first).
+int train_reserve(ofx_mlp* n, int samples) {
+    const int Mp = (samples + 63) / 64 * 64;
+    if (Mp <= n->tcap) return 0;
+    OFX_HIP(hipStreamSynchronize(n->stream));
+    if (n->tbuf) (void)hipFree(n->tbuf);
+    n->tbuf = nullptr;
+    n->tcap = 0;
+    // a smaller call may split into more pieces than a larger one (an odd
+    // multiple of 64 stops early), so the partials are sized for any size up to Mp:
+    // wgrad_splits(m) < 2 m / SPLITK_CHUNK + 1
+    const size_t ns = 2 * (size_t)(Mp / SPLITK_CHUNK) + 1;
+    size_t all = 0, one = 0;
+    for (int l = 0; l < NLAYER; ++l) { all += wgrad_elems(l); one = std::max<size_t>(one, wgrad_elems(l)); }
+    const size_t pel = std::max(std::min<size_t>(ns, SPLITS_TOGETHER) * all, ns * one);
+    size_t o = 0;
+    auto take = [&](size_t bytes) { size_t at = o; o += (bytes + 255) / 256 * 256; return at; };
+    size_t hT[NLAYER], gT[NLAYER], cs[NLAYER];
+    for (int l = 0; l < NLAYER; ++l) {
+        hT[l] = take(sizeof(bf16) * (size_t)Mp * lay_kin(l));
+        gT[l] = take(sizeof(bf16) * (size_t)Mp * lay_gcols(l));
+        cs[l] = take(sizeof(float) * (size_t)(Mp / 16) * lay_gcols(l));
+    }
+    const size_t lp = take(sizeof(float) * (size_t)(Mp / 4)), lo = take(sizeof(float)), pa = take(sizeof(float) * pel),
+                 tx = take(sizeof(float) * (size_t)Mp * NIN), tt = take(sizeof(float) * (size_t)Mp * NOUT);
+    if (hipMalloc((void**)&n->tbuf, o) != hipSuccess) {
+        n->tbuf = nullptr;
+        set_error("mlp: out of device memory");
+        return OFX_ENOMEM;
+    }
+    for (int l = 0; l < NLAYER; ++l) {
+        n->hT[l] = (bf16*)(n->tbuf + hT[l]);
+        n->gT[l] = (bf16*)(n->tbuf + gT[l]);
+        n->cs[l] = (float*)(n->tbuf + cs[l]);
+    }
+    n->lpart = (float*)(n->tbuf + lp);
+    n->loss = (float*)(n->tbuf + lo);
+    n->part = (float*)(n->tbuf + pa);
+    n->tx = (float*)(n->tbuf + tx);
+    n->tt = (float*)(n->tbuf + tt);
+    n->tcap = Mp;
     return 0;
 }
 
@@ -560,71 +883,44 @@ int io_reserve(ofx_mlp* n, int samples) {
 
 // C = A Bt^T (see k_gemm): A [M][K], Bt [N][K].
 template <int EPI>
-int gemm_on(hipStream_t st, const bf16* A, int lda, const bf16* Bt, int ldb, int M, int N, int K, int nsplit, float* Cf,
-            bf16* Cb, int ldc, const float* bias, const float* zin, float* zout) {
-    if (M % 64 || N % 64 || K % 16 || K % nsplit || (K / nsplit) % 16) {
+int gemm_on(hipStream_t st, const bf16* A, int lda, const bf16* Bt, int ldb, int M, int N, int K, float* Cf, bf16* Cb,
+            int ldc, const float* bias) {
+    if (M % 64 || N % 64 || K % 16) {
         set_error("mlp: GEMM shape not tiled");
         return OFX_EINVAL;
     }
-    int kc = K / nsplit;
     // 128-row tiles (and 128 columns where N allows) once there are rows
     // enough to fill the GPU with them: fewer L2 re-reads of both operands
-    if (nsplit == 1 && M % 128 == 0 && M >= 65536 && kc % 64 == 0) {
-        if (N % 128 == 0)
-            k_gemm<EPI, 64, 128, 128><<<dim3(N / 128, M / 128, 1), 256, 0, st>>>(A, lda, Bt, ldb, kc, M, Cf, Cb, ldc,
-                                                                                 bias, zin, zout);
-        else
-            k_gemm<EPI, 64, 128, 64><<<dim3(N / 64, M / 128, 1), 256, 0, st>>>(A, lda, Bt, ldb, kc, M, Cf, Cb, ldc,
-                                                                               bias, zin, zout);
+    if (M % 128 == 0 && M >= 65536 && K % 64 == 0) {
+        if (N % 128 == 0) k_gemm<EPI, 64, 128, 128><<<dim3(N / 128, M / 128), 256, 0, st>>>(A, lda, Bt, ldb, K, Cf, Cb, ldc, bias);
+        else k_gemm<EPI, 64, 128, 64><<<dim3(N / 64, M / 128), 256, 0, st>>>(A, lda, Bt, ldb, K, Cf, Cb, ldc, bias);
     } else {
-        dim3 grid(N / 64, M / 64, nsplit);
-        if (kc % 64 == 0)
-            k_gemm<EPI, 64, 64, 64><<<grid, 256, 0, st>>>(A, lda, Bt, ldb, kc, M, Cf, Cb, ldc, bias, zin, zout);
-        else
-            k_gemm<EPI, 32, 64, 64><<<grid, 256, 0, st>>>(A, lda, Bt, ldb, kc, M, Cf, Cb, ldc, bias, zin, zout);
+        dim3 grid(N / 64, M / 64);
+        if (K % 64 == 0) k_gemm<EPI, 64, 64, 64><<<grid, 256, 0, st>>>(A, lda, Bt, ldb, K, Cf, Cb, ldc, bias);
+        else k_gemm<EPI, 32, 64, 64><<<grid, 256, 0, st>>>(A, lda, Bt, ldb, K, Cf, Cb, ldc, bias);
     }
     OFX_HIP(hipGetLastError());
     return 0;
 }
 
-template <int EPI>
-int gemm(ofx_mlp* n, const bf16* A, int lda, const bf16* Bt, int ldb, int M, int N, int K, int nsplit, float* Cf, bf16* Cb,
-         int ldc, const float* bias, const float* zin, float* zout) {
-    return gemm_on<EPI>(n->stream, A, lda, Bt, ldb, M, N, K, nsplit, Cf, Cb, ldc, bias, zin, zout);
+// All layers on packed inputs in [Mp][16] -> padded outputs yp [Mp][64]; layer
+// l's output in act(l).
+template <class ACT>
+int forward_layered(const ofx_mlp* n, hipStream_t st, const bf16* in, int Mp, ACT act, float* yp) {
+    const bf16* h = in;
+    for (int l = 0; l < NLAYER - 1; ++l) {
+        OFX_TRY(gemm_on<EPI_BIAS_SILU>(st, h, n->kin[l], n->wt[l], n->kin[l], Mp, n->kout[l], n->kin[l], nullptr, act(l),
+                                       n->kout[l], n->b[l]));
+        h = act(l);
+    }
+    const int L = NLAYER - 1;
+    return gemm_on<EPI_BIAS>(st, h, n->kin[L], n->wt[L], n->kin[L], Mp, n->kout[L], n->kin[L], yp, nullptr, n->kout[L],
+                             n->b[L]);
 }
 
 int transpose(ofx_mlp* n, const bf16* in, int R, int C, bf16* out, int Cp) {
     dim3 grid((std::max(C, Cp) + 31) / 32, (R + 31) / 32);
     k_transpose<<<grid, dim3(32, 8), 0, n->stream>>>(in, R, C, out, Cp);
-    OFX_HIP(hipGetLastError());
-    return 0;
-}
-
-// Weight gradient dW[kin x kout] = H^T[kin x Mp] G[Mp x kout], split over
-// samples: both factors transposed so that k (the sample) is contiguous.
-int weight_grad(ofx_mlp* n, int l, const bf16* H, const bf16* G, int Mp) {
-    int ki = n->kin[l], ko = n->kout[l];
-    int rows = (ki + 63) / 64 * 64;  // the input layer's 16 rows padded to one tile
-    OFX_TRY(transpose(n, H, Mp, ki, n->ht, rows));
-    OFX_TRY(transpose(n, G, Mp, ko, n->gt, ko));
-    int nsplit = 1;
-    while (Mp / nsplit > SPLITK_CHUNK && Mp % (nsplit * 2) == 0 && (Mp / (nsplit * 2)) % 16 == 0) nsplit *= 2;
-    if (nsplit > n->max_split || Mp > n->cap) { set_error("mlp: split-K buffer too small"); return OFX_EINVAL; }
-    OFX_TRY(gemm<EPI_PARTIAL>(n, n->ht, Mp, n->gt, Mp, rows, ko, Mp, nsplit, n->part, nullptr, ko, nullptr, nullptr, nullptr));
-    size_t cnt = (size_t)rows * ko;
-    // rows beyond kin are zero inputs (their sums are zero); keep the first kin rows
-    k_splitk_sum<<<(unsigned)((cnt + 255) / 256), 256, 0, n->stream>>>(n->part, nsplit, cnt, n->part + (size_t)nsplit * cnt);
-    OFX_HIP(hipGetLastError());
-    OFX_HIP(hipMemcpyAsync(n->gw[l], n->part + (size_t)nsplit * cnt, sizeof(float) * (size_t)ki * ko,
-                           hipMemcpyDeviceToDevice, n->stream));
-    return 0;
-}
-
-int colsum(ofx_mlp* n, const float* g, int M, int N, float* out) {
-    int chunks = (M + COLSUM_ROWS - 1) / COLSUM_ROWS;
-    if ((size_t)chunks * N > (size_t)n->cap / COLSUM_ROWS * NHID + NHID) { set_error("mlp: column-sum buffer too small"); return OFX_EINVAL; }
-    k_colsum_part<<<dim3((N + 63) / 64, chunks), 256, 0, n->stream>>>(g, M, N, n->cpart);
-    k_colsum_final<<<(N + 63) / 64, 256, 0, n->stream>>>(n->cpart, chunks, N, out);
     OFX_HIP(hipGetLastError());
     return 0;
 }
@@ -655,68 +951,67 @@ int forward_fused(const ofx_mlp* n, hipStream_t st, const float* x, int nsamp, f
     return forward_shape<4, 8, 4, true>(n, st, x, nsamp, y);
 }
 
-// keep_z: store the pre-activations (a backward pass follows).
-int forward(ofx_mlp* n, int Mp, bool keep_z) {
-    for (int l = 0; l < NLAYER - 1; ++l)
-        OFX_TRY(gemm<EPI_BIAS_SILU>(n, n->h[l], n->kin[l], n->wt[l], n->kin[l], Mp, n->kout[l], n->kin[l], 1, nullptr,
-                                    n->h[l + 1], n->kout[l], n->b[l], nullptr, keep_z ? n->z[l] : nullptr));
-    int L = NLAYER - 1;
-    OFX_TRY(gemm<EPI_BIAS>(n, n->h[L], n->kin[L], n->wt[L], n->kin[L], Mp, n->kout[L], n->kin[L], 1, n->y, nullptr,
-                           n->kout[L], n->b[L], nullptr, nullptr));
-    return 0;
-}
-
-// The operand-ordered weights of the one-kernel forward.
+// The operand-ordered weights of the one-kernel forward and of training.
 int refresh_frag(ofx_mlp* n) {
     MlpFrag P;
     int vec = 0;
-    for (int l = 0; l < NLAYER; ++l) { P.wb[l] = n->wb[l]; P.wf[l] = n->wf[l]; vec += 64 * frag_tiles(l) * frag_steps(l); }
+    for (int l = 0; l < NLAYER; ++l) {
+        P.wb[l] = n->wb[l]; P.wf[l] = n->wf[l]; P.wb_frag[l] = n->wb_frag[l];
+        vec += 64 * frag_tiles(l) * frag_steps(l) + (l == 0 ? 0 : 64 * (NHID / 16) * (l == NLAYER - 1 ? 1 : NHID / 32));
+    }
     k_frag<<<(vec + 255) / 256, 256, 0, n->stream>>>(P);
     OFX_HIP(hipGetLastError());
     return 0;
 }
 
-// The transposed bf16 weights [kout][kin] that the layered forward products
-// read, refreshed whenever the bf16 weights change (and the operand-ordered
-// ones, for training at its end only).
-int refresh_wt(ofx_mlp* n, bool frag = true) {
-    if (frag) OFX_TRY(refresh_frag(n));
+// The transposed bf16 weights [kout][kin] that the layered forward products read.
+int refresh_wt(ofx_mlp* n) {
     for (int l = 0; l < NLAYER; ++l) OFX_TRY(transpose(n, n->wb[l], n->kin[l], n->kout[l], n->wt[l], n->kout[l]));
     return 0;
 }
 
-int backward(ofx_mlp* n, int nsamp, int Mp) {
-    int L = NLAYER - 1;
-    int nb = (Mp * NOUT_P + 255) / 256;
-    k_mse<<<nb, 256, 0, n->stream>>>(n->y, n->tgt, nsamp, Mp, n->dyb, n->dyf, n->lpart);
-    k_sum_partials<<<1, 256, 0, n->stream>>>(n->lpart, nb, 1.0f / (float)(nsamp * NOUT), n->loss);
-    OFX_HIP(hipGetLastError());
-    // output layer
-    OFX_TRY(weight_grad(n, L, n->h[L], n->dyb, Mp));
-    OFX_TRY(colsum(n, n->dyf, Mp, NOUT_P, n->gb[L]));
-    const bf16* g = n->dyb;
-    bf16* gnext = n->gzb;
-    for (int l = L; l >= 1; --l) {
-        // gradient of layer l-1's pre-activation: (G W_l^T) * silu'(z_{l-1});
-        // the second factor read along k is W_l itself
-        OFX_TRY(gemm<EPI_DSILU>(n, g, n->kout[l], n->wb[l], n->kout[l], Mp, n->kin[l], n->kout[l], 1, n->gz, gnext,
-                                n->kin[l], nullptr, n->z[l - 1], nullptr));
-        OFX_TRY(weight_grad(n, l - 1, n->h[l - 1], gnext, Mp));
-        OFX_TRY(colsum(n, n->gz, Mp, NHID, n->gb[l - 1]));
-        OFX_HIP(hipGetLastError());
-        g = gnext;
-        gnext = (gnext == n->gzb) ? n->gzb2 : n->gzb;
+// Loss and gradients of n samples (rows idx of x, t; null: all of them), then
+// an Adam step or the gradient vector.  The loss goes to loss.
+int grad_step(ofx_mlp* n, const float* x, const float* t, const int* idx, int nsamp, bool adam, float lr, float* loss) {
+    const int Mp = (nsamp + 63) / 64 * 64;
+    MlpTrain T;
+    for (int l = 0; l < NLAYER; ++l) {
+        T.wf[l] = n->wf[l]; T.wb_frag[l] = n->wb_frag[l]; T.b[l] = n->b[l];
+        T.hT[l] = n->hT[l]; T.gT[l] = n->gT[l]; T.cs[l] = n->cs[l];
     }
-    return 0;
-}
-
-int load_batch(ofx_mlp* n, const float* x, const float* t, int nsamp, bool on_device) {
-    OFX_TRY(mlp_reserve(n, nsamp));
-    int Mp = (nsamp + 63) / 64 * 64;
-    hipMemcpyKind kind = on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
-    OFX_HIP(hipMemcpyAsync(n->xin, x, sizeof(float) * (size_t)nsamp * NIN, kind, n->stream));
-    if (t) OFX_HIP(hipMemcpyAsync(n->tgt, t, sizeof(float) * (size_t)nsamp * NOUT, kind, n->stream));
-    k_pack_inputs<<<(Mp * NIN_P + 255) / 256, 256, 0, n->stream>>>(n->xin, nsamp, Mp, n->h[0]);
+    T.lpart = n->lpart; T.x = x; T.t = t; T.idx = idx; T.n = nsamp; T.Mp = Mp;
+    if (Mp <= 16 * 256) k_mlp_grad<1, 8, 8><<<Mp / 16, 512, 0, n->stream>>>(T);
+    else k_mlp_grad<2, 8, 3><<<Mp / 32, 512, 0, n->stream>>>(T);
+    OFX_HIP(hipGetLastError());
+    MlpWgrad G;
+    MlpUpdate U;
+    const int ns = wgrad_splits(Mp);
+    const bool together = ns <= SPLITS_TOGETHER;
+    size_t o = 0;
+    for (int l = 0; l < NLAYER; ++l) {
+        G.hT[l] = n->hT[l]; G.gT[l] = n->gT[l];
+        G.part[l] = n->part + o;
+        if (together) o += (size_t)ns * wgrad_elems(l);
+        U.w[l] = n->w[l]; U.m[l] = n->mw[l]; U.v[l] = n->vw[l]; U.b[l] = n->b[l]; U.mb[l] = n->mb[l]; U.vb[l] = n->vb[l];
+        U.wb[l] = n->wb[l]; U.wf[l] = n->wf[l]; U.wb_frag[l] = n->wb_frag[l];
+        U.part[l] = G.part[l]; U.cs[l] = n->cs[l];
+    }
+    G.Mp = Mp; G.ks = Mp / ns;
+    U.lpart = n->lpart; U.grad = n->grad; U.loss = loss; U.nsplit = ns; U.Mp = Mp; U.n = nsamp;
+    U.lr = lr; U.b1 = 0.9f; U.b2 = 0.999f; U.eps = 1e-8f; U.c1 = U.c2 = 0.f;
+    if (adam) {
+        ++n->step;
+        U.c1 = 1.0f / (1.0f - std::pow(U.b1, (float)n->step));
+        U.c2 = 1.0f / (1.0f - std::pow(U.b2, (float)n->step));
+    }
+    for (int l0 = 0; l0 < NLAYER; l0 = together ? NLAYER : l0 + 1) {
+        const int l1 = together ? NLAYER : l0 + 1;
+        int tiles = 0, blocks = l0 == 0 ? 1 : 0;
+        for (int l = l0; l < l1; ++l) { tiles += wg_tm(l) * wg_tn(l); blocks += upd_wblocks(l) + upd_bblocks(l); }
+        k_wgrad<<<dim3(tiles, ns), 256, 0, n->stream>>>(G, l0, l1);
+        if (adam) k_update<true><<<blocks, 256, 0, n->stream>>>(U, l0, l1);
+        else k_update<false><<<blocks, 256, 0, n->stream>>>(U, l0, l1);
+    }
     OFX_HIP(hipGetLastError());
     return 0;
 }
@@ -783,7 +1078,7 @@ int ofx_mlp_create(ofx_mlp** out, int device, unsigned long long seed) {
     }
     unsigned char* sp = nullptr;  // the allocation-free forward's work array on this device
     rc = scratch_address(device, &sp);
-    // parameters first (mlp_reserve keeps the first NLAYER * 12 allocations)
+    if (!rc) { void* p; rc = mlp_alloc(n, &p, sizeof(float) * lay_off(NLAYER)); n->grad = (float*)p; }
     std::vector<float> hw, hb;
     uint64_t s = seed * 6364136223846793005ull + 1442695040888963407ull;
     auto urand = [&]() {  // uniform in [-1, 1)
@@ -808,10 +1103,8 @@ int ofx_mlp_create(ofx_mlp** out, int device, unsigned long long seed) {
         if (!rc) { rc = mlp_alloc(n, &p, sizeof(float) * nw); n->vw[l] = (float*)p; }
         if (!rc) { rc = mlp_alloc(n, &p, sizeof(float) * n->kout[l]); n->mb[l] = (float*)p; }
         if (!rc) { rc = mlp_alloc(n, &p, sizeof(float) * n->kout[l]); n->vb[l] = (float*)p; }
-        if (!rc) { rc = mlp_alloc(n, &p, sizeof(float) * nw); n->gw[l] = (float*)p; }
-        if (!rc) { rc = mlp_alloc(n, &p, sizeof(float) * n->kout[l]); n->gb[l] = (float*)p; }
         if (!rc) { rc = mlp_alloc(n, &p, sizeof(bf16) * 512 * frag_tiles(l) * frag_steps(l)); n->wf[l] = (bf16*)p; }
-        if (!rc) { rc = mlp_alloc(n, &p, 16); }  // a spare slot keeps the count at 12 per layer
+        if (!rc) { rc = mlp_alloc(n, &p, sizeof(bf16) * 512 * (NHID / 16) * (NHID / 32)); n->wb_frag[l] = (bf16*)p; }
         if (!rc && hipMemcpyAsync(n->w[l], hw.data(), sizeof(float) * nw, hipMemcpyHostToDevice, n->stream) != hipSuccess)
             rc = OFX_EHIP;
         if (!rc) {
@@ -821,6 +1114,7 @@ int ofx_mlp_create(ofx_mlp** out, int device, unsigned long long seed) {
         if (!rc && hipStreamSynchronize(n->stream) != hipSuccess) rc = OFX_EHIP;
     }
     if (!rc) rc = refresh_wt(n);
+    if (!rc) rc = refresh_frag(n);
     if (rc) {
         ofx_mlp_destroy(n);
         return rc;
@@ -834,7 +1128,9 @@ int ofx_mlp_destroy(ofx_mlp* n) {
     (void)hipSetDevice(n->device);
     if (n->stream) (void)hipStreamSynchronize(n->stream);
     for (void* p : n->allocs) (void)hipFree(p);
+    for (void* p : n->fwd_allocs) (void)hipFree(p);
     if (n->io_x) (void)hipFree(n->io_x);
+    if (n->tbuf) (void)hipFree(n->tbuf);
     if (n->stream) (void)hipStreamDestroy(n->stream);
     delete n;
     return 0;
@@ -848,38 +1144,37 @@ int ofx_mlp_param_count(ofx_mlp* n, int* count) {
     return 0;
 }
 
-// Parameters (or gradients) as one fp32 vector: for each layer W[kin_p][kout_p]
+// Parameters as one fp32 vector: for each layer W[kin_p][kout_p]
 // then b[kout_p] (padded shapes: 16/256/.../256 -> 256/.../64).
-static int mlp_copy(ofx_mlp* n, float* host, bool grads, bool to_device) {
-    size_t o = 0;
+static int mlp_copy(ofx_mlp* n, float* host, bool to_device) {
     for (int l = 0; l < NLAYER; ++l) {
-        size_t nw = (size_t)n->kin[l] * n->kout[l];
-        float* dw = grads ? n->gw[l] : n->w[l];
-        float* db = grads ? n->gb[l] : n->b[l];
+        size_t nw = (size_t)n->kin[l] * n->kout[l], o = lay_off(l);
         if (to_device) {
-            OFX_HIP(hipMemcpyAsync(dw, host + o, sizeof(float) * nw, hipMemcpyHostToDevice, n->stream));
-            OFX_HIP(hipMemcpyAsync(db, host + o + nw, sizeof(float) * n->kout[l], hipMemcpyHostToDevice, n->stream));
-            if (!grads) k_to_bf16<<<(unsigned)((nw + 255) / 256), 256, 0, n->stream>>>(n->w[l], nw, n->wb[l]);
+            OFX_HIP(hipMemcpyAsync(n->w[l], host + o, sizeof(float) * nw, hipMemcpyHostToDevice, n->stream));
+            OFX_HIP(hipMemcpyAsync(n->b[l], host + o + nw, sizeof(float) * n->kout[l], hipMemcpyHostToDevice, n->stream));
+            k_to_bf16<<<(unsigned)((nw + 255) / 256), 256, 0, n->stream>>>(n->w[l], nw, n->wb[l]);
         } else {
-            OFX_HIP(hipMemcpyAsync(host + o, dw, sizeof(float) * nw, hipMemcpyDeviceToHost, n->stream));
-            OFX_HIP(hipMemcpyAsync(host + o + nw, db, sizeof(float) * n->kout[l], hipMemcpyDeviceToHost, n->stream));
+            OFX_HIP(hipMemcpyAsync(host + o, n->w[l], sizeof(float) * nw, hipMemcpyDeviceToHost, n->stream));
+            OFX_HIP(hipMemcpyAsync(host + o + nw, n->b[l], sizeof(float) * n->kout[l], hipMemcpyDeviceToHost, n->stream));
         }
-        o += nw + n->kout[l];
     }
-    if (to_device && !grads) OFX_TRY(refresh_wt(n));
+    if (to_device) {
+        OFX_TRY(refresh_wt(n));
+        OFX_TRY(refresh_frag(n));
+    }
     OFX_HIP(hipStreamSynchronize(n->stream));
     return 0;
 }
 
 int ofx_mlp_get_params(ofx_mlp* n, float* host) {
     if (!n || !host) { set_error("null argument"); return OFX_EINVAL; }
-    return mlp_copy(n, host, false, false);
+    return mlp_copy(n, host, false);
 }
 
 int ofx_mlp_set_params(ofx_mlp* n, const float* host) {
     if (!n || !host) { set_error("null argument"); return OFX_EINVAL; }
     n->step = 0;
-    return mlp_copy(n, const_cast<float*>(host), false, true);
+    return mlp_copy(n, const_cast<float*>(host), true);
 }
 
 int ofx_mlp_forward(ofx_mlp* n, const float* x, int nsamp, float* y) {
@@ -892,12 +1187,14 @@ int ofx_mlp_forward(ofx_mlp* n, const float* x, int nsamp, float* y) {
         OFX_TRY(forward_fused(n, n->stream, n->io_x, nsamp, n->io_y));
         OFX_HIP(hipMemcpyAsync(y, n->io_y, sizeof(float) * cnt, hipMemcpyDeviceToHost, n->stream));
     } else {
-        OFX_TRY(load_batch(n, x, nullptr, nsamp, false));
-        OFX_TRY(forward(n, (nsamp + 63) / 64 * 64, false));
-        // tgt (Mp x NOUT floats) is free in a forward-only call: pack there, copy once
-        k_pack_outputs<<<(unsigned)((cnt + 255) / 256), 256, 0, n->stream>>>(n->y, nsamp, n->tgt);
+        OFX_TRY(layered_reserve(n, nsamp));
+        const int Mp = (nsamp + 63) / 64 * 64;
+        OFX_HIP(hipMemcpyAsync(n->xin, x, sizeof(float) * (size_t)nsamp * NIN, hipMemcpyHostToDevice, n->stream));
+        k_pack_inputs<<<(Mp * NIN_P + 255) / 256, 256, 0, n->stream>>>(n->xin, nsamp, Mp, n->h[0]);
+        OFX_TRY(forward_layered(n, n->stream, n->h[0], Mp, [&](int l) { return n->h[l + 1]; }, n->y));
+        k_pack_outputs<<<(unsigned)((cnt + 255) / 256), 256, 0, n->stream>>>(n->y, nsamp, n->yd);
         OFX_HIP(hipGetLastError());
-        OFX_HIP(hipMemcpyAsync(y, n->tgt, sizeof(float) * cnt, hipMemcpyDeviceToHost, n->stream));
+        OFX_HIP(hipMemcpyAsync(y, n->yd, sizeof(float) * cnt, hipMemcpyDeviceToHost, n->stream));
     }
     OFX_HIP(hipStreamSynchronize(n->stream));
     return 0;
@@ -920,15 +1217,7 @@ int ofx_mlp_forward_noalloc(ofx_mlp* n, const float* x_dev, int nsamp, float* y_
     const int Mp = (nsamp + 63) / 64 * 64;
     k_pack_inputs<<<(Mp * NIN_P + 255) / 256, 256, 0, st>>>(x_dev, nsamp, Mp, in);
     OFX_HIP(hipGetLastError());
-    const bf16* h = in;
-    for (int l = 0; l < NLAYER - 1; ++l) {
-        OFX_TRY(gemm_on<EPI_BIAS_SILU>(st, h, n->kin[l], n->wt[l], n->kin[l], Mp, n->kout[l], n->kin[l], 1, nullptr,
-                                       act[l & 1], n->kout[l], n->b[l], nullptr, nullptr));
-        h = act[l & 1];
-    }
-    const int L = NLAYER - 1;
-    OFX_TRY(gemm_on<EPI_BIAS>(st, h, n->kin[L], n->wt[L], n->kin[L], Mp, n->kout[L], n->kin[L], 1, yp, nullptr,
-                              n->kout[L], n->b[L], nullptr, nullptr));
+    OFX_TRY(forward_layered(n, st, in, Mp, [&](int l) { return act[l & 1]; }, yp));
     size_t cnt = (size_t)nsamp * NOUT;
     k_pack_outputs<<<(unsigned)((cnt + 255) / 256), 256, 0, st>>>(yp, nsamp, y_dev);
     OFX_HIP(hipGetLastError());
@@ -944,33 +1233,14 @@ int ofx_mlp_set_forward_variant(ofx_mlp* n, int variant) {
 int ofx_mlp_gradients(ofx_mlp* n, const float* x, const float* t, int nsamp, float* loss, float* grads) {
     if (!n || !x || !t || nsamp < 1 || nsamp > MLP_MAXN) { set_error("mlp_gradients: bad arguments"); return OFX_EINVAL; }
     OFX_HIP(hipSetDevice(n->device));
-    OFX_TRY(load_batch(n, x, t, nsamp, false));
-    int Mp = (nsamp + 63) / 64 * 64;
-    OFX_TRY(forward(n, Mp, true));
-    OFX_TRY(backward(n, nsamp, Mp));
+    OFX_TRY(train_reserve(n, nsamp));
+    OFX_HIP(hipMemcpyAsync(n->tx, x, sizeof(float) * (size_t)nsamp * NIN, hipMemcpyHostToDevice, n->stream));
+    OFX_HIP(hipMemcpyAsync(n->tt, t, sizeof(float) * (size_t)nsamp * NOUT, hipMemcpyHostToDevice, n->stream));
+    OFX_TRY(grad_step(n, n->tx, n->tt, nullptr, nsamp, false, 0.f, n->loss));
     if (loss) OFX_HIP(hipMemcpyAsync(loss, n->loss, sizeof(float), hipMemcpyDeviceToHost, n->stream));
+    if (grads) OFX_HIP(hipMemcpyAsync(grads, n->grad, sizeof(float) * lay_off(NLAYER), hipMemcpyDeviceToHost, n->stream));
     OFX_HIP(hipStreamSynchronize(n->stream));
-    if (grads) OFX_TRY(mlp_copy(n, grads, true, false));
     return 0;
-}
-
-static int train_step(ofx_mlp* n, int nsamp, float lr) {
-    int Mp = (nsamp + 63) / 64 * 64;
-    OFX_TRY(forward(n, Mp, true));
-    OFX_TRY(backward(n, nsamp, Mp));
-    ++n->step;
-    const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    float c1 = 1.0f / (1.0f - std::pow(b1, (float)n->step));
-    float c2 = 1.0f / (1.0f - std::pow(b2, (float)n->step));
-    for (int l = 0; l < NLAYER; ++l) {
-        size_t nw = (size_t)n->kin[l] * n->kout[l];
-        k_adam<<<(unsigned)((nw + 255) / 256), 256, 0, n->stream>>>(n->w[l], n->gw[l], n->mw[l], n->vw[l], n->wb[l], nw,
-                                                                   lr, b1, b2, eps, c1, c2);
-        k_adam<<<(n->kout[l] + 255) / 256, 256, 0, n->stream>>>(n->b[l], n->gb[l], n->mb[l], n->vb[l], nullptr,
-                                                               (size_t)n->kout[l], lr, b1, b2, eps, c1, c2);
-    }
-    OFX_HIP(hipGetLastError());
-    return refresh_wt(n, false);
 }
 
 int ofx_mlp_train(ofx_mlp* n, const float* x, const float* t, int nsamp, int batch, int steps, float lr,
@@ -981,7 +1251,7 @@ int ofx_mlp_train(ofx_mlp* n, const float* x, const float* t, int nsamp, int bat
     }
     OFX_HIP(hipSetDevice(n->device));
     int bsz = std::min(batch, nsamp);
-    OFX_TRY(mlp_reserve(n, bsz));
+    OFX_TRY(train_reserve(n, bsz));
     // training set, epoch permutation and per-step losses live on the device
     float *dx = nullptr, *dt = nullptr, *dl = nullptr;
     int* dperm = nullptr;
@@ -1000,7 +1270,6 @@ int ofx_mlp_train(ofx_mlp* n, const float* x, const float* t, int nsamp, int bat
     for (int i = 0; i < nsamp; ++i) perm[i] = i;
     uint64_t s = seed * 2862933555777941757ull + 3037000493ull;
     int pos = nsamp;
-    int Mp = (bsz + 63) / 64 * 64;
     for (int st = 0; st < steps && !rc; ++st) {
         if (pos + bsz > nsamp) {  // new epoch: reshuffle (Fisher-Yates) and upload
             for (int i = nsamp - 1; i > 0; --i) {
@@ -1015,14 +1284,10 @@ int ofx_mlp_train(ofx_mlp* n, const float* x, const float* t, int nsamp, int bat
             }
             pos = 0;
         }
-        k_gather_batch<<<(bsz + 255) / 256, 256, 0, n->stream>>>(dx, dt, dperm + pos, bsz, n->xin, n->tgt);
-        k_pack_inputs<<<(Mp * NIN_P + 255) / 256, 256, 0, n->stream>>>(n->xin, bsz, Mp, n->h[0]);
-        if (hipGetLastError() != hipSuccess) { rc = OFX_EHIP; break; }
+        rc = grad_step(n, dx, dt, dperm + pos, bsz, true, lr, dl + st);
         pos += bsz;
-        rc = train_step(n, bsz, lr);
-        if (!rc) k_copy1<<<1, 64, 0, n->stream>>>(n->loss, dl + st);
     }
-    if (const int r2 = refresh_frag(n)) rc = rc ? rc : r2;
+    if (const int r2 = refresh_wt(n)) rc = rc ? rc : r2;
     if (!rc && hipStreamSynchronize(n->stream) != hipSuccess) rc = OFX_EHIP;
     if (!rc && loss_out && hipMemcpy(loss_out, dl, sizeof(float) * (size_t)steps, hipMemcpyDeviceToHost) != hipSuccess)
         rc = OFX_EHIP;

@@ -100,3 +100,44 @@ def test_one_kernel_forward_shapes(n):
     m.set_forward_variant(1)
     y1 = m.forward(x)
     assert np.array_equal(y0, y1, equal_nan=True)
+
+
+@pytest.mark.parametrize("n", [1, 63, 65, 1050, 2048, 4096, 4097, 131072])
+def test_gradient_shapes(n):
+    """Both workgroup shapes of the gradient kernel, one and several splits of
+    the weight products (one layer at a time from 65 splits), and a ragged last
+    64 samples, against the oracle.  Tolerance: all elements of a block one
+    bf16 step (2^-8 = 4e-3) apart."""
+    rng = np.random.default_rng(n)
+    p = random_params(rng, scale=1.0).astype(np.float32)
+    x = rng.normal(0, 1, (n, NIN)).astype(np.float32)
+    t = rng.normal(0, 1, (n, NOUT)).astype(np.float32)
+    loss, g = net(p).gradients(x, t)
+    lo, go = MlpOracle(p, bf16=True).gradients(x, t)
+    assert abs(loss - lo) <= 1e-4 * abs(lo), (loss, lo)
+    o = 0
+    for l, (i, k) in enumerate(zip(KIN, KOUT)):
+        for name, cnt in (("W", i * k), ("b", k)):
+            a, b = g[o:o + cnt], go[o:o + cnt]
+            e = float(np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-30))
+            assert e <= 5e-3, (l, name, e)
+            o += cnt
+
+
+@pytest.mark.parametrize("n,batch", [(70, 64), (5000, 4096), (9000, 8192)])
+def test_training_keeps_weight_copies(n, batch):
+    """After training, every copy of the weights (fp32, bf16, both operand
+    orders, transposed) holds the same network: the two forward forms and the
+    gradients equal those of a net given the trained parameters, bit for bit."""
+    rng = np.random.default_rng(n)
+    x = rng.normal(0, 1, (n, NIN)).astype(np.float32)
+    t = rng.normal(0, 1, (n, NOUT)).astype(np.float32)
+    m = net()
+    m.train(x, t, batch=batch, steps=3, lr=1e-3)
+    ref = net(m.params())
+    for v in (0, 1):
+        m.set_forward_variant(v)
+        ref.set_forward_variant(v)
+        assert np.array_equal(m.forward(x), ref.forward(x))
+    (l0, g0), (l1, g1) = m.gradients(x, t), ref.gradients(x, t)
+    assert l0 == l1 and np.array_equal(g0, g1)
