@@ -521,22 +521,24 @@ int step_launch(ofx_ctx* c, int iter) {
         return 0;
     }
     OFX_TRY(ns_timestep(c, iter));
-    // the first lower-sweep level is computed by the residual gathers when the
-    // schedule allows it (fusable_l0), and the sweeps start at level 1
-    const int L0 = fusable_l0(c);
-    const int ns_l0 = c->gather_variant == 1 ? L0 : 0;
-    c->fuse_l0 = ns_l0;
+    // sweeps launched level by level: the residual gathers compute the first
+    // lower-sweep level (the launches start at the second), and the sweeps raise
+    // the update's flag as increments become final
+    const bool levels = !c->sweep, ns_first = levels && c->gather_variant == 1;
+    const bool flag = levels && !(ns_first && c->sched.lone);
+    if (flag) c->par_fix ^= 1;
+    c->fuse_first = ns_first;
     int rc = ns_residual(c, true);
-    c->fuse_l0 = 0;
+    c->fuse_first = 0;
     OFX_TRY(rc);
-    OFX_TRY(ns_lusgs(c, ns_l0 > 0 ? 1 : 0));
-    OFX_TRY(ns_update_fused(c));
+    OFX_TRY(ns_lusgs(c, ns_first, flag));
+    OFX_TRY(ns_update_fused(c, flag));
     if (c->k.vismodel == 3) {
-        c->fuse_l0 = L0;
+        c->fuse_first = levels;
         rc = sa_residual(c);
-        c->fuse_l0 = 0;
+        c->fuse_first = 0;
         OFX_TRY(rc);
-        OFX_TRY(sa_lusgs(c, L0 > 0 ? 1 : 0));
+        OFX_TRY(sa_lusgs(c, levels));
         OFX_TRY(sa_update_fused(c));
     }
     return 0;

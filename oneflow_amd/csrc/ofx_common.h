@@ -144,6 +144,7 @@ struct HostSched {
     // per level: first cell when the level's cells are one ascending run of
     // consecutive cells (a colouring stored colour by colour), else -1
     std::vector<int> loBase, upBase;
+    bool lone = false;  // some cell has no interior face (it is in the first level of both sweeps)
 };
 
 struct Consts {
@@ -237,7 +238,7 @@ struct ofx_ctx {
     int normal_variant = 1;
     int gen = 0;  // bumped whenever launch parameters change (mesh, config, tiles)
     bool dist_valid = false;  // wall distance computed for the current mesh / zones
-    int fuse_l0 = 0;  // > 0 while a full step fuses the first lower-sweep level into the gathers
+    int fuse_first = 0;  // 1 while a full step computes the first lower-sweep level in the residual gathers
     // several zones: cell / boundary-face starts (nz + 1 each), host copies of
     // the per-zone constants and configurations
     std::vector<int> zc, zb;
@@ -653,8 +654,7 @@ int ns_residual_parts(ofx_ctx* c, unsigned parts, bool reuse_ext = true);
 int step_launch(ofx_ctx* c, int iter);
 int sa_residual(ofx_ctx* c);
 int sa_residual_parts(ofx_ctx* c, unsigned parts);  // bits: gradient, face terms, cell terms
-int ns_lusgs(ofx_ctx* c, int lo_first = 0);
-int fusable_l0(const ofx_ctx* c);
+int ns_lusgs(ofx_ctx* c, int lo_first = 0, bool flag = false);
 int sweep_build(ofx_ctx* c, const std::vector<int>& off, const std::vector<int>& nb, const std::vector<int>& id,
                 const std::vector<int>& lev, const std::vector<int>& levU);
 void sweep_free(ofx_ctx* c);
@@ -671,7 +671,7 @@ int aero_row(ofx_ctx* c, double* out12);
 int wall_data(ofx_ctx* c, double* host_out);
 int fill_ghost_grad(ofx_ctx* c);
 int materialize_timestep(ofx_ctx* c);
-int ns_update_fused(ofx_ctx* c);
+int ns_update_fused(ofx_ctx* c, bool flagged = false);
 int sa_update_fused(ofx_ctx* c);
 int lhs(ofx_ctx* c, int solver, double lhscoef);
 

@@ -92,13 +92,13 @@ __device__ __forceinline__ LuFace ns_lusgs_coef(const Consts& k, double xfn, dou
     return f;
 }
 
-// The face term added to rhs0: the split flux increment of the neighbour's
-// dqj and, with viscosity, its viscous radius.
+// The split flux increment dfj of the neighbour's dqj; returns the viscous radius
+// (a sweep adds the face as rhs0 -= radius * dqj, then rhs0 += dfj).
 template <int VM>
-__device__ __forceinline__ void ns_lusgs_face(const Consts& k, double xfn, double yfn, double zfn, double vfn,
-                                              double farea, double rl, double ul, double vl, double wl, double pl,
-                                              const double* pj, const double* dqj, double visl, double vist,
-                                              double volr, double dist, double* rhs0) {
+__device__ __forceinline__ double ns_lusgs_term(const Consts& k, double xfn, double yfn, double zfn, double vfn,
+                                                double farea, double rl, double ul, double vl, double wl, double pl,
+                                                const double* pj, const double* dqj, double visl, double vist,
+                                                double volr, double dist, double* dfj) {
     const LuFace f = ns_lusgs_coef<VM>(k, xfn, yfn, zfn, vfn, farea, rl, ul, vl, wl, pl, pj, visl, vist, volr, dist);
     double dc = f.vn * dqj[0] - xfn * dqj[1] - yfn * dqj[2] - zfn * dqj[3];
     double c2dc = f.c2 * dc;
@@ -107,16 +107,62 @@ __device__ __forceinline__ void ns_lusgs_face(const Consts& k, double xfn, doubl
     dh += f.af * dqj[0];
     double term1 = dh * f.x1 + dc * f.x2;
     double term2 = c2dc * f.x1 + dh * f.x2;
-    double dfj[5];
     dfj[0] = f.lmd1 * dqj[0] - term1;
     dfj[1] = f.lmd1 * dqj[1] - pj[1] * term1 + xfn * term2;
     dfj[2] = f.lmd1 * dqj[2] - pj[2] * term1 + yfn * term2;
     dfj[3] = f.lmd1 * dqj[3] - pj[3] * term1 + zfn * term2;
     dfj[4] = f.lmd1 * dqj[4] - f.hm * term1 + f.vn * term2;
     for (int e = 0; e < 5; ++e) dfj[e] *= farea;
+    return f.visrad;
+}
+
+// The face term added to rhs0.
+template <int VM>
+__device__ __forceinline__ void ns_lusgs_face(const Consts& k, double xfn, double yfn, double zfn, double vfn,
+                                              double farea, double rl, double ul, double vl, double wl, double pl,
+                                              const double* pj, const double* dqj, double visl, double vist,
+                                              double volr, double dist, double* rhs0) {
+    double dfj[5];
+    const double visrad = ns_lusgs_term<VM>(k, xfn, yfn, zfn, vfn, farea, rl, ul, vl, wl, pl, pj, dqj, visl, vist,
+                                            volr, dist, dfj);
     if (VM != 0)
-        for (int e = 0; e < 5; ++e) rhs0[e] -= f.visrad * dqj[e];
+        for (int e = 0; e < 5; ++e) rhs0[e] -= visrad * dqj[e];
     for (int e = 0; e < 5; ++e) rhs0[e] += dfj[e];
+}
+
+// UNsUpdate::UpdateFlowField + NsUpdate::CalcFlowField / WeekSolutionFix
+// (codes/uns/src/UNsUpdate.cpp:46-146, codes/ns/src/NsUpdate.cpp:40-67,192-217):
+// the new primitive state of a cell; false when it needs SolutionFix.
+__device__ __forceinline__ bool ns_update_state(const Consts& k, const double* prim0, const double* dq, double* prim) {
+    double q0[5], q[5];
+    double gama = k.gama;
+    prim_to_q(prim0, gama, q0);
+    for (int e = 0; e < 5; ++e) q[e] = q0[e] + dq[e];
+    double density = dabs(q[0]);
+    double rd = 1.0 / density;
+    double um = q[1] * rd, vm = q[2] * rd, wm = q[3] * rd, rem = q[4];
+    double v2 = sqr3(um, vm, wm);
+    double reint = rem - 0.5 * density * v2;
+    prim[0] = density; prim[1] = um; prim[2] = vm; prim[3] = wm; prim[4] = (gama - 1.0) * reint;
+    if (prim[0] <= 0.0 || prim[4] <= 0.0) {
+        const double coefs[3] = {0.5, 0.1, 0.01};
+        for (int kk = 0; kk < 3; ++kk) {
+            for (int e = 0; e < 5; ++e) prim[e] += coefs[kk] * dq[e];
+            if (!(prim[0] < 0.0 || prim[4] < 0.0)) return true;
+        }
+        return false;
+    }
+    return true;
+}
+
+// A cell whose increment dq is final needs SolutionFix or not: if so, it raises the
+// grid's flag (RQ_FIX) of parity `par`.  The update clears the other parity's.
+__device__ __forceinline__ void ns_update_flag(const DevMesh& m, const DevFields& d, const Consts& k,
+                                               const double* prim0, const double* dq, int par) {
+    double prim[5];
+    if (!ns_update_state(k, prim0, dq, prim))
+        atomicMax(&d.slots[((size_t)par * m.nz * RQ_N + RQ_FIX) * NSLOT + blockIdx.x % NSLOT],
+                  (unsigned long long)__double_as_longlong(1.0));
 }
 
 }  // namespace ofx

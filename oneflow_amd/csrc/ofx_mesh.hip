@@ -643,6 +643,8 @@ int mesh_build(ofx_ctx* c, const double* x, const double* y, const double* z, co
     runs(loOrd, c->sched.loOff, c->sched.loBase);
     runs(upOrd, c->sched.upOff, c->sched.upBase);
     m.nLevLo = nlo; m.nLevUp = nup;
+    c->sched.lone = false;
+    for (int i = 0; i < C; ++i) c->sched.lone = c->sched.lone || (lev[i] == 0 && levU[i] == 0);
     // Segments for XCD placement: cells stored sorted by lower-sweep level with
     // at most 8 levels are a colouring stored colour by colour; each colour is
     // one segment, and the interior faces (sorted by left cell) split at the

@@ -517,13 +517,12 @@ __global__ void __launch_bounds__(TB) k_ns_grad(DevMesh m, DevFields d, Consts k
 
 // The residual gather with one thread per cell (face loads of the cell all
 // issued first, then the ordered sums: inviscid chain, then viscous).
-// L0 (> 0 inside a full pseudo-time step): cells [0, L0) are the first level
-// of the lower LU-SGS sweep (no lower-numbered neighbour), whose increment is
+// FUSE (inside a full pseudo-time step): a cell without a lower-numbered
+// neighbour is in the first level of the lower LU-SGS sweep, whose increment is
 // dq = (res - 0) / D; the gather writes it with the residual and the sweep
 // starts at its second level.
 template <int MAXF, bool VISC, bool F32, bool FUSE>
-__device__ __forceinline__ void ns_gather_cell(const DevMesh& m, const DevFields& d, const Consts& k0, int par,
-                                               int L0) {
+__device__ __forceinline__ void ns_gather_cell(const DevMesh& m, const DevFields& d, const Consts& k0, int par) {
     const int T = m.T, F = m.F;
     // Every lane stays active to the end (the fused path reduces the time-step
     // slots per wave): lanes past the last cell evaluate it and store nothing.
@@ -533,7 +532,8 @@ __device__ __forceinline__ void ns_gather_cell(const DevMesh& m, const DevFields
     double mindt1 = 0.0;
     if (FUSE) wave_slot_result<1, false>(d.slots, par, m.nz * RQ_N, RQ_DTMIN, &mindt1);
     double rad = 1.0;
-    if (FUSE && i < L0) {
+    const bool first = FUSE && m.lomask[i] == 0;
+    if (first) {
         const Consts k = zoned(k0, m, cell_zone(m, i));
         rad = ns_impsr(m, d, k, i, zone_mindt(m, d, i, mindt1));
     }
@@ -574,18 +574,18 @@ __device__ __forceinline__ void ns_gather_cell(const DevMesh& m, const DevFields
                 sum = sum + live_or_nz(j < n, fv[s][j]);
         }
         if (live) d.res[s * T + i] = sum;
-        if (FUSE && live && i < L0) { double t = sum - 0.0; t /= rad; d.dq[s * T + i] = t; }
+        if (first && live) { double t = sum - 0.0; t /= rad; d.dq[s * T + i] = t; }
     }
 }
 
 template <int MAXF, bool VISC, bool F32>
 __global__ void __launch_bounds__(TB) k_ns_gather_c(DevMesh m, DevFields d) {
-    ns_gather_cell<MAXF, VISC, F32, false>(m, d, Consts{}, 0, 0);
+    ns_gather_cell<MAXF, VISC, F32, false>(m, d, Consts{}, 0);
 }
 
 template <int MAXF, bool VISC, bool F32>
-__global__ void __launch_bounds__(TB) k_ns_gather_cf(DevMesh m, DevFields d, Consts k0, int par, int L0) {
-    ns_gather_cell<MAXF, VISC, F32, true>(m, d, k0, par, L0);
+__global__ void __launch_bounds__(TB) k_ns_gather_cf(DevMesh m, DevFields d, Consts k0, int par) {
+    ns_gather_cell<MAXF, VISC, F32, true>(m, d, k0, par);
 }
 
 // Viscous face flux (UNsVisFlux::CalcFlux, codes/uns/src/UNsVisFlux.cpp:127-440)
@@ -857,14 +857,13 @@ static void launch_cells(ofx_ctx* c, unsigned parts, bool reuse_ext) {
     }
     if (parts & 4u) launch_face_dim<DIM>(c, visc);
     if ((parts & 8u) && c->gather_variant == 1) {
-        const int L0 = c->fuse_l0;
-        if (L0 > 0) {
+        if (c->fuse_first) {
             if (k.flux_fp32) {
-                if (visc) k_ns_gather_cf<MAXF, true, true><<<nblk(C1), TB, 0, c->stream>>>(c->m, c->d, k, c->par_dt, L0);
-                else k_ns_gather_cf<MAXF, false, true><<<nblk(C1), TB, 0, c->stream>>>(c->m, c->d, k, c->par_dt, L0);
+                if (visc) k_ns_gather_cf<MAXF, true, true><<<nblk(C1), TB, 0, c->stream>>>(c->m, c->d, k, c->par_dt);
+                else k_ns_gather_cf<MAXF, false, true><<<nblk(C1), TB, 0, c->stream>>>(c->m, c->d, k, c->par_dt);
             } else {
-                if (visc) k_ns_gather_cf<MAXF, true, false><<<nblk(C1), TB, 0, c->stream>>>(c->m, c->d, k, c->par_dt, L0);
-                else k_ns_gather_cf<MAXF, false, false><<<nblk(C1), TB, 0, c->stream>>>(c->m, c->d, k, c->par_dt, L0);
+                if (visc) k_ns_gather_cf<MAXF, true, false><<<nblk(C1), TB, 0, c->stream>>>(c->m, c->d, k, c->par_dt);
+                else k_ns_gather_cf<MAXF, false, false><<<nblk(C1), TB, 0, c->stream>>>(c->m, c->d, k, c->par_dt);
             }
         } else if (k.flux_fp32) {
             if (visc) k_ns_gather_c<MAXF, true, true><<<nblk(C1), TB, 0, c->stream>>>(c->m, c->d);
@@ -931,7 +930,7 @@ int fill_ghost_grad(ofx_ctx* c) {
 // areas come from the per-entry copies (DevMesh::ellg plane 2).
 template <bool UPPER, int MAXF, int VM, bool EN>
 __device__ __forceinline__ void ns_lusgs_cell(const DevMesh& m, const DevFields& d, const Consts& k0, int i, double mindt1,
-                                              bool store = true) {
+                                              int par_fix, bool store = true) {
     const int T = m.T;
     const Consts k = zoned(k0, m, cell_zone(m, i));
     const double mindt = zone_mindt(m, d, i, mindt1);
@@ -940,12 +939,13 @@ __device__ __forceinline__ void ns_lusgs_cell(const DevMesh& m, const DevFields&
     int ent[MAXF], nb[MAXF];
     cell_faces<MAXF>(m, i, ent, nb);
     const int lomask = m.lomask[i];
-    bool act[MAXF];
+    bool act[MAXF], last = true;  // last: no higher neighbour, so the lower sweep's increment is final
 #pragma unroll
     for (int j = 0; j < MAXF; ++j) {
         int f = ent[j] >= 0 ? ent[j] : ~ent[j];
         const bool lower = (lomask >> j) & 1;  // neighbour's id below the cell's
         act[j] = j < n && f >= m.B && (UPPER ? !lower : lower);
+        last = last && (lower || j >= n || f < m.B);
     }
     double rl = d.q[i], ul = d.q[T + i], vl = d.q[2 * T + i], wl = d.q[3 * T + i], pl = d.q[4 * T + i];
     double xi = 0.0, yi = 0.0, zi = 0.0;
@@ -993,32 +993,137 @@ __device__ __forceinline__ void ns_lusgs_cell(const DevMesh& m, const DevFields&
     }
     double rad = ns_impsr(m, d, k, i, mindt);
     if (!store) return;
+    double dqi[5];
     if (!UPPER) {
-        for (int e = 0; e < 5; ++e) { double t = d.res[e * T + i] - rhs0[e]; t /= rad; d.dq[e * T + i] = t; }
+        for (int e = 0; e < 5; ++e) { double t = d.res[e * T + i] - rhs0[e]; t /= rad; dqi[e] = t; }
     } else {
-        for (int e = 0; e < 5; ++e) { double t = -rhs0[e]; t /= rad; d.dq[e * T + i] += t; }
+        for (int e = 0; e < 5; ++e) { double t = -rhs0[e]; t /= rad; dqi[e] = d.dq[e * T + i] + t; }
+    }
+    for (int e = 0; e < 5; ++e) d.dq[e * T + i] = dqi[e];
+    if (par_fix >= 0 && (UPPER || last)) {
+        const double prim0[5] = {rl, ul, vl, wl, pl};
+        ns_update_flag(m, d, k0, prim0, dqi, par_fix);
     }
 }
 
 // One level per launch (wide levels on large meshes).
 // base >= 0: the level's cells are base, base + 1, ... (no order lookup).
+// par_fix >= 0: cells whose increment is final raise the update's flag.
 template <bool UPPER, int MAXF, int VM, bool EN>
 __global__ void __launch_bounds__(TB) k_ns_sweep_level(DevMesh m, DevFields d, Consts k, int b, int e, int base,
-                                                       int par) {
+                                                       int par, int par_fix) {
     // Every lane stays active (the minimum time step is reduced per wave, its
     // slot loads overlapping the cell's own): lanes past the level's end
     // evaluate its last cell and store nothing.
-    const int idx0 = b + blockIdx.x * TB + threadIdx.x;
+    const int idx0 = b + xcd_block((int)gridDim.x) * TB + (int)threadIdx.x;
     const bool live = idx0 < e;
     const int idx = live ? idx0 : e - 1;
     double mindt;
     wave_slot_result<1, false>(d.slots, par, m.nz * RQ_N, RQ_DTMIN, &mindt);
     int i = base >= 0 ? base + (idx - b) : (UPPER ? m.upOrder : m.loOrder)[idx];
-    ns_lusgs_cell<UPPER, MAXF, VM, EN>(m, d, k, i, mindt, live);
+    ns_lusgs_cell<UPPER, MAXF, VM, EN>(m, d, k, i, mindt, par_fix, live);
 }
 
+// A level of few cells, 64 of them per block: wave j evaluates entry j of their
+// face lists, a last wave their diagonals, then wave e adds up equation e in
+// face order from LDS and divides.  A level of a 2-D grid of ordinary size is about
+// one wave per SIMD, so the kernel above takes as long as one thread does
+// for all of a cell's faces.  (Four adjacent lanes per cell instead took 23.4 us on
+// 60,160 cells, this form 9.9: its loads touch four planes per instruction and
+// every lane repeats the sums.)
+template <bool UPPER, int MAXF, int VM>
+__global__ void __launch_bounds__(64 * (MAXF + 1)) k_ns_sweep_split(DevMesh m, DevFields d, Consts k0, int b, int e,
+                                                                    int base, int par, int par_fix) {
+    static_assert(MAXF >= 4, "a wave per equation");
+    __shared__ double term[2][5][MAXF][64];  // viscous radius x dq, flux increment
+    __shared__ double diag[64], inc[5][64];
+    __shared__ unsigned long long acts[MAXF], high[MAXF];
+    const int w = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
+    const int idx0 = b + xcd_block((int)gridDim.x) * 64 + lane;
+    const bool live = idx0 < e;
+    const int idx = live ? idx0 : e - 1;  // lanes past the level's end evaluate its last cell and store nothing
+    const int T = m.T;
+    double prim0[5], old = 0.0;
+    const double* from = UPPER ? d.dq : d.res;
+    int i;
+    if (w < MAXF) {
+        i = base >= 0 ? base + (idx - b) : (UPPER ? m.upOrder : m.loOrder)[idx];
+        const size_t o = (size_t)w * m.C + i;
+        const bool in = w < m.ellw;
+        const int ent = in ? m.ellf[o] : 0, nb = in ? m.elln[o] : i;
+        const int n = m.c2fOff[i + 1] - m.c2fOff[i], lomask = m.lomask[i];
+        dvec4 r4 = {};
+        double rx = 0.0;  // SR model 1: the neighbour's volume, otherwise the distance along the normal
+        if (in) {
+            r4 = m.ellg[(size_t)2 * m.ellw * m.C + o];
+            if (VM != 0) rx = m.elldv[(VM == 1 ? (size_t)m.ellw * m.C : 0) + o];
+        }
+        for (int q = 0; q < 5; ++q) prim0[q] = d.q[q * T + i];
+        if (w < 5) old = from[w * T + i];
+        const Consts k = zoned(k0, m, cell_zone(m, i));
+        const int f = ent >= 0 ? ent : ~ent;
+        const bool lower = (lomask >> w) & 1, inner = w < n && f >= m.B;
+        const bool act = inner && (UPPER ? !lower : lower);
+        const unsigned long long ma = __ballot(act), mh = __ballot(inner && !lower);
+        if (lane == 0) { acts[w] = ma; high[w] = mh; }
+        if (act) {
+            double pj[5], dqj[5], df[5], vl = 0.0, vt = 0.0;
+            for (int q = 0; q < 5; ++q) { pj[q] = d.q[q * T + nb]; dqj[q] = d.dq[q * T + nb]; }
+            if (VM != 0) { vl = d.visl[nb]; vt = d.vist[nb]; }
+            const bool own = ent >= 0;  // GCom::SetGeometry: the normal points out of i
+            const double xfn = own ? r4.x : -r4.x, yfn = own ? r4.y : -r4.y, zfn = own ? r4.z : -r4.z;
+            const double visrad = ns_lusgs_term<VM>(k, xfn, yfn, zfn, own ? 0.0 : -0.0, r4.w, prim0[0], prim0[1],
+                                                    prim0[2], prim0[3], prim0[4], pj, dqj, vl, vt, rx, rx, df);
+            for (int q = 0; q < 5; ++q) {
+                if (VM != 0) term[0][q][w][lane] = visrad * dqj[q];
+                term[1][q][w][lane] = df[q];
+            }
+        }
+    } else {
+        double mindt;
+        wave_slot_result<1, false>(d.slots, par, m.nz * RQ_N, RQ_DTMIN, &mindt);
+        i = base >= 0 ? base + (idx - b) : (UPPER ? m.upOrder : m.loOrder)[idx];
+        if (w < 5) old = from[w * T + i];
+        for (int q = 0; q < 5; ++q) prim0[q] = d.q[q * T + i];
+        const Consts k = zoned(k0, m, cell_zone(m, i));
+        diag[lane] = ns_impsr(m, d, k, i, zone_mindt(m, d, i, mindt));
+    }
+    __syncthreads();
+    if (w < 5) {
+        double rhs = 0.0;
+#pragma unroll
+        for (int j = 0; j < MAXF; ++j) {
+            double t = VM != 0 ? rhs - term[0][w][j][lane] : rhs;
+            t += term[1][w][j][lane];
+            rhs = (acts[j] >> lane) & 1 ? t : rhs;
+        }
+        double t = UPPER ? -rhs : old - rhs;
+        t /= diag[lane];
+        if (UPPER) t = old + t;
+        if (live) d.dq[w * T + i] = t;
+        inc[w][lane] = t;
+    }
+    if (par_fix < 0) return;
+    __syncthreads();
+    if (w != MAXF || !live) return;
+    bool last = true;  // no higher neighbour: the lower sweep's increment is final
+    if (!UPPER)
+        for (int j = 0; j < MAXF; ++j) last = last && !((high[j] >> lane) & 1);
+    if (!last) return;
+    const double dqi[5] = {inc[0][lane], inc[1][lane], inc[2][lane], inc[3][lane], inc[4][lane]};
+    ns_update_flag(m, d, k0, prim0, dqi, par_fix);
+}
+
+// Whether a level of nc cells goes to k_ns_sweep_split.  us by one thread per cell /
+// split: quads and triangles (at most four faces) 256 cells 8.9 / 4.4, 23,040
+// 10.5 / 6.0, 60,160 12.5 / 9.9, 377,600 44 / 51 (there the memory system is
+// busy either way and the exchange through LDS costs); 3-D cells 1,024 10.4 / 5.7,
+// 53,504 12.4 / 9.1, 321,280 58.5 / 56.4, 910,336 155 / 151, so always.
+template <int MAXF>
+static bool split_level(int nc) { return MAXF == 6 || nc <= 131072; }
+
 template <int MAXF, int VM, bool EN>
-static void launch_lusgs(ofx_ctx* c, int lo_first) {
+static void launch_lusgs(ofx_ctx* c, int lo_first, int pf) {
     const DevMesh& m = c->m;
     for (int pass = 0; pass < 2; ++pass) {
         bool up = pass == 1;
@@ -1029,44 +1134,44 @@ static void launch_lusgs(ofx_ctx* c, int lo_first) {
         for (size_t L = up ? 1 : (size_t)lo_first; L + 1 < off.size(); ++L) {
             int b = off[L], e = off[L + 1];
             if (e <= b) continue;
-            if (up)
-                k_ns_sweep_level<true, MAXF, VM, EN><<<nblk(e - b), TB, 0, c->stream>>>(m, c->d, c->k, b, e, base[L],
-                                                                                   c->par_dt);
-            else
-                k_ns_sweep_level<false, MAXF, VM, EN><<<nblk(e - b), TB, 0, c->stream>>>(m, c->d, c->k, b, e, base[L],
-                                                                                    c->par_dt);
+            const int nc = e - b, bs = base[L], pd = c->par_dt;
+            if constexpr (EN && MAXF <= 6) {
+                if (split_level<MAXF>(nc)) {
+                    const int nbk = (nc + 63) / 64, nt = 64 * (MAXF + 1);
+                    if (up) k_ns_sweep_split<true, MAXF, VM><<<nbk, nt, 0, c->stream>>>(m, c->d, c->k, b, e, bs, pd, pf);
+                    else k_ns_sweep_split<false, MAXF, VM><<<nbk, nt, 0, c->stream>>>(m, c->d, c->k, b, e, bs, pd, pf);
+                    continue;
+                }
+            }
+            if constexpr (!(EN && MAXF == 6)) {
+                if (up) k_ns_sweep_level<true, MAXF, VM, EN><<<nblk(nc), TB, 0, c->stream>>>(m, c->d, c->k, b, e, bs, pd, pf);
+                else k_ns_sweep_level<false, MAXF, VM, EN><<<nblk(nc), TB, 0, c->stream>>>(m, c->d, c->k, b, e, bs, pd, pf);
+            }
         }
     }
 }
 
 template <int MAXF, bool EN>
-static void launch_lusgs_vm(ofx_ctx* c, int lo_first) {
-    if (c->k.vismodel == 0) launch_lusgs<MAXF, 0, EN>(c, lo_first);
-    else if (c->k.visSRModel == 1) launch_lusgs<MAXF, 1, EN>(c, lo_first);
-    else launch_lusgs<MAXF, 2, EN>(c, lo_first);
+static void launch_lusgs_vm(ofx_ctx* c, int lo_first, int pf) {
+    if (c->k.vismodel == 0) launch_lusgs<MAXF, 0, EN>(c, lo_first, pf);
+    else if (c->k.visSRModel == 1) launch_lusgs<MAXF, 1, EN>(c, lo_first, pf);
+    else launch_lusgs<MAXF, 2, EN>(c, lo_first, pf);
 }
 template <int MAXF>
-static void launch_lusgs_vm(ofx_ctx* c, int lo_first) {
-    if (c->normal_variant == 1) launch_lusgs_vm<MAXF, true>(c, lo_first);
-    else launch_lusgs_vm<MAXF, false>(c, lo_first);
+static void launch_lusgs_vm(ofx_ctx* c, int lo_first, int pf) {
+    if (c->normal_variant == 1) launch_lusgs_vm<MAXF, true>(c, lo_first, pf);
+    else launch_lusgs_vm<MAXF, false>(c, lo_first, pf);
 }
 
-// The first level of the lower sweep that may be fused into the residual
-// gathers: its cells must be the run 0..loOff[1]-1 and the sweeps launched
-// per level.  Returns loOff[1], or 0.
-int fusable_l0(const ofx_ctx* c) {
-    const HostSched& h = c->sched;
-    if (c->sweep || h.loBase.empty() || h.loBase[0] != 0) return 0;
-    return h.loOff[1];
-}
-
-int ns_lusgs(ofx_ctx* c, int lo_first) {
+// lo_first: the first level of the lower sweep to launch.  flag: raise the
+// update's flag (ns_update_flag, parity c->par_fix) as increments become final.
+int ns_lusgs(ofx_ctx* c, int lo_first, bool flag) {
     if (c->sweep) return pipelined_lusgs_ns(c);
-    int mf = c->m.maxFacesPerCell;
-    if (mf <= 4) launch_lusgs_vm<4>(c, lo_first);
-    else if (mf <= 6) launch_lusgs_vm<6>(c, lo_first);
-    else if (mf <= 8) launch_lusgs_vm<8>(c, lo_first);
-    else if (mf <= 16) launch_lusgs_vm<16>(c, lo_first);
+    const int mf = c->m.maxFacesPerCell, pf = flag ? c->par_fix : -1;
+    if (mf <= 4) launch_lusgs_vm<4>(c, lo_first, pf);
+    else if (mf <= 6) launch_lusgs_vm<6>(c, lo_first, pf);
+    else if (mf <= 8) launch_lusgs_vm<8>(c, lo_first, pf);
+    else if (mf <= 16) launch_lusgs_vm<16>(c, lo_first, pf);
     else { set_error("cells with more than 16 faces are not supported"); return OFX_EINVAL; }
     OFX_HIP(hipGetLastError());
     return 0;
@@ -1074,42 +1179,25 @@ int ns_lusgs(ofx_ctx* c, int lo_first) {
 
 // ============================================================ update
 
-// UNsUpdate::UpdateFlowField + NsUpdate::CalcFlowField / WeekSolutionFix /
-// SolutionFix (codes/uns/src/UNsUpdate.cpp:46-146, codes/ns/src/NsUpdate.cpp:40-67,192-217).
+// The update of cell i (ns_update_state); false when it needs SolutionFix
+// (codes/ns/src/NsUpdate.cpp:192-217).
 __device__ __forceinline__ bool ns_update_cell(const DevFields& d, const Consts& k, int T, int i, double* prim) {
-    double prim0[5], q0[5], q[5], dq[5];
+    double prim0[5], dq[5];
     for (int e = 0; e < 5; ++e) { prim0[e] = d.q[e * T + i]; dq[e] = d.dq[e * T + i]; }
-    double gama = k.gama;
-    prim_to_q(prim0, gama, q0);
-    for (int e = 0; e < 5; ++e) q[e] = q0[e] + dq[e];
-    double density = dabs(q[0]);
-    double rd = 1.0 / density;
-    double um = q[1] * rd, vm = q[2] * rd, wm = q[3] * rd, rem = q[4];
-    double v2 = sqr3(um, vm, wm);
-    double reint = rem - 0.5 * density * v2;
-    prim[0] = density; prim[1] = um; prim[2] = vm; prim[3] = wm; prim[4] = (gama - 1.0) * reint;
-    if (prim[0] <= 0.0 || prim[4] <= 0.0) {
-        const double coefs[3] = {0.5, 0.1, 0.01};
-        for (int kk = 0; kk < 3; ++kk) {
-            for (int e = 0; e < 5; ++e) prim[e] += coefs[kk] * dq[e];
-            if (!(prim[0] < 0.0 || prim[4] < 0.0)) return true;
-        }
-        return false;  // needs SolutionFix
-    }
-    return true;
+    return ns_update_state(k, prim0, dq, prim);
 }
 
 // Pass 1: does any cell need SolutionFix?  (The neighbour average of
 // SolutionFix reads neighbours in the serial loop's half-updated state, so
-// such an update runs serially in cell order.)
+// such an update runs serially in cell order.)  A full step's level sweeps raise
+// the flag themselves; this pass is for an update on its own and after the
+// pipelined sweeps.
 __global__ void __launch_bounds__(TB) k_ns_update_check(DevMesh m, DevFields d, Consts k, int par) {
     int i = xcd_block(gridDim.x) * blockDim.x + threadIdx.x;
-    double flag = 0.0;
-    if (i < m.C) {
-        double prim[5];
-        if (!ns_update_cell(d, k, m.T, i, prim)) flag = 1.0;
-    }
-    slot_reduce<1, true>(&flag, d.slots, par, m.nz * RQ_N, RQ_FIX);
+    if (i >= m.C) return;
+    double prim0[5], dq[5];
+    for (int e = 0; e < 5; ++e) { prim0[e] = d.q[e * m.T + i]; dq[e] = d.dq[e * m.T + i]; }
+    ns_update_flag(m, d, k, prim0, dq, par);
 }
 
 __device__ void ns_solution_fix(const DevMesh& m, const DevFields& d, int i, double* prim) {
@@ -1161,6 +1249,8 @@ template <bool BC>
 __global__ void __launch_bounds__(TB) k_ns_update_apply(DevMesh m, DevFields d, Consts k, int par) {
     const int T = m.T;
     double anyfix = slot_result<true>(d.slots, par, m.nz * RQ_N, RQ_FIX);
+    if (blockIdx.x == 0 && threadIdx.x < NSLOT)  // the next update's flag
+        d.slots[((size_t)(1 - par) * m.nz * RQ_N + RQ_FIX) * NSLOT + threadIdx.x] = 0;
     if (anyfix == 0.0) {
         int i = xcd_block(gridDim.x) * blockDim.x + threadIdx.x;
         if (i >= m.C) return;
@@ -1199,11 +1289,14 @@ int ns_update(ofx_ctx* c) {
     return 0;
 }
 
-int ns_update_fused(ofx_ctx* c) {
+// flagged: the sweeps have raised the flag of parity c->par_fix.
+int ns_update_fused(ofx_ctx* c, bool flagged) {
     const DevFields d = update_fields(c);
     ++c->qgen;
-    c->par_fix ^= 1;
-    k_ns_update_check<<<nblk(c->m.C), TB, 0, c->stream>>>(c->m, d, c->k, c->par_fix);
+    if (!flagged) {
+        c->par_fix ^= 1;
+        k_ns_update_check<<<nblk(c->m.C), TB, 0, c->stream>>>(c->m, d, c->k, c->par_fix);
+    }
     k_ns_update_apply<true><<<nblk(c->m.C), TB, 0, c->stream>>>(c->m, d, c->k, c->par_fix);
     OFX_HIP(hipGetLastError());
     return 0;

@@ -346,7 +346,7 @@ __device__ __forceinline__ void sa_source(const DevMesh& m, const DevFields& d, 
 // gathered in ascending face order) -- TurbCalcRHS order
 // (codes/turb/src/TurbRhs.cpp:57-71).
 template <int MAXF>
-__global__ void __launch_bounds__(TBS) k_sa_cell(DevMesh m, DevFields d, Consts k0, int par, int L0) {
+__global__ void __launch_bounds__(TBS) k_sa_cell(DevMesh m, DevFields d, Consts k0, int par, int first) {
     // Every lane stays active to the end (the time-step slots are reduced per
     // wave): lanes past the last cell evaluate the last cell and store nothing.
     const int i0 = cell_block(m, TBS) * TBS + threadIdx.x;
@@ -399,8 +399,8 @@ __global__ void __launch_bounds__(TBS) k_sa_cell(DevMesh m, DevFields d, Consts 
     if (!live) return;
     d.turbimpsr[i] = imp;
     d.turbres[i] = res;
-    // cells [0, L0): the first level of the lower sweep, turbdq = (res - 0) / D
-    if (i < L0) { double t = res - 0.0; t /= imp; d.turbdq[i] = t; }
+    // the first level of the lower sweep (no lower neighbour): turbdq = (res - 0) / D
+    if (first && m.lomask[i] == 0) { double t = res - 0.0; t /= imp; d.turbdq[i] = t; }
 }
 
 // parts: bit 0 gradient (+ ghosts), bit 1 face terms, bit 2 cell terms.
@@ -418,7 +418,7 @@ static void launch_sa(ofx_ctx* c, unsigned parts) {
         else
             k_sa_face<DIM, 0><<<nb, tb, 0, c->stream>>>(m, c->d, c->k, tb);
     }
-    if (parts & 4u) k_sa_cell<MAXF><<<nblks(m.C), TBS, 0, c->stream>>>(m, c->d, c->k, c->par_dt, c->fuse_l0);
+    if (parts & 4u) k_sa_cell<MAXF><<<nblks(m.C), TBS, 0, c->stream>>>(m, c->d, c->k, c->par_dt, c->fuse_first);
 }
 
 int sa_residual_parts(ofx_ctx* c, unsigned parts) {
