@@ -532,11 +532,13 @@ int step_launch(ofx_ctx* c, int iter) {
     c->fuse_first = 0;
     OFX_TRY(rc);
     OFX_TRY(ns_lusgs(c, ns_first, flag));
-    OFX_TRY(ns_update_fused(c, flag));
-    if (c->k.vismodel == 3) {
+    const bool sa = c->k.vismodel == 3;
+    OFX_TRY(ns_update_fused(c, flag, !sa));
+    if (sa) {
         c->fuse_first = levels;
+        c->sa_ghosts = 1;
         rc = sa_residual(c);
-        c->fuse_first = 0;
+        c->fuse_first = c->sa_ghosts = 0;
         OFX_TRY(rc);
         OFX_TRY(sa_lusgs(c, levels));
         OFX_TRY(sa_update_fused(c));

@@ -238,6 +238,7 @@ struct ofx_ctx {
     int normal_variant = 1;
     int gen = 0;  // bumped whenever launch parameters change (mesh, config, tiles)
     bool dist_valid = false;  // wall distance computed for the current mesh / zones
+    int sa_ghosts = 0;   // 1 while a full step leaves the NS ghosts of its update to the SA gradient
     int fuse_first = 0;  // 1 while a full step computes the first lower-sweep level in the residual gathers
     // several zones: cell / boundary-face starts (nz + 1 each), host copies of
     // the per-zone constants and configurations
@@ -354,9 +355,10 @@ __device__ __forceinline__ bool has_bface(const DevMesh& m, int i) {
     return e >= 0 && e < m.B;
 }
 
-// Logical block of a launch over the cells (faces), `per` items per block.
-__device__ __forceinline__ int cell_block(const DevMesh& m, int per) {
-    return xcd_remap_seg((int)blockIdx.x, (int)gridDim.x, per, m.segc, m.nsegc);
+// Logical block of a launch over the cells (faces), `per` items per block; the
+// first `skip` blocks of the launch (a multiple of 8) do something else.
+__device__ __forceinline__ int cell_block(const DevMesh& m, int per, int skip = 0) {
+    return xcd_remap_seg((int)blockIdx.x - skip, (int)gridDim.x - skip, per, m.segc, m.nsegc);
 }
 // per: a power of two (the face tiles are 64 .. 512)
 __device__ __forceinline__ int face_block(const DevMesh& m, int per) {
@@ -671,7 +673,7 @@ int aero_row(ofx_ctx* c, double* out12);
 int wall_data(ofx_ctx* c, double* host_out);
 int fill_ghost_grad(ofx_ctx* c);
 int materialize_timestep(ofx_ctx* c);
-int ns_update_fused(ofx_ctx* c, bool flagged = false);
+int ns_update_fused(ofx_ctx* c, bool flagged = false, bool ghosts = true);
 int sa_update_fused(ofx_ctx* c);
 int lhs(ofx_ctx* c, int solver, double lhscoef);
 

@@ -29,88 +29,9 @@ __global__ void __launch_bounds__(TB) k_ns_cellstate(DevMesh m, DevFields d, Con
     d.visl[i] = sutherland(t, k.ts_suth);
 }
 
-// UNsBcSolver::CalcBc + NsBcSolver for one boundary face given the owner's
-// primitive state s and temperature towner (codes/uns/src/UNsBcSolver.cpp:55-168,
-// codes/ns/src/NsBcSolver.cpp:51-410); writes the ghost state, then the ghost
-// gamma/T/viscosity (NsCalcGamaT / CalcLaminarViscosity on F_GHOST).
-__device__ __forceinline__ void ns_bc_face(const DevMesh& m, const DevFields& d, const Consts& k, int f,
-                                           const double* s, double towner) {
-    const int T = m.T;
-    int bt = m.bct[f];
-    int r = m.C + f;
-    double xfn = m.xfn[f], yfn = m.yfn[f], zfn = m.zfn[f];
-    const double vfn = 0.0;
-    double t[5];
-    double gama = 0.5 * (k.gama + k.gama);
-    if (bt == BC_EXTRAPOLATION || bt == BC_OUTFLOW) {
-        for (int e = 0; e < 5; ++e) t[e] = s[e];
-    } else if (bt == BC_INFLOW) {
-        for (int e = 0; e < 5; ++e) t[e] = k.inflow[e];
-    } else if (bt == BC_SOLID_SURFACE && k.vismodel != 0) {
-        for (int e = 0; e < 5; ++e) t[e] = s[e];
-        t[1] = -t[1] + 2.0 * 0.0; t[2] = -t[2] + 2.0 * 0.0; t[3] = -t[3] + 2.0 * 0.0;
-        if (k.isowallbc != 0) {
-            // IsothermalVisWallBc (codes/ns/src/NsBcSolver.cpp:271-324)
-            double tlim = 0.1 * k.twall;
-            double rm = s[0], pm = s[4];
-            double pg1 = pm;
-            double tg1 = 2.0 * k.twall - towner;
-            if (tg1 < tlim) tg1 = tlim;
-            double rw = pg1 / (k.statecoef * k.twall * 1.0);
-            double rg1 = 2.0 * rw - rm;
-            rg1 = dmax(0.5 * rw, rg1);
-            t[0] = rg1; t[4] = pg1;
-        }
-    } else if (bt == BC_SYMMETRY || bt == BC_SOLID_SURFACE) {
-        double vn = xfn * s[1] + yfn * s[2] + zfn * s[3] - vfn;
-        for (int e = 0; e < 5; ++e) t[e] = s[e];
-        t[1] = s[1] - 2.0 * xfn * vn;
-        t[2] = s[2] - 2.0 * yfn * vn;
-        t[3] = s[3] - 2.0 * zfn * vn;
-    } else {  // BC_FARFIELD (codes/ns/src/NsBcSolver.cpp:140-236)
-        double rin = s[0], uin = s[1], vin = s[2], win = s[3], pin = s[4];
-        double rref = k.inflow[0], uref = k.inflow[1], vref = k.inflow[2], wref = k.inflow[3], pref = k.inflow[4];
-        double vnref = xfn * uref + yfn * vref + zfn * wref - vfn;
-        double vnin = xfn * uin + yfn * vin + zfn * win - vfn;
-        double cref = sqrt(dabs(k.gama * pref / rref));
-        double cin = sqrt(dabs(gama * pin / rin));
-        double gamm1 = gama - 1.0;
-        double velin = sqrt(sqr3(uin, vin, win));
-        if (velin > cin) {
-            if (vnin >= 0.0) { for (int e = 0; e < 5; ++e) t[e] = s[e]; }
-            else { for (int e = 0; e < 5; ++e) t[e] = k.inflow[e]; }
-        } else {
-            double riemp = vnin + 2.0 * cin / gamm1;
-            double riemm = vnref - 2.0 * cref / gamm1;
-            double vnb = 0.5 * (riemp + riemm);
-            double cb = 0.25 * (riemp - riemm) * gamm1;
-            double vtx, vty, vtz, entr;
-            if (vnb >= 0.0) {
-                entr = pin / ofxm::ofx_pow(rin, gama);
-                vtx = uin - xfn * vnin; vty = vin - yfn * vnin; vtz = win - zfn * vnin;
-            } else {
-                entr = pref / ofxm::ofx_pow(rref, gama);
-                vtx = uref - xfn * vnref; vty = vref - yfn * vnref; vtz = wref - zfn * vnref;
-            }
-            double rb = ofxm::ofx_pow((cb * cb / (entr * gama)), 1.0 / gamm1);
-            t[0] = rb; t[1] = vtx + xfn * vnb; t[2] = vty + yfn * vnb; t[3] = vtz + zfn * vnb;
-            t[4] = cb * cb * rb / gama;
-        }
-    }
-    for (int e = 0; e < 5; ++e) d.q[e * T + r] = t[e];
-    double tt = temperature(t[0], t[4], k.statecoef);
-    d.tempr[r] = tt;
-    d.visl[r] = sutherland(tt, k.ts_suth);
-}
-
 __global__ void __launch_bounds__(TB) k_ns_bc(DevMesh m, DevFields d, Consts k0) {
     int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= m.B) return;
-    const Consts k = zoned(k0, m, face_zone(m, f));
-    int l = m.lc[f];
-    double s[5];
-    for (int e = 0; e < 5; ++e) s[e] = d.q[e * m.T + l];
-    ns_bc_face(m, d, k, f, s, d.tempr[l]);
+    if (f < m.B) ns_ghost(m, d, k0, f);
 }
 
 int ns_boundary(ofx_ctx* c) {
@@ -1219,63 +1140,56 @@ __device__ void ns_solution_fix(const DevMesh& m, const DevFields& d, int i, dou
     for (int s = 0; s < 5; ++s) prim[s] *= rVol;
 }
 
-// NsCalcBoundary of one updated cell: its temperature and laminar viscosity,
-// and the ghost states of its boundary faces (boundary faces come first in
-// the cell's list; entries of faces where it is the right cell are ~f < 0).
-__device__ __forceinline__ void ns_cell_boundary(const DevMesh& m, const DevFields& d, const Consts& k, int i,
-                                                 const double* prim) {
+// NsCalcGamaT + CalcLaminarViscosity of one updated cell.
+__device__ __forceinline__ void ns_cell_gas(const DevMesh& m, const DevFields& d, const Consts& k, int i,
+                                            const double* prim) {
     const Consts kz = zoned(k, m, cell_zone(m, i));
     double t = temperature(prim[0], prim[4], kz.statecoef);
     d.tempr[i] = t;
     d.visl[i] = sutherland(t, kz.ts_suth);
-    if (!has_bface(m, i)) return;
-    for (int kk = m.c2fOff[i]; kk < m.c2fOff[i + 1]; ++kk) {
-        int f = m.c2f[kk];
-        if (f < 0 || f >= m.B) break;
-        ns_bc_face(m, d, kz, f, prim, t);
-    }
 }
 
-// Pass 2: UPDATE_FLOWFIELD; with BC also the following CALC_BOUNDARY
-// (NsCalcBoundary): T / viscosity of the cell and its boundary faces' ghosts.
+// Pass 2: UPDATE_FLOWFIELD; with GAS also the cells' part of the following
+// CALC_BOUNDARY (T and viscosity).  The ghosts are another kernel's, a thread
+// per boundary face: here a wave with a boundary cell would evaluate them one
+// after another behind the update (two dependent list loads, two pow), which took as
+// long again as everything else (12.2 us on 120,832 cells and 83 on
+// 2,524,160 with them, 6.3 and 54 without).
 // When some cell needs SolutionFix, the reference's serial loop gives its
 // neighbour average the half-updated state: lower-numbered neighbours
 // updated, higher-numbered ones not.  The lower-sweep levels of the LU-SGS
 // schedule have exactly that order (a cell's lower-numbered neighbours lie in
 // earlier levels, its higher-numbered ones in later levels), so block 0 walks
 // them in order, a barrier between levels, updating each level's cells in
-// parallel in place; the boundary pass follows once every cell is final.
-template <bool BC>
+// parallel in place.
+template <bool GAS>
 __global__ void __launch_bounds__(TB) k_ns_update_apply(DevMesh m, DevFields d, Consts k, int par) {
-    const int T = m.T;
-    double anyfix = slot_result<true>(d.slots, par, m.nz * RQ_N, RQ_FIX);
+    // the cell's loads are under way before the flag is waited for; lanes past
+    // the last cell stay active for it and store nothing
+    const int T = m.T, i0 = xcd_block((int)gridDim.x) * TB + (int)threadIdx.x;
+    const bool live = i0 < m.C;
+    const int i = live ? i0 : m.C - 1;
+    double prim0[5], dq[5], prim[5], anyfix;
+    for (int e = 0; e < 5; ++e) { prim0[e] = d.q[e * T + i]; dq[e] = d.dq[e * T + i]; }
+    wave_slot_result<1, true>(d.slots, par, m.nz * RQ_N, RQ_FIX, &anyfix);
     if (blockIdx.x == 0 && threadIdx.x < NSLOT)  // the next update's flag
         d.slots[((size_t)(1 - par) * m.nz * RQ_N + RQ_FIX) * NSLOT + threadIdx.x] = 0;
     if (anyfix == 0.0) {
-        int i = xcd_block(gridDim.x) * blockDim.x + threadIdx.x;
-        if (i >= m.C) return;
-        double prim[5];
-        ns_update_cell(d, k, T, i, prim);
+        if (!live) return;
+        ns_update_state(k, prim0, dq, prim);
         for (int e = 0; e < 5; ++e) d.q[e * T + i] = prim[e];
-        if (BC) ns_cell_boundary(m, d, k, i, prim);
+        if (GAS) ns_cell_gas(m, d, k, i, prim);
         return;
     }
     if (blockIdx.x != 0) return;
     for (int L = 0; L < m.nLevLo; ++L) {
         for (int idx = m.loOff[L] + threadIdx.x; idx < m.loOff[L + 1]; idx += blockDim.x) {
-            const int i = m.loOrder[idx];
-            double prim[5];
-            if (!ns_update_cell(d, k, T, i, prim)) ns_solution_fix(m, d, i, prim);
-            for (int e = 0; e < 5; ++e) d.q[e * T + i] = prim[e];
+            const int c = m.loOrder[idx];
+            if (!ns_update_cell(d, k, T, c, prim)) ns_solution_fix(m, d, c, prim);
+            for (int e = 0; e < 5; ++e) d.q[e * T + c] = prim[e];
+            if (GAS) ns_cell_gas(m, d, k, c, prim);
         }
         __syncthreads();
-    }
-    if (BC) {
-        for (int i = threadIdx.x; i < m.C; i += blockDim.x) {
-            double prim[5];
-            for (int e = 0; e < 5; ++e) prim[e] = d.q[e * T + i];
-            ns_cell_boundary(m, d, k, i, prim);
-        }
     }
 }
 
@@ -1289,8 +1203,10 @@ int ns_update(ofx_ctx* c) {
     return 0;
 }
 
-// flagged: the sweeps have raised the flag of parity c->par_fix.
-int ns_update_fused(ofx_ctx* c, bool flagged) {
+// With the following CALC_BOUNDARY.  flagged: the sweeps have raised the flag of
+// parity c->par_fix.  ghosts: set here, or else by the SA gradient that follows
+// (ofx_ctx::sa_ghosts).
+int ns_update_fused(ofx_ctx* c, bool flagged, bool ghosts) {
     const DevFields d = update_fields(c);
     ++c->qgen;
     if (!flagged) {
@@ -1298,6 +1214,7 @@ int ns_update_fused(ofx_ctx* c, bool flagged) {
         k_ns_update_check<<<nblk(c->m.C), TB, 0, c->stream>>>(c->m, d, c->k, c->par_fix);
     }
     k_ns_update_apply<true><<<nblk(c->m.C), TB, 0, c->stream>>>(c->m, d, c->k, c->par_fix);
+    if (ghosts && c->m.B) k_ns_bc<<<nblk(c->m.B), TB, 0, c->stream>>>(c->m, c->d, c->k);
     OFX_HIP(hipGetLastError());
     return 0;
 }

@@ -319,4 +319,87 @@ __device__ __forceinline__ double barth_fn(double dq, double minv, double maxv, 
     return (dq > maxv || dq < minv) ? r : 1.0;
 }
 
+// UNsBcSolver::CalcBc + NsBcSolver for one boundary face given the owner's
+// primitive state s and temperature towner (codes/uns/src/UNsBcSolver.cpp:55-168,
+// codes/ns/src/NsBcSolver.cpp:51-410); writes the ghost state, then the ghost
+// gamma/T/viscosity (NsCalcGamaT / CalcLaminarViscosity on F_GHOST).
+__device__ __forceinline__ void ns_bc_face(const DevMesh& m, const DevFields& d, const Consts& k, int f,
+                                           const double* s, double towner) {
+    const int T = m.T;
+    int bt = m.bct[f];
+    int r = m.C + f;
+    double xfn = m.xfn[f], yfn = m.yfn[f], zfn = m.zfn[f];
+    const double vfn = 0.0;
+    double t[5];
+    double gama = 0.5 * (k.gama + k.gama);
+    if (bt == BC_EXTRAPOLATION || bt == BC_OUTFLOW) {
+        for (int e = 0; e < 5; ++e) t[e] = s[e];
+    } else if (bt == BC_INFLOW) {
+        for (int e = 0; e < 5; ++e) t[e] = k.inflow[e];
+    } else if (bt == BC_SOLID_SURFACE && k.vismodel != 0) {
+        for (int e = 0; e < 5; ++e) t[e] = s[e];
+        t[1] = -t[1] + 2.0 * 0.0; t[2] = -t[2] + 2.0 * 0.0; t[3] = -t[3] + 2.0 * 0.0;
+        if (k.isowallbc != 0) {
+            // IsothermalVisWallBc (codes/ns/src/NsBcSolver.cpp:271-324)
+            double tlim = 0.1 * k.twall;
+            double rm = s[0], pm = s[4];
+            double pg1 = pm;
+            double tg1 = 2.0 * k.twall - towner;
+            if (tg1 < tlim) tg1 = tlim;
+            double rw = pg1 / (k.statecoef * k.twall * 1.0);
+            double rg1 = 2.0 * rw - rm;
+            rg1 = dmax(0.5 * rw, rg1);
+            t[0] = rg1; t[4] = pg1;
+        }
+    } else if (bt == BC_SYMMETRY || bt == BC_SOLID_SURFACE) {
+        double vn = xfn * s[1] + yfn * s[2] + zfn * s[3] - vfn;
+        for (int e = 0; e < 5; ++e) t[e] = s[e];
+        t[1] = s[1] - 2.0 * xfn * vn;
+        t[2] = s[2] - 2.0 * yfn * vn;
+        t[3] = s[3] - 2.0 * zfn * vn;
+    } else {  // BC_FARFIELD (codes/ns/src/NsBcSolver.cpp:140-236)
+        double rin = s[0], uin = s[1], vin = s[2], win = s[3], pin = s[4];
+        double rref = k.inflow[0], uref = k.inflow[1], vref = k.inflow[2], wref = k.inflow[3], pref = k.inflow[4];
+        double vnref = xfn * uref + yfn * vref + zfn * wref - vfn;
+        double vnin = xfn * uin + yfn * vin + zfn * win - vfn;
+        double cref = sqrt(dabs(k.gama * pref / rref));
+        double cin = sqrt(dabs(gama * pin / rin));
+        double gamm1 = gama - 1.0;
+        double velin = sqrt(sqr3(uin, vin, win));
+        if (velin > cin) {
+            if (vnin >= 0.0) { for (int e = 0; e < 5; ++e) t[e] = s[e]; }
+            else { for (int e = 0; e < 5; ++e) t[e] = k.inflow[e]; }
+        } else {
+            double riemp = vnin + 2.0 * cin / gamm1;
+            double riemm = vnref - 2.0 * cref / gamm1;
+            double vnb = 0.5 * (riemp + riemm);
+            double cb = 0.25 * (riemp - riemm) * gamm1;
+            double vtx, vty, vtz, entr;
+            if (vnb >= 0.0) {
+                entr = pin / ofxm::ofx_pow(rin, gama);
+                vtx = uin - xfn * vnin; vty = vin - yfn * vnin; vtz = win - zfn * vnin;
+            } else {
+                entr = pref / ofxm::ofx_pow(rref, gama);
+                vtx = uref - xfn * vnref; vty = vref - yfn * vnref; vtz = wref - zfn * vnref;
+            }
+            double rb = ofxm::ofx_pow((cb * cb / (entr * gama)), 1.0 / gamm1);
+            t[0] = rb; t[1] = vtx + xfn * vnb; t[2] = vty + yfn * vnb; t[3] = vtz + zfn * vnb;
+            t[4] = cb * cb * rb / gama;
+        }
+    }
+    for (int e = 0; e < 5; ++e) d.q[e * T + r] = t[e];
+    double tt = temperature(t[0], t[4], k.statecoef);
+    d.tempr[r] = tt;
+    d.visl[r] = sutherland(tt, k.ts_suth);
+}
+
+// The ghost of boundary face f from its owner's state in memory.
+__device__ __forceinline__ void ns_ghost(const DevMesh& m, const DevFields& d, const Consts& k0, int f) {
+    const Consts k = zoned(k0, m, face_zone(m, f));
+    int l = m.lc[f];
+    double s[5];
+    for (int e = 0; e < 5; ++e) s[e] = d.q[e * m.T + l];
+    ns_bc_face(m, d, k, f, s, d.tempr[l]);
+}
+
 }  // namespace ofx

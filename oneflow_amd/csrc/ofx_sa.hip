@@ -79,9 +79,17 @@ int sa_boundary(ofx_ctx* c) {
 // EG: the face terms come from the per-entry copies (DevMesh::ellg, as seen
 // from the cell; the same sums bit for bit, see k_ns_grad), a boundary
 // entry being one whose neighbour is a ghost (id C + f).
+// The first `nbc` blocks of a launch set the NS ghosts of the update before it,
+// a thread per boundary face (nothing else here reads or writes them): their
+// long chain runs beside the gradient instead of in a kernel of its own.
 template <int DIM, int MAXF, bool EG = false>
-__global__ void __launch_bounds__(TBS) k_sa_grad(DevMesh m, DevFields d, Consts k0) {
-    int i = cell_block(m, TBS) * TBS + threadIdx.x;
+__global__ void __launch_bounds__(TBS) k_sa_grad(DevMesh m, DevFields d, Consts k0, int nbc) {
+    if ((int)blockIdx.x < nbc) {
+        const int f = blockIdx.x * TBS + threadIdx.x;
+        if (f < m.B) ns_ghost(m, d, k0, f);
+        return;
+    }
+    int i = cell_block(m, TBS, nbc) * TBS + threadIdx.x;
     if (i >= m.C) return;
     const Consts k = zoned(k0, m, cell_zone(m, i));
     const int T = m.T;
@@ -408,8 +416,9 @@ template <int DIM, int MAXF>
 static void launch_sa(ofx_ctx* c, unsigned parts) {
     const DevMesh& m = c->m;
     if (parts & 1u) {
-        if (c->sagrad_variant == 1) k_sa_grad<DIM, MAXF, true><<<nblks(m.C), TBS, 0, c->stream>>>(m, c->d, c->k);
-        else k_sa_grad<DIM, MAXF><<<nblks(m.C), TBS, 0, c->stream>>>(m, c->d, c->k);
+        const int nbc = c->sa_ghosts ? (nblks(m.B) + 7) / 8 * 8 : 0, nb = nblks(m.C) + nbc;
+        if (c->sagrad_variant == 1) k_sa_grad<DIM, MAXF, true><<<nb, TBS, 0, c->stream>>>(m, c->d, c->k, nbc);
+        else k_sa_grad<DIM, MAXF><<<nb, TBS, 0, c->stream>>>(m, c->d, c->k, nbc);
     }
     if (parts & 2u) {
         const int tb = face_tile(c->saface_tb, m.F), nb = (m.F + tb - 1) / tb;
