@@ -66,13 +66,11 @@ class Mlp:
     def forward(self, x) -> np.ndarray:
         x = np.ascontiguousarray(x, np.float32)
         n = x.shape[0]
-        y = np.zeros((n, NOUT), np.float32)
+        y = np.empty((n, NOUT), np.float32)
         step = 1 << 20
         for i in range(0, n, step):
-            xs = np.ascontiguousarray(x[i:i + step])
-            ys = np.zeros((xs.shape[0], NOUT), np.float32)
+            xs, ys = x[i:i + step], y[i:i + step]  # rows in place
             self._check(self._L.ofx_mlp_forward(self.h, _fp(xs), xs.shape[0], _fp(ys)))
-            y[i:i + step] = ys
         return y
 
     def set_forward_variant(self, variant) -> None:

@@ -141,3 +141,16 @@ def test_training_keeps_weight_copies(n, batch):
         assert np.array_equal(m.forward(x), ref.forward(x))
     (l0, g0), (l1, g1) = m.gradients(x, t), ref.gradients(x, t)
     assert l0 == l1 and np.array_equal(g0, g1)
+
+
+@pytest.mark.parametrize("n", [262143, 262144, 262145, 393217, 1048576, 1048577])
+def test_piped_forward(n):
+    """Many host samples pass through in pieces (copies beside the computing):
+    the same bits as calls of fewer samples, twice in a row with other inputs."""
+    rng = np.random.default_rng(n)
+    m = net(random_params(rng, scale=1.0).astype(np.float32))
+    for _ in range(2):
+        x = rng.normal(0, 1, (n, NIN)).astype(np.float32)
+        y = m.forward(x)
+        parts = np.concatenate([m.forward(x[i:i + 100000]) for i in range(0, n, 100000)])
+        assert y.shape == (n, parts.shape[1]) and np.array_equal(y, parts)
