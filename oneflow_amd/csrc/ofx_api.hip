@@ -88,10 +88,10 @@ static int alloc_fields(ofx_ctx* c) {
     OFX_TRY(A(&d.red, 16));
     OFX_TRY(A(&d.norms, 6 * 512));
     OFX_TRY(host_sums(c, 1));
-    OFX_TRY(alloc_bytes(c, (void**)&d.slots, 2 * 12 * NSLOT * sizeof(unsigned long long)));
+    OFX_TRY(alloc_bytes(c, (void**)&d.slots, 2 * RQ_N * NSLOT * sizeof(unsigned long long)));
     // identity values in both parity buffers: min-reduced quantity 0 starts at LARGE, the others at +0
     for (int p = 0; p < 2; ++p)
-        k_fill_field<<<1, 64, 0, c->stream>>>(reinterpret_cast<double*>(d.slots) + p * 12 * NSLOT, NSLOT, LARGE);
+        k_fill_field<<<1, 64, 0, c->stream>>>(reinterpret_cast<double*>(d.slots) + (p * RQ_N + RQ_DTMIN) * NSLOT, NSLOT, LARGE);
     OFX_HIP(hipGetLastError());
     return 0;
 }

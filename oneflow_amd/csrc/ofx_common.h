@@ -554,10 +554,47 @@ __device__ __forceinline__ double group_max(double x) {
 
 // Grid-reduction quantities (slot_reduce / slot_result):
 //   0      : min time step (min)
-//   1..5   : -qmin per primitive (Venkat, max)
-//   6..10  : qmax per primitive (Venkat, max)
-//   11     : 1 if some cell needs SolutionFix (max; one flag per context)
-constexpr int RQ_DTMIN = 0, RQ_QMIN = 1, RQ_QMAX = 6, RQ_FIX = 11, RQ_N = 12;
+//   1..5   : largest difference across an interior face per primitive (Venkat, max)
+//   6      : 1 if some cell needs SolutionFix (max; one flag per context)
+// The Venkatakrishnan epsilon needs the grid's largest q_i - min(q_i, q_j) and
+// max(q_i, q_j) - q_i.  A face gives each of its cells one of the two, so both
+// are the largest |q_i - q_j| (a difference and its reverse round alike).
+constexpr int RQ_DTMIN = 0, RQ_DIFF = 1, RQ_FIX = 6, RQ_N = 7;
+
+// The minimum time step and, with QEXT, the largest differences of a single-zone
+// grid in one block reduction (the minimum as the maximum of its negative).
+template <bool QEXT>
+__device__ __forceinline__ void step_reduce(double dt, const double* diff, unsigned long long* buf, int par,
+                                            int par_lim) {
+    constexpr int NQ = QEXT ? 6 : 1;
+    __shared__ double sm[NQ][16];
+    const int nw = (int)(blockDim.x >> 6), w = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
+    double v[NQ];
+    v[0] = -dt;
+    for (int q = 1; q < NQ; ++q) v[q] = diff[q - 1];
+    int qi;
+    bool holder;
+    const double xw = wave_reduce_scatter<NQ, true>(v, lane, qi, holder);
+    if (holder) sm[qi][w] = xw;
+    __syncthreads();
+    const int slot = (int)(blockIdx.x % NSLOT), t = (int)threadIdx.x;
+    if (t < NQ) {
+        double x = sm[t][0];
+        for (int j = 1; j < nw; ++j) x = (x > sm[t][j]) ? x : sm[t][j];
+        if (t == 0)
+            atomicMin(&buf[((size_t)par * RQ_N + RQ_DTMIN) * NSLOT + slot], (unsigned long long)__double_as_longlong(-x));
+        else
+            atomicMax(&buf[((size_t)par_lim * RQ_N + RQ_DIFF + t - 1) * NSLOT + slot],
+                      (unsigned long long)__double_as_longlong(x));
+    }
+    if (blockIdx.x == 0)  // re-arm the other parities
+        for (int k = t; k < NQ * NSLOT; k += (int)blockDim.x) {
+            if (k < NSLOT)
+                buf[((size_t)(1 - par) * RQ_N + RQ_DTMIN) * NSLOT + k] = (unsigned long long)__double_as_longlong(LARGE);
+            else
+                buf[((size_t)(1 - par_lim) * RQ_N + RQ_DIFF - 1) * NSLOT + k] = 0ull;
+        }
+}
 
 // Zone of a cell / face (contexts holding several independent cases).
 __device__ __forceinline__ int cell_zone(const DevMesh& m, int i) { return m.nz > 1 ? m.zcell[i] : 0; }

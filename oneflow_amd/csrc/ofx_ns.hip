@@ -53,8 +53,8 @@ int ns_boundary(ofx_ctx* c) {
 // QEXT: the same pass also reduces the extrema of the neighbour differences
 // that fix the Venkatakrishnan epsilon (Limiter::CalcMinMaxDiff, the global
 // part, codes/usolver/src/ULimiter.cpp:597-644): per primitive the largest
-// q_i - min(q_i, q_j) and max(q_i, q_j) - q_i over interior faces, into the
-// limiter's slots of parity par_lim; the residual's gradient kernel reads them.
+// |q_i - q_j| over interior faces (RQ_DIFF), into the limiter's slots of
+// parity par_lim; the residual's gradient kernel reads them.
 // EN: the faces' normals and areas come from the per-entry copies
 // (DevMesh::ellg plane 2).
 template <int DIM, int MAXF, bool QEXT, bool EN = false>
@@ -65,7 +65,7 @@ __global__ void __launch_bounds__(TB) k_ns_timestep(DevMesh m, DevFields d, Cons
     const Consts k = zoned(k0, m, zone);
     const bool visc = k.vismodel > 0;
     double dtv = LARGE;
-    double ext[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    double ext[5] = {0, 0, 0, 0, 0};
     if (i < m.C) {
         // every load of the cell's faces is issued before the sums; each face
         // is then evaluated with its own left / right roles, in face order.
@@ -94,15 +94,12 @@ __global__ void __launch_bounds__(TB) k_ns_timestep(DevMesh m, DevFields d, Cons
             }
         }
         if (QEXT) {
-            double mn[5], mx[5];
-            for (int e = 0; e < 5; ++e) { mn[e] = qi[e]; mx[e] = qi[e]; }
 #pragma unroll
             for (int j = 0; j < MAXF; ++j) {
                 int f = ent[j] >= 0 ? ent[j] : ~ent[j];
                 if (j < n && f >= m.B)
-                    for (int e = 0; e < 5; ++e) { mn[e] = dmin(mn[e], qn[j][e]); mx[e] = dmax(mx[e], qn[j][e]); }
+                    for (int e = 0; e < 5; ++e) ext[e] = dmax(dabs(qi[e] - qn[j][e]), ext[e]);
             }
-            for (int e = 0; e < 5; ++e) { mn[e] -= qi[e]; mx[e] -= qi[e]; ext[e] = 0.0 - mn[e]; ext[5 + e] = mx[e]; }
         }
         double invsr = 0.0, vissr = 0.0;
 #pragma unroll
@@ -163,11 +160,11 @@ __global__ void __launch_bounds__(TB) k_ns_timestep(DevMesh m, DevFields d, Cons
         d.timestep[i] = dt;
         dtv = dt;
     }
-    if (m.nz > 1) zslot_reduce<1, false>(&dtv, zone, d.slots, par, RQ_N, RQ_DTMIN, m.nz);
-    else slot_reduce<1, false>(&dtv, d.slots, par, RQ_N, RQ_DTMIN);
-    if (QEXT) {
-        if (m.nz > 1) zslot_reduce<10, true>(ext, zone, d.slots, par_lim, RQ_N, RQ_QMIN, m.nz);
-        else slot_reduce<10, true>(ext, d.slots, par_lim, RQ_N, RQ_QMIN);
+    if (m.nz > 1) {
+        zslot_reduce<1, false>(&dtv, zone, d.slots, par, RQ_N, RQ_DTMIN, m.nz);
+        if (QEXT) zslot_reduce<5, true>(ext, zone, d.slots, par_lim, RQ_N, RQ_DIFF, m.nz);
+    } else {
+        step_reduce<QEXT>(dtv, ext, d.slots, par, par_lim);
     }
 }
 
@@ -178,7 +175,7 @@ __global__ void __launch_bounds__(TB) k_ns_qext(DevMesh m, DevFields d, int par_
     int i = cell_block(m, TB) * TB + threadIdx.x;
     const int T = m.T;
     const int zone = (i < m.C) ? cell_zone(m, i) : -1;
-    double ext[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    double ext[5] = {0, 0, 0, 0, 0};
     if (i < m.C) {
         const int n = m.c2fOff[i + 1] - m.c2fOff[i];
         int nb[MAXF];
@@ -188,17 +185,14 @@ __global__ void __launch_bounds__(TB) k_ns_qext(DevMesh m, DevFields d, int par_
 #pragma unroll
         for (int j = 0; j < MAXF; ++j)
             for (int e = 0; e < 5; ++e) qn[j][e] = (DIM == 2 && e == 3) ? 0.0 : d.q[e * T + nb[j]];
-        double mn[5], mx[5];
-        for (int e = 0; e < 5; ++e) { mn[e] = qi[e]; mx[e] = qi[e]; }
 #pragma unroll
         for (int j = 0; j < MAXF; ++j) {
             if (j < n && nb[j] < m.C)  // interior faces (a boundary face's neighbour is its ghost, C + f)
-                for (int e = 0; e < 5; ++e) { mn[e] = dmin(mn[e], qn[j][e]); mx[e] = dmax(mx[e], qn[j][e]); }
+                for (int e = 0; e < 5; ++e) ext[e] = dmax(dabs(qi[e] - qn[j][e]), ext[e]);
         }
-        for (int e = 0; e < 5; ++e) { mn[e] -= qi[e]; mx[e] -= qi[e]; ext[e] = 0.0 - mn[e]; ext[5 + e] = mx[e]; }
     }
-    if (m.nz > 1) zslot_reduce<10, true>(ext, zone, d.slots, par_lim, RQ_N, RQ_QMIN, m.nz);
-    else slot_reduce<10, true>(ext, d.slots, par_lim, RQ_N, RQ_QMIN);
+    if (m.nz > 1) zslot_reduce<5, true>(ext, zone, d.slots, par_lim, RQ_N, RQ_DIFF, m.nz);
+    else slot_reduce<5, true>(ext, d.slots, par_lim, RQ_N, RQ_DIFF);
 }
 
 
@@ -247,7 +241,8 @@ int ns_timestep(ofx_ctx* c, int iter) {
         else if (mf <= 8) OFX_TS(2, 8);
         else { set_error("cells with more than 8 faces are not supported"); return OFX_EINVAL; }
     } else {
-        if (mf <= 6) OFX_TS(3, 6);
+        if (mf <= 5) OFX_TS(3, 5);
+        else if (mf <= 6) OFX_TS(3, 6);
         else if (mf <= 16) OFX_TS(3, 16);
         else { set_error("cells with more than 16 faces are not supported"); return OFX_EINVAL; }
     }
@@ -255,7 +250,7 @@ int ns_timestep(ofx_ctx* c, int iter) {
     if (c->m.nz > 1) {
         k_zone_extract<false><<<c->m.nz, 64, 0, c->stream>>>(c->d.slots, c->par_dt, RQ_N, RQ_DTMIN, 1, c->m.nz, c->d.zred);
         if (qext)
-            k_zone_extract<true><<<c->m.nz, 256, 0, c->stream>>>(c->d.slots, c->par_lim, RQ_N, RQ_QMIN, 10, c->m.nz,
+            k_zone_extract<true><<<c->m.nz, 256, 0, c->stream>>>(c->d.slots, c->par_lim, RQ_N, RQ_DIFF, 5, c->m.nz,
                                                                  c->d.zred);
     }
     OFX_HIP(hipGetLastError());
@@ -289,8 +284,8 @@ __global__ void __launch_bounds__(TB) k_ns_grad(DevMesh m, DevFields d, Consts k
     const int i = live ? i0 : m.C - 1;
     const int T = m.T;
     const Consts k = zoned(k0, m, cell_zone(m, i));
-    double ext[10];
-    if (LIM == 2 && m.nz == 1) wave_slot_result<10, true>(d.slots, par, m.nz * RQ_N, RQ_QMIN, ext);
+    double ext[5];
+    if (LIM == 2 && m.nz == 1) wave_slot_result<5, true>(d.slots, par, m.nz * RQ_N, RQ_DIFF, ext);
     const int n = m.c2fOff[i + 1] - m.c2fOff[i];
     int ent[MAXF], nb[MAXF];
     if (EG && LIM != 1) cell_nbs<MAXF>(m, i, nb);
@@ -409,16 +404,12 @@ __global__ void __launch_bounds__(TB) k_ns_grad(DevMesh m, DevFields d, Consts k
             double lo_d = w2 ? 0.0 : mn[s] - qi[s], hi_d = w2 ? 0.0 : mx[s] - qi[s];
             double eps1 = 0.0;
             if (LIM == 2) {
-                double lo, hi;
+                double diff = ext[s];
                 if (m.nz > 1) {
-                    const double* zr = d.zred + (size_t)m.zcell[i] * RQ_N;
-                    lo = zr[RQ_QMIN + s];
-                    hi = zr[RQ_QMAX + s];
-                } else {
-                    lo = ext[s];
-                    hi = ext[5 + s];
+                    diff = d.zred[(size_t)m.zcell[i] * RQ_N + RQ_DIFF + s];
+                    asm volatile("" : "+v"(diff));  // (a select of the two addresses would put ext in scratch)
                 }
-                double eps = k.vencat_coef * dmax(hi - (-lo), 1.0);
+                double eps = k.vencat_coef * dmax(diff - (-diff), 1.0);
                 eps1 = eps * eps + SMALL;
             }
 #pragma unroll
@@ -744,7 +735,7 @@ static void launch_qext(ofx_ctx* c, bool force) {
     c->par_lim ^= 1;
     k_ns_qext<DIM, MAXF><<<nblk(c->m.C), TB, 0, c->stream>>>(c->m, c->d, c->par_lim);
     if (c->m.nz > 1)
-        k_zone_extract<true><<<c->m.nz, 256, 0, c->stream>>>(c->d.slots, c->par_lim, RQ_N, RQ_QMIN, 10, c->m.nz,
+        k_zone_extract<true><<<c->m.nz, 256, 0, c->stream>>>(c->d.slots, c->par_lim, RQ_N, RQ_DIFF, 5, c->m.nz,
                                                              c->d.zred);
     c->qext_gen = c->qgen;
 }
@@ -814,7 +805,8 @@ int ns_residual_parts(ofx_ctx* c, unsigned parts, bool reuse_ext) {
         else if (mf <= 8) launch_cells<2, 8>(c, parts, reuse_ext);
         else { set_error("cells with more than 8 faces are not supported"); return OFX_EINVAL; }
     } else {
-        if (mf <= 6) launch_cells<3, 6>(c, parts, reuse_ext);
+        if (mf <= 5) launch_cells<3, 5>(c, parts, reuse_ext);
+        else if (mf <= 6) launch_cells<3, 6>(c, parts, reuse_ext);
         else if (mf <= 8) launch_cells<3, 8>(c, parts, reuse_ext);
         else if (mf <= 16) launch_cells<3, 16>(c, parts, reuse_ext);
         else { set_error("cells with more than 16 faces are not supported"); return OFX_EINVAL; }
@@ -1040,8 +1032,11 @@ __global__ void __launch_bounds__(64 * (MAXF + 1)) k_ns_sweep_split(DevMesh m, D
 // 10.5 / 6.0, 60,160 12.5 / 9.9, 377,600 44 / 51 (there the memory system is
 // busy either way and the exchange through LDS costs); 3-D cells 1,024 10.4 / 5.7,
 // 53,504 12.4 / 9.1, 321,280 58.5 / 56.4, 910,336 155 / 151, so always.
+// (Cells of at most five faces, prisms and tets, have kernels of their own throughout:
+// two of 182 registers with six, the time step fits three waves per SIMD with five,
+// 235 -> 202 us on 2,524,160 cells, and the limiter's gradient takes 299 for 307.)
 template <int MAXF>
-static bool split_level(int nc) { return MAXF == 6 || nc <= 131072; }
+static bool split_level(int nc) { return MAXF >= 5 || nc <= 131072; }
 
 template <int MAXF, int VM, bool EN>
 static void launch_lusgs(ofx_ctx* c, int lo_first, int pf) {
@@ -1064,7 +1059,7 @@ static void launch_lusgs(ofx_ctx* c, int lo_first, int pf) {
                     continue;
                 }
             }
-            if constexpr (!(EN && MAXF == 6)) {
+            if constexpr (!(EN && (MAXF == 5 || MAXF == 6))) {
                 if (up) k_ns_sweep_level<true, MAXF, VM, EN><<<nblk(nc), TB, 0, c->stream>>>(m, c->d, c->k, b, e, bs, pd, pf);
                 else k_ns_sweep_level<false, MAXF, VM, EN><<<nblk(nc), TB, 0, c->stream>>>(m, c->d, c->k, b, e, bs, pd, pf);
             }
@@ -1090,6 +1085,7 @@ int ns_lusgs(ofx_ctx* c, int lo_first, bool flag) {
     if (c->sweep) return pipelined_lusgs_ns(c);
     const int mf = c->m.maxFacesPerCell, pf = flag ? c->par_fix : -1;
     if (mf <= 4) launch_lusgs_vm<4>(c, lo_first, pf);
+    else if (mf <= 5) launch_lusgs_vm<5>(c, lo_first, pf);
     else if (mf <= 6) launch_lusgs_vm<6>(c, lo_first, pf);
     else if (mf <= 8) launch_lusgs_vm<8>(c, lo_first, pf);
     else if (mf <= 16) launch_lusgs_vm<16>(c, lo_first, pf);

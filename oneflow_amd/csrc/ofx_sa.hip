@@ -439,7 +439,8 @@ int sa_residual_parts(ofx_ctx* c, unsigned parts) {
         else if (mf <= 8) launch_sa<2, 8>(c, parts);
         else { set_error("cells with more than 8 faces are not supported"); return OFX_EINVAL; }
     } else {
-        if (mf <= 6) launch_sa<3, 6>(c, parts);
+        if (mf <= 5) launch_sa<3, 5>(c, parts);
+        else if (mf <= 6) launch_sa<3, 6>(c, parts);
         else if (mf <= 12) launch_sa<3, 12>(c, parts);
         else { set_error("cells with more than 12 faces are not supported"); return OFX_EINVAL; }
     }
@@ -515,6 +516,7 @@ int sa_lusgs(ofx_ctx* c, int lo_first) {
     if (c->sweep) return pipelined_lusgs_sa(c);
     int mf = c->m.maxFacesPerCell;
     if (mf <= 4) launch_sa_lusgs<4>(c, lo_first);
+    else if (mf <= 5) launch_sa_lusgs<5>(c, lo_first);
     else if (mf <= 6) launch_sa_lusgs<6>(c, lo_first);
     else if (mf <= 8) launch_sa_lusgs<8>(c, lo_first);
     else if (mf <= 16) launch_sa_lusgs<16>(c, lo_first);
