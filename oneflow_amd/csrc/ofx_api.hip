@@ -528,8 +528,10 @@ int step_launch(ofx_ctx* c, int iter) {
     const bool flag = levels && !(ns_first && c->sched.lone);
     if (flag) c->par_fix ^= 1;
     c->fuse_first = ns_first;
+    const int early = sa_early_ok(c);
+    c->sa_early = early;
     int rc = ns_residual(c, true);
-    c->fuse_first = 0;
+    c->fuse_first = c->sa_early = 0;
     OFX_TRY(rc);
     OFX_TRY(ns_lusgs(c, ns_first, flag));
     const bool sa = c->k.vismodel == 3;
@@ -537,8 +539,9 @@ int step_launch(ofx_ctx* c, int iter) {
     if (sa) {
         c->fuse_first = levels;
         c->sa_ghosts = 1;
+        c->sa_early = early;
         rc = sa_residual(c);
-        c->fuse_first = c->sa_ghosts = 0;
+        c->fuse_first = c->sa_ghosts = c->sa_early = 0;
         OFX_TRY(rc);
         OFX_TRY(sa_lusgs(c, levels));
         OFX_TRY(sa_update_fused(c));

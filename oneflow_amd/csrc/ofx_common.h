@@ -239,6 +239,7 @@ struct ofx_ctx {
     int gen = 0;  // bumped whenever launch parameters change (mesh, config, tiles)
     bool dist_valid = false;  // wall distance computed for the current mesh / zones
     int sa_ghosts = 0;   // 1 while a full step leaves the NS ghosts of its update to the SA gradient
+    int sa_early = 0;    // 1 while a full step's NS gradient evaluates the SA gradient (sa_early_ok)
     int fuse_first = 0;  // 1 while a full step computes the first lower-sweep level in the residual gathers
     // several zones: cell / boundary-face starts (nz + 1 each), host copies of
     // the per-zone constants and configurations
@@ -248,6 +249,14 @@ struct ofx_ctx {
 };
 
 namespace ofx {
+// Faces per cell the NS gradient with the SA gradient in it is built for: more
+// would not fit the registers (222 of 256 without it in 3-D).
+constexpr int sa_early_faces(int dim) { return dim == 2 ? 4 : 5; }
+inline bool sa_early_ok(const ofx_ctx* c) {
+    const int mf = c->m.maxFacesPerCell;
+    return c->k.vismodel == 3 && c->grad_variant == 1 && c->sagrad_variant == 1 &&
+           (c->m.dim == 2 ? mf <= 4 : mf <= 5);
+}
 // Threads per block of a face kernel over F faces.  256 unless that leaves
 // fewer than two blocks per CU: 64 then spreads the faces over all of them
 // (11,264 cells: 6.2 -> 5.1 us, 46,080: 9.0 -> 7.6; 120,832 and more: the same).

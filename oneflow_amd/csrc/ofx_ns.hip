@@ -10,6 +10,7 @@
 #include "ofx_lusgs.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace ofx {
 
@@ -275,7 +276,10 @@ int ns_timestep(ofx_ctx* c, int iter) {
 // EG: the face terms come from the per-entry copies (DevMesh::ellg), loaded
 // with the neighbour ids rather than after the face ids; a boundary entry is
 // one whose neighbour is a ghost (id >= C).
-template <int DIM, int MAXF, int LIM, bool EG = false>
+// SAG (with EG, inside a full step): the SA gradient of nu_tilde from the same
+// terms, which the NS update does not change; cells with boundary faces, whose
+// ghosts depend on the updated state, are done again by k_sa_grad_boundary.
+template <int DIM, int MAXF, int LIM, bool EG = false, bool SAG = false>
 __global__ void __launch_bounds__(TB) k_ns_grad(DevMesh m, DevFields d, Consts k0, int par) {
     // Every lane stays active to the end (the extrema are read per wave):
     // lanes past the last cell evaluate it and store nothing.
@@ -296,7 +300,8 @@ __global__ void __launch_bounds__(TB) k_ns_grad(DevMesh m, DevFields d, Consts k
     // x A, y A}, gz = outward z A; otherwise the face's record as stored.
     // dx, dy, dz: face centre - this cell's centre.
     dvec4 gw[MAXF];
-    double gz[MAXF], qn[MAXF][5], dx[MAXF], dy[MAXF], dz[MAXF];
+    double gz[MAXF], qn[MAXF][5], dx[MAXF], dy[MAXF], dz[MAXF], nun[SAG ? MAXF : 1];
+    const double nui = SAG ? d.turbq[i] : 0.0;
     const size_t S = (size_t)m.ellw * m.C;
     int imask = 0;  // EG: bit j set for an interior entry
 #pragma unroll
@@ -328,6 +333,7 @@ __global__ void __launch_bounds__(TB) k_ns_grad(DevMesh m, DevFields d, Consts k
                 }
             }
             for (int e2 = 0; e2 < 5; ++e2) qn[j][e2] = (DIM == 2 && e2 == 3) ? 0.0 : d.q[e2 * T + c];
+            if (SAG) nun[j] = d.turbq[c];
         }
     }
     double mn[5], mx[5];
@@ -335,6 +341,7 @@ __global__ void __launch_bounds__(TB) k_ns_grad(DevMesh m, DevFields d, Consts k
     double ti = temperature(qi[0], qi[4], k.statecoef);
     double acc[6][3];
     for (int s = 0; s < 6; ++s) acc[s][0] = acc[s][1] = acc[s][2] = 0.0;
+    double nx = 0.0, ny = 0.0, nz = 0.0;
     // EG: with the weights and the normal taken as seen from this cell, the
     // sums are those of the face records: for the right cell, cl*vn + cr*vi
     // is w_self*vi + w_nb*vn (a commuted sum) and acc - n*v is acc + (-n)*v,
@@ -350,6 +357,10 @@ __global__ void __launch_bounds__(TB) k_ns_grad(DevMesh m, DevFields d, Consts k
                     double vi = s < 5 ? qi[s] : ti, vn = s < 5 ? qn[j][s] : tn;
                     double value = ws * vi + wn * vn;
                     acc[s][0] += fnxa * value; acc[s][1] += fnya * value; acc[s][2] += fnza * value;
+                }
+                if (SAG) {
+                    double value = ws * nui + wn * nun[j];
+                    nx += fnxa * value; ny += fnya * value; nz += fnza * value;
                 }
             } else {
                 bool own = ent[j] >= 0;  // this cell is the face's left cell
@@ -378,6 +389,11 @@ __global__ void __launch_bounds__(TB) k_ns_grad(DevMesh m, DevFields d, Consts k
             if (DIM == 2 && s == 3) continue;
             for (int a = 0; a < DIM; ++a) d.grad[(a * 6 + s) * T + i] = g[s][a];
         }
+    if (SAG && live) {
+        d.tgrad[i] = nx * ovol;
+        d.tgrad[T + i] = ny * ovol;
+        d.tgrad[2 * T + i] = nz * ovol;
+    }
     if (LIM == 0) return;
     double dot[MAXF];
     if (LIM == 1) {
@@ -755,17 +771,22 @@ static void launch_cells(ofx_ctx* c, unsigned parts, bool reuse_ext) {
     if (parts & 2u) launch_qext<DIM, MAXF>(c, true);
     if (parts & 1u) {
         const bool eg = c->grad_variant == 1;
-        if (k.ilim == 2) {
-            if (!(parts & 2u)) launch_qext<DIM, MAXF>(c, !reuse_ext);
-            if (eg) k_ns_grad<DIM, MAXF, 2, true><<<nblk(C1), TB, 0, c->stream>>>(c->m, c->d, k, c->par_lim);
-            else k_ns_grad<DIM, MAXF, 2><<<nblk(C1), TB, 0, c->stream>>>(c->m, c->d, k, c->par_lim);
-        } else if (k.ilim == 1) {
-            if (eg) k_ns_grad<DIM, MAXF, 1, true><<<nblk(C1), TB, 0, c->stream>>>(c->m, c->d, k, 0);
-            else k_ns_grad<DIM, MAXF, 1><<<nblk(C1), TB, 0, c->stream>>>(c->m, c->d, k, 0);
-        } else {
-            if (eg) k_ns_grad<DIM, MAXF, 0, true><<<nblk(C1), TB, 0, c->stream>>>(c->m, c->d, k, 0);
-            else k_ns_grad<DIM, MAXF, 0><<<nblk(C1), TB, 0, c->stream>>>(c->m, c->d, k, 0);
-        }
+        if (k.ilim == 2 && !(parts & 2u)) launch_qext<DIM, MAXF>(c, !reuse_ext);
+        const int par = k.ilim == 2 ? c->par_lim : 0;
+        auto grad = [&](auto lim) {
+            constexpr int LIM = decltype(lim)::value;
+            if constexpr (MAXF == sa_early_faces(DIM)) {
+                if (c->sa_early) {
+                    k_ns_grad<DIM, MAXF, LIM, true, true><<<nblk(C1), TB, 0, c->stream>>>(c->m, c->d, k, par);
+                    return;
+                }
+            }
+            if (eg) k_ns_grad<DIM, MAXF, LIM, true><<<nblk(C1), TB, 0, c->stream>>>(c->m, c->d, k, par);
+            else k_ns_grad<DIM, MAXF, LIM><<<nblk(C1), TB, 0, c->stream>>>(c->m, c->d, k, par);
+        };
+        if (k.ilim == 2) grad(std::integral_constant<int, 2>{});
+        else if (k.ilim == 1) grad(std::integral_constant<int, 1>{});
+        else grad(std::integral_constant<int, 0>{});
     }
     if (parts & 4u) launch_face_dim<DIM>(c, visc);
     if ((parts & 8u) && c->gather_variant == 1) {

@@ -79,18 +79,8 @@ int sa_boundary(ofx_ctx* c) {
 // EG: the face terms come from the per-entry copies (DevMesh::ellg, as seen
 // from the cell; the same sums bit for bit, see k_ns_grad), a boundary
 // entry being one whose neighbour is a ghost (id C + f).
-// The first `nbc` blocks of a launch set the NS ghosts of the update before it,
-// a thread per boundary face (nothing else here reads or writes them): their
-// long chain runs beside the gradient instead of in a kernel of its own.
-template <int DIM, int MAXF, bool EG = false>
-__global__ void __launch_bounds__(TBS) k_sa_grad(DevMesh m, DevFields d, Consts k0, int nbc) {
-    if ((int)blockIdx.x < nbc) {
-        const int f = blockIdx.x * TBS + threadIdx.x;
-        if (f < m.B) ns_ghost(m, d, k0, f);
-        return;
-    }
-    int i = cell_block(m, TBS, nbc) * TBS + threadIdx.x;
-    if (i >= m.C) return;
+template <int DIM, int MAXF, bool EG>
+__device__ __forceinline__ void sa_grad_cell(const DevMesh& m, const DevFields& d, const Consts& k0, int i) {
     const Consts k = zoned(k0, m, cell_zone(m, i));
     const int T = m.T;
     const int n = m.c2fOff[i + 1] - m.c2fOff[i];
@@ -149,6 +139,33 @@ __global__ void __launch_bounds__(TBS) k_sa_grad(DevMesh m, DevFields d, Consts 
     d.tgrad[i] = ax * ovol;
     d.tgrad[T + i] = ay * ovol;
     d.tgrad[2 * T + i] = az * ovol;
+}
+
+// The first `nbc` blocks of a launch set the NS ghosts of the update before it,
+// a thread per boundary face (nothing else here reads or writes them): their
+// long chain runs beside the gradient instead of in a kernel of its own.
+template <int DIM, int MAXF, bool EG = false>
+__global__ void __launch_bounds__(TBS) k_sa_grad(DevMesh m, DevFields d, Consts k0, int nbc) {
+    if ((int)blockIdx.x < nbc) {
+        const int f = blockIdx.x * TBS + threadIdx.x;
+        if (f < m.B) ns_ghost(m, d, k0, f);
+        return;
+    }
+    int i = cell_block(m, TBS, nbc) * TBS + threadIdx.x;
+    if (i < m.C) sa_grad_cell<DIM, MAXF, EG>(m, d, k0, i);
+}
+
+// After an NS gradient that held the SA gradient: the cells with boundary faces
+// (a thread per boundary face, the cell's first one does it) and, in the
+// first half of the blocks, the NS ghosts.
+template <int DIM, int MAXF>
+__global__ void __launch_bounds__(TBS) k_sa_grad_boundary(DevMesh m, DevFields d, Consts k0) {
+    const int half = (int)gridDim.x / 2, b = (int)blockIdx.x;
+    const int f = (b < half ? b : b - half) * TBS + threadIdx.x;
+    if (f >= m.B) return;
+    if (b < half) { ns_ghost(m, d, k0, f); return; }
+    const int i = m.lc[f];
+    if (m.ellf[i] == f) sa_grad_cell<DIM, MAXF, true>(m, d, k0, i);
 }
 
 // Normal derivative of nu_tilde at face f by face-gradient method VM
@@ -415,6 +432,14 @@ __global__ void __launch_bounds__(TBS) k_sa_cell(DevMesh m, DevFields d, Consts 
 template <int DIM, int MAXF>
 static void launch_sa(ofx_ctx* c, unsigned parts) {
     const DevMesh& m = c->m;
+    if (parts & 1u) {
+        if constexpr (MAXF == sa_early_faces(DIM)) {
+            if (c->sa_early) {
+                if (m.B) k_sa_grad_boundary<DIM, MAXF><<<2 * nblks(m.B), TBS, 0, c->stream>>>(m, c->d, c->k);
+                parts &= ~1u;
+            }
+        }
+    }
     if (parts & 1u) {
         const int nbc = c->sa_ghosts ? (nblks(m.B) + 7) / 8 * 8 : 0, nb = nblks(m.C) + nbc;
         if (c->sagrad_variant == 1) k_sa_grad<DIM, MAXF, true><<<nb, TBS, 0, c->stream>>>(m, c->d, c->k, nbc);
