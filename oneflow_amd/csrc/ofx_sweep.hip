@@ -39,10 +39,10 @@
 // operations, the division), 0.6-1 us where levels are wider than a round or
 // cells have three dependencies, and ~2 us per range the chain crosses.
 // Measured, lower + upper sweep with the preparation, NS / SA in us:
-//   RAE2822, 23,552 cells, 431 levels:      594 / 351 (one 1024-thread workgroup
+//   RAE2822, 23,552 cells, 431 levels:      585 / 351 (one 1024-thread workgroup
 //     walking all levels with a barrier between them: 9564 / 1188)
 //   O-grid, 120,832 cells, 747 levels:     1430 / 722 (18645 / 2661)
-//   plate, 960 cells, 63 levels:             89 / 58 (a launch per level: 862 / 474)
+//   plate, 960 cells, 63 levels:             82 / 58 (a launch per level: 862 / 474)
 #include <algorithm>
 #include <memory>
 #include <new>
@@ -115,6 +115,8 @@ struct SweepSet {
 
 namespace {
 
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+
 // The static parts of the streams (SweepMeta, increment slots).
 template <int NEQ>
 __global__ void __launch_bounds__(256) k_sweep_init(SweepDev s, int NE, bool upper) {
@@ -140,35 +142,56 @@ __device__ __forceinline__ void sweep_reset(const SweepDev& lo, const SweepDev& 
 // NS preparation: every interior face term of every cell without its
 // increment, the residual and the diagonal, into both streams.  A record is
 // {lmd1, x1, x2, c2, af, area, visrad, u, v, w, hm, nx, ny, nz, vn, slot}.
+// A block takes 64 cells: wave j evaluates entry j of their face lists (and j +
+// PREP_W .. of long ones), a last wave the diagonals.  A thread that evaluated
+// all faces of its cell was one long chain per wave with few waves: 960 cells
+// 13.5 us, 23,552 cells 17.0 (now 6.4 and 10.9).
+template <int MAXF>
+constexpr int PREP_W = MAXF < 6 ? MAXF : 6;
 template <int MAXF, int VM, bool EN>
-__global__ void __launch_bounds__(256) k_sweep_prep_ns(DevMesh m, DevFields d, Consts k0, int par, SweepDev lo,
-                                                       SweepDev up, int NE, int* ticket) {
+__global__ void __launch_bounds__(64 * (PREP_W<MAXF> + 1)) k_sweep_prep_ns(DevMesh m, DevFields d, Consts k0, int par,
+                                                                          SweepDev lo, SweepDev up, int NE,
+                                                                          int* ticket) {
     using S = Shape<5>;
+    constexpr int PW = PREP_W<MAXF>;
     sweep_reset(lo, up, 0, 5, ticket);
-    const int i0 = xcd_block(gridDim.x) * 256 + threadIdx.x;
+    const int w = uniform((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
+    const int i0 = xcd_block((int)gridDim.x) * 64 + lane;
     const bool live = i0 < m.C;
     const int i = live ? i0 : m.C - 1;  // every lane stays active for the wave reduction
-    double mindt;
-    wave_slot_result<1, false>(d.slots, par, m.nz * RQ_N, RQ_DTMIN, &mindt);
-    mindt = zone_mindt(m, d, i, mindt);
-    const Consts k = zoned(k0, m, cell_zone(m, i));
     const int T = m.T;
-    const int n = m.c2fOff[i + 1] - m.c2fOff[i];
-    int ent[MAXF], nb[MAXF];
-    cell_faces<MAXF>(m, i, ent, nb);
-    const int lomask = m.lomask[i];
-    const double rl = d.q[i], ul = d.q[T + i], vl = d.q[2 * T + i], wl = d.q[3 * T + i], pl = d.q[4 * T + i];
-    double xi = 0.0, yi = 0.0, zi = 0.0;
-    if (VM == 2 && !EN) { xi = m.xcc[i]; yi = m.ycc[i]; zi = m.zcc[i]; }
-    const double rad = ns_impsr(m, d, k, i, mindt);
+    const Consts k = zoned(k0, m, cell_zone(m, i));
     const size_t st = (size_t)S::stride(NE);
     char* cl = lo.stream[0] + lo.posOf[i] * st;
     char* cu = up.stream[0] + up.posOf[i] * st;
-    int nl = 0, nu = 0;
+    if (w == PW) {
+        double mindt;
+        wave_slot_result<1, false>(d.slots, par, m.nz * RQ_N, RQ_DTMIN, &mindt);
+        const double rad = ns_impsr(m, d, k, i, zone_mindt(m, d, i, mindt));
+        if (!live) return;
+        double* vl5 = reinterpret_cast<double*>(cl);
+        for (int e = 0; e < 5; ++e) vl5[e] = d.res[e * T + i];
+        const double y = ofxm::div_reciprocal(rad);
+        vl5[5] = rad;
+        vl5[6] = y;
+        reinterpret_cast<double*>(cu)[5] = rad;
+        reinterpret_cast<double*>(cu)[6] = y;
+        return;
+    }
+    const int n = m.c2fOff[i + 1] - m.c2fOff[i], lomask = m.lomask[i];
+    int ent[MAXF];
+#pragma unroll
+    for (int j = 0; j < MAXF; ++j) ent[j] = (j < m.ellw) ? m.ellf[(size_t)j * m.C + i] : 0;
+    int nbound = 0;  // boundary faces come first
+#pragma unroll
+    for (int j = 0; j < MAXF; ++j) nbound += j < n && ent[j] >= 0 && ent[j] < m.B;
+    const double rl = d.q[i], ul = d.q[T + i], vl = d.q[2 * T + i], wl = d.q[3 * T + i], pl = d.q[4 * T + i];
+    double xi = 0.0, yi = 0.0, zi = 0.0;
+    if (VM == 2 && !EN) { xi = m.xcc[i]; yi = m.ycc[i]; zi = m.zcc[i]; }
 #pragma unroll
     for (int j = 0; j < MAXF; ++j) {
-        const int f = ent[j] >= 0 ? ent[j] : ~ent[j], r = nb[j];
-        if (!live || j >= n || f < m.B) continue;
+        if (j % PW != w || !live || j >= n || j < nbound) continue;
+        const int f = ent[j] >= 0 ? ent[j] : ~ent[j], r = m.elln[(size_t)j * m.C + i];
         double nx, ny, nz, ar;
         if (EN) {
             const dvec4 r4 = m.ellg[(size_t)(2 * m.ellw + j) * m.C + i];
@@ -188,9 +211,10 @@ __global__ void __launch_bounds__(256) k_sweep_prep_ns(DevMesh m, DevFields d, C
             else dist = dabs(nx * (m.xcc[r] - xi) + ny * (m.ycc[r] - yi) + nz * (m.zcc[r] - zi));
         }
         const LuFace c = ns_lusgs_coef<VM>(k, nx, ny, nz, vfn, ar, rl, ul, vl, wl, pl, pj, visl, vist, volr, dist);
+        // the record's place: lower (upper) neighbours among the entries before it
+        const int before = __popc(lomask & ((1 << j) - 1));
         const bool lower = (lomask >> j) & 1;
-        dvec2* o = reinterpret_cast<dvec2*>((lower ? cl : cu) + S::HDR + S::REC * (lower ? nl : nu));
-        if (lower) ++nl; else ++nu;
+        dvec2* o = reinterpret_cast<dvec2*>((lower ? cl : cu) + S::HDR + S::REC * (lower ? before : j - nbound - before));
         o[0] = dvec2{c.lmd1, c.x1};
         o[1] = dvec2{c.x2, c.c2};
         o[2] = dvec2{c.af, ar};
@@ -199,15 +223,6 @@ __global__ void __launch_bounds__(256) k_sweep_prep_ns(DevMesh m, DevFields d, C
         o[5] = dvec2{c.hm, nx};
         o[6] = dvec2{ny, nz};
         reinterpret_cast<double*>(o)[14] = c.vn;
-    }
-    if (live) {
-        double* vl5 = reinterpret_cast<double*>(cl);
-        for (int e = 0; e < 5; ++e) vl5[e] = d.res[e * T + i];
-        const double y = ofxm::div_reciprocal(rad);
-        vl5[5] = rad;
-        vl5[6] = y;
-        reinterpret_cast<double*>(cu)[5] = rad;
-        reinterpret_cast<double*>(cu)[6] = y;
     }
 }
 
@@ -250,8 +265,6 @@ __global__ void __launch_bounds__(256) k_sweep_prep_sa(DevMesh m, DevFields d, S
 // The compiler keeps LDS accesses on their side (and loads counters anew); the
 // hardware completes a wave's LDS operations in order.
 #define SW_ORDER() asm volatile("" ::: "memory")
-
-__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
 // The value of the lane eight up in the row of 16.
 __device__ __forceinline__ double from_upper_half(double x) {
@@ -552,11 +565,11 @@ int sweep_pair_ne(ofx_ctx* c, SweepSet& s, double* dq) {
 
 template <int MAXF, int VM>
 void prep_ns(ofx_ctx* c, SweepSet& s) {
-    const int nb = (c->m.C + 255) / 256;
+    const int nb = (c->m.C + 63) / 64, nt = 64 * (PREP_W<MAXF> + 1);
     if (c->normal_variant == 1)
-        k_sweep_prep_ns<MAXF, VM, true><<<nb, 256, 0, c->stream>>>(c->m, c->d, c->k, c->par_dt, s.d[0], s.d[1], s.NE, s.ticket);
+        k_sweep_prep_ns<MAXF, VM, true><<<nb, nt, 0, c->stream>>>(c->m, c->d, c->k, c->par_dt, s.d[0], s.d[1], s.NE, s.ticket);
     else
-        k_sweep_prep_ns<MAXF, VM, false><<<nb, 256, 0, c->stream>>>(c->m, c->d, c->k, c->par_dt, s.d[0], s.d[1], s.NE, s.ticket);
+        k_sweep_prep_ns<MAXF, VM, false><<<nb, nt, 0, c->stream>>>(c->m, c->d, c->k, c->par_dt, s.d[0], s.d[1], s.NE, s.ticket);
 }
 template <int MAXF>
 void prep_ns_vm(ofx_ctx* c, SweepSet& s) {
