@@ -88,8 +88,9 @@ struct DevMesh {
     //     cell; cr, cl when it is the right one) and the area-weighted normal
     //     pointing out of the cell (negated for the right cell);
     //   plane 1 {nz A, xf - xc, yf - yc, zf - zc}: the normal's z part (out of
-    //     the cell) and the face centre relative to the cell centre (z parts
-    //     zero in 2-D).
+    //     the cell) and the face centre relative to the cell centre; in 2-D
+    //     only {xf - xc, yf - yc}, packed 16 bytes apart from the plane's start
+    //     (half the bytes of records with zero z parts).
     // The gradients' sums are the same bits as from fgg / frec / fz (a sum is
     // commutative, and acc - x == acc + (-x) in IEEE arithmetic).  For the
     // time step and the LU-SGS sweeps, as the face stores them:

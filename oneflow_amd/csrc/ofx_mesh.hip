@@ -193,7 +193,8 @@ __global__ void k_ell_geom(DevMesh m) {
             v[7] = (DIM == 3) ? (own ? z4.y : z4.z) : 0.0;
         }
         m.ellg[o] = dvec4{v[0], v[1], v[2], v[3]};
-        m.ellg[S + o] = dvec4{v[4], v[5], v[6], v[7]};
+        if (DIM == 3) m.ellg[S + o] = dvec4{v[4], v[5], v[6], v[7]};
+        else reinterpret_cast<dvec2*>(m.ellg + S)[o] = dvec2{v[5], v[6]};
         dvec4 nrm{0.0, 0.0, 0.0, 0.0};
         if (j < n) {
             const int e = m.ellf[o], f = e >= 0 ? e : ~e;

@@ -312,14 +312,19 @@ __global__ void __launch_bounds__(TB) k_ns_grad(DevMesh m, DevFields d, Consts k
                 imask |= (c < m.C) << j;
                 const size_t o = (size_t)j * m.C + i;
                 gw[j] = m.ellg[o];
-                if (DIM == 3 || LIM != 0) {
+                if (DIM == 3) {
                     const dvec4 b4 = m.ellg[S + o];
-                    gz[j] = (DIM == 3) ? b4.x : 0.0;
+                    gz[j] = b4.x;
                     dx[j] = b4.y;
                     dy[j] = b4.z;
-                    dz[j] = (DIM == 3) ? b4.w : 0.0;
+                    dz[j] = b4.w;
                 } else {
-                    gz[j] = 0.0;
+                    gz[j] = dz[j] = 0.0;
+                    if (LIM != 0) {
+                        const dvec2 b2 = reinterpret_cast<const dvec2*>(m.ellg + S)[o];
+                        dx[j] = b2.x;
+                        dy[j] = b2.y;
+                    }
                 }
             } else {
                 const int e = ent[j], f = e >= 0 ? e : ~e;
