@@ -41,7 +41,7 @@
 // Measured, lower + upper sweep with the preparation, NS / SA in us:
 //   RAE2822, 23,552 cells, 431 levels:      585 / 351 (one 1024-thread workgroup
 //     walking all levels with a barrier between them: 9564 / 1188)
-//   O-grid, 120,832 cells, 747 levels:     1430 / 722 (18645 / 2661)
+//   O-grid, 120,832 cells, 747 levels:     1380 / 656 (18645 / 2661)
 //   plate, 960 cells, 63 levels:             82 / 58 (a launch per level: 862 / 474)
 #include <algorithm>
 #include <memory>
@@ -60,11 +60,20 @@ typedef int sw_int2 __attribute__((ext_vector_type(2)));
 constexpr unsigned long long SW_EMPTY = 0x7FF0A5A5DEADBEEFull;  // a signalling NaN: never a result of arithmetic
 constexpr int SPIN_MAX = 1 << 22;
 constexpr int SW_LDS = 160 * 1024;
-// Most cells of a range, and cells per level it may hold.  Measured (NS + SA
-// pair, us) on the 23,552-cell RAE2822, the 11,088-cell plate and a 120,832-cell
-// O-grid: width 6 and 1024 cells 945 / 441 / 2152; width 16 and 2048 cells
-// 974 / 607 / 2030: narrow ranges keep a level to one round of the compute waves.
-constexpr int SW_RMAX = 1024, SW_WIDTH = 6;
+// Most cells of a range, and cells per level it may hold.  Narrow ranges keep a
+// level to one round of the compute waves; wide ones spare the chain handovers
+// between ranges (~2 us), which pays where it crosses many: at 128 or more
+// cells a level and at least as many levels as a level has cells (a front that is a
+// line, not a surface).  us per step, 6 and 1024 / 16 and 2048: O-grids of 120,832
+// cells and 747 levels 2240 / 2116, 168,000 and 879 2845 / 2704, 46,080 and 435
+// 1315 / 1329, 15,360 and 247 790 / 1010; 150,000 quads and 799 1145 / 1068; 120,000
+// triangles and 400 624 / 573; 30,720 quads and 367 497 / 817; 120,000 hexes and 148
+// 597 / 803; 46,080 tets and 65 207 / 283.
+struct RangeShape { int cells, width; };
+inline RangeShape range_shape(int C, int nlev) {
+    const int per = C / nlev;
+    return per >= 128 && nlev >= per ? RangeShape{2048, 16} : RangeShape{1024, 6};
+}
 
 // Shapes per solver: NS 5 increments per cell, 16 lanes per cell; SA 1 and 1.
 // CH cells per loader step, ring of 4 steps.
@@ -625,7 +634,8 @@ static bool use_pipeline(int C, int nlev) { return nlev > 8 && C / nlev < 3000; 
 int sweep_build(ofx_ctx* c, const std::vector<int>& off, const std::vector<int>& nb, const std::vector<int>& id,
                 const std::vector<int>& lev, const std::vector<int>& levU) {
     const int C = c->m.C;
-    if (!use_pipeline(C, std::max(c->m.nLevLo, c->m.nLevUp)) || c->m.maxFacesPerCell > 16) return 0;
+    const int nlev = std::max(c->m.nLevLo, c->m.nLevUp);
+    if (!use_pipeline(C, nlev) || c->m.maxFacesPerCell > 16) return 0;
     std::vector<int> level[2] = {std::vector<int>(C), std::vector<int>(C)};  // by storage cell
     for (int sc = 0; sc < C; ++sc) { level[0][sc] = lev[id[sc]]; level[1][sc] = levU[id[sc]]; }
     // dependencies per cell in either direction, which size the ring
@@ -641,10 +651,11 @@ int sweep_build(ofx_ctx* c, const std::vector<int>& off, const std::vector<int>&
     // the largest ranges whose increments, groups and ring fit in LDS
     SweepPlan P[2];
     SweepGroups G[2][2];  // [direction][solver]
+    const RangeShape shape = range_shape(C, nlev);
     for (int k = 0; k < 2; ++k) {
         bool fits = false;
-        for (int R = SW_RMAX; R >= SW_RMIN && !fits; R = R * 3 / 4) {
-            if (!build_sweep_plan(C, off, nb, id, level[k], k == 1, R, SW_WIDTH, P[k])) return 0;
+        for (int R = shape.cells; R >= SW_RMIN && !fits; R = R * 3 / 4) {
+            if (!build_sweep_plan(C, off, nb, id, level[k], k == 1, R, shape.width, P[k])) return 0;
             G[k][0] = sweep_groups(P[k], Shape<5>::CPG, Shape<5>::NW);
             G[k][1] = sweep_groups(P[k], Shape<1>::CPG, Shape<1>::NW);
             fits = Shape<5>::lds(P[k], G[k][0].max, NE) <= (size_t)SW_LDS &&
