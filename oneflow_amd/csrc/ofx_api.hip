@@ -23,6 +23,7 @@ int alloc_bytes(ofx_ctx* c, void** p, size_t bytes) {
     if (bytes == 0) bytes = 8;
     hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess) {
+        (void)hipGetLastError();  // reported here: the next call does not see it
         set_error(std::string("hipMalloc(") + std::to_string(bytes) + "): " + hipGetErrorString(e));
         return OFX_ENOMEM;
     }

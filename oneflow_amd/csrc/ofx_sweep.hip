@@ -633,6 +633,7 @@ static bool use_pipeline(int C, int nlev) { return nlev > 8 && C / nlev < 3000; 
 // id of each storage cell; lev, levU: levels by grid id.
 int sweep_build(ofx_ctx* c, const std::vector<int>& off, const std::vector<int>& nb, const std::vector<int>& id,
                 const std::vector<int>& lev, const std::vector<int>& levU) {
+    sweep_free(c);  // of a mesh whose upload failed later on
     const int C = c->m.C;
     const int nlev = std::max(c->m.nLevLo, c->m.nLevUp);
     if (!use_pipeline(C, nlev) || c->m.maxFacesPerCell > 16) return 0;

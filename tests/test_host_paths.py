@@ -1,0 +1,109 @@
+"""Host side of libofx.so without a GPU: failed allocations, retries, and the
+order of what is launched, on a stand-in for the HIP runtime (fake_hip.cpp;
+kernels do not run).  Each scenario runs in a process of its own, which loads
+the stand-in before the library."""
+import ctypes
+import shutil
+import subprocess
+import sys
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+HERE = Path(__file__).resolve().parent
+if str(HERE.parent) not in sys.path:
+    sys.path.insert(0, str(HERE.parent))
+
+SCENARIOS = {}
+
+
+def scenario(f):
+    SCENARIOS[f.__name__] = f
+    return f
+
+
+# ---- what the scenarios share
+
+def mesh(name):
+    from oneflow_amd import meshgen
+    if name == "chain":  # one cell per level: pipelined sweeps
+        return meshgen.box2d(300, 1)
+    g = meshgen.box2d(40, 30)  # coloured: a launch per level
+    return meshgen.renumber(g, meshgen.multicolor_order(g))
+
+
+def config(**kw):
+    from oneflow_amd.config import CaseConfig
+    return CaseConfig(**{**dict(dim=2, ischeme=1, ilim=-1, vismodel=3, mach_ref=0.5, reynolds=1e4), **kw})
+
+
+def upload(L, h, g):
+    """The return code of a mesh upload."""
+    from oneflow_amd.solver import _dp, _ip
+    x, y, z = (np.ascontiguousarray(a, np.float64) for a in (g.x, g.y, g.z))
+    n, f, lc, rc, bc = (np.ascontiguousarray(a, np.int32) for a in (g.face_node_count, g.face_nodes, g.lc, g.rc, g.bc_type))
+    return L.ofx_mesh_upload(h, g.dim, g.n_nodes, _dp(x), _dp(y), _dp(z), g.n_faces, g.n_cells, g.n_bfaces, _ip(n),
+                             _ip(f), _ip(lc), _ip(rc), _ip(bc))
+
+
+def context(fake):
+    from oneflow_amd.solver import load_library
+    L, h = load_library(), ctypes.c_void_p()
+    assert L.ofx_ctx_create(ctypes.byref(h), 0) == 0
+    return L, h
+
+
+def lines(fake, word):
+    return [s for s in fake.fake_log().decode().splitlines() if s.startswith(word)]
+
+
+def sweep_kernels(fake, L, h):
+    """Kernels of one NS and one SA sweep pair."""
+    c = config().to_c()
+    assert L.ofx_config_set(h, ctypes.byref(c)) == 0
+    fake.fake_clear()
+    assert L.ofx_lusgs_ns(h) == 0 and L.ofx_lusgs_sa(h) == 0
+    return lines(fake, "launch")
+
+
+# ---- scenarios
+
+@scenario
+def retried_upload(fake):
+    """An upload that fails after the sweeps' schedule is built, then another
+    mesh: its sweeps are its own."""
+    L, h = context(fake)
+    assert upload(L, h, mesh("chain")) == 0
+    n = len(lines(fake, "hipMalloc"))
+    assert any("k_sweep_pipe" in k for k in sweep_kernels(fake, L, h))
+    for other in ("coloured", "chain"):
+        for k in range(n - 3, n + 1):  # the upload's last allocations
+            L, h = context(fake)
+            fake.fake_fail(b"hipMalloc", k)
+            if upload(L, h, mesh("chain")) == 0:
+                continue
+            assert upload(L, h, mesh(other)) == 0
+            piped = [s for s in sweep_kernels(fake, L, h) if "k_sweep_pipe" in s]
+            assert bool(piped) == (other == "chain"), (other, k, piped)
+
+
+@pytest.mark.parametrize("name", list(SCENARIOS))
+def test_host_path(name, tmp_path):
+    if not shutil.which("g++"):
+        pytest.skip("g++ not available")
+    so = tmp_path / "libfake_hip.so"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-pthread", str(HERE / "fake_hip.cpp"), "-o", str(so)],
+                   check=True)
+    r = subprocess.run([sys.executable, str(HERE / "test_host_paths.py"), str(so), name], capture_output=True, text=True,
+                       timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+if __name__ == "__main__":
+    lib = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)  # before libofx.so: its symbols come first
+    lib.fake_log.restype = ctypes.c_char_p
+    lib.fake_held.restype = ctypes.c_size_t
+    lib.fake_capacity.argtypes = [ctypes.c_size_t]
+    lib.fake_cost.argtypes = [ctypes.c_char_p, ctypes.c_double]
+    SCENARIOS[sys.argv[2]](lib)
