@@ -22,6 +22,12 @@ void set_error(const std::string& msg) { g_err = msg; }
 int alloc_bytes(ofx_ctx* c, void** p, size_t bytes) {
     if (bytes == 0) bytes = 8;
     hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess && c->sweep) {  // the pipelined sweeps' memory goes first
+        (void)hipGetLastError();
+        sweep_free(c);
+        ++c->gen;  // graphs recorded with them are recorded again
+        e = hipMalloc(p, bytes);
+    }
     if (e != hipSuccess) {
         (void)hipGetLastError();  // reported here: the next call does not see it
         set_error(std::string("hipMalloc(") + std::to_string(bytes) + "): " + hipGetErrorString(e));
@@ -260,8 +266,10 @@ int ofx_mesh_upload(ofx_ctx* c, int dim, int nNodes, const double* x, const doub
     OFX_HIP(hipSetDevice(c->device));
     c->m.dim = dim; c->m.nNodes = nNodes; c->m.C = nCells; c->m.F = nFaces; c->m.B = nBFaces;
     c->m.T = nCells + nBFaces;
-    OFX_TRY(mesh_build(c, x, y, z, faceNodeCount, faceNodes, lc, rc, bcType));
+    MeshLists lists;
+    OFX_TRY(mesh_build(c, x, y, z, faceNodeCount, faceNodes, lc, rc, bcType, lists));
     OFX_TRY(alloc_fields(c));
+    OFX_TRY(sweep_build(c, lists));
     OFX_HIP(hipStreamSynchronize(c->stream));
     c->has_mesh = true;
     ++c->gen;

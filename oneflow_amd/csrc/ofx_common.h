@@ -190,6 +190,13 @@ struct DevFields {
 
 struct SweepSet;  // schedule of the pipelined LU-SGS sweeps (ofx_sweep.hip)
 
+// A mesh's cell lists, which the sweeps' schedule is built from: faces per storage cell
+// (CSR), each entry's neighbour (>= C: ghost), grid id of a storage cell, and
+// dependency level of either sweep by grid id.
+struct MeshLists {
+    std::vector<int> off, nb, id, lev, levU;
+};
+
 }  // namespace ofx
 
 struct ofx_ctx {
@@ -268,6 +275,7 @@ inline int face_tile(int set, int F) { return set ? set : F < 2 * 256 * 256 ? 64
     do {                                                                           \
         hipError_t e_ = (call);                                                    \
         if (e_ != hipSuccess) {                                                    \
+            (void)hipGetLastError(); /* reported here: the next call does not see it */ \
             ofx::set_error(std::string(#call) + ": " + hipGetErrorString(e_));     \
             return OFX_EHIP;                                                       \
         }                                                                          \
@@ -694,7 +702,7 @@ int upload(ofx_ctx* c, void* dst, const void* src, size_t bytes);
 
 // Kernel launch wrappers (defined in the .hip files)
 int mesh_build(ofx_ctx* c, const double* x, const double* y, const double* z, const int* fnc,
-               const int* fnn, const int* lc, const int* rc, const int* bct);
+               const int* fnn, const int* lc, const int* rc, const int* bct, MeshLists& lists);
 int ns_boundary(ofx_ctx* c);
 int sa_boundary(ofx_ctx* c);
 int ns_timestep(ofx_ctx* c, int iter);
@@ -704,8 +712,7 @@ int step_launch(ofx_ctx* c, int iter);
 int sa_residual(ofx_ctx* c);
 int sa_residual_parts(ofx_ctx* c, unsigned parts);  // bits: gradient, face terms, cell terms
 int ns_lusgs(ofx_ctx* c, int lo_first = 0, bool flag = false);
-int sweep_build(ofx_ctx* c, const std::vector<int>& off, const std::vector<int>& nb, const std::vector<int>& id,
-                const std::vector<int>& lev, const std::vector<int>& levU);
+int sweep_build(ofx_ctx* c, const MeshLists& lists);
 void sweep_free(ofx_ctx* c);
 int pipelined_lusgs_ns(ofx_ctx* c);
 int pipelined_lusgs_sa(ofx_ctx* c);

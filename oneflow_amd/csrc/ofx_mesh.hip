@@ -512,7 +512,7 @@ static void spatial_order(int dim, int C, int F, int B, const double* x, const d
 }
 
 int mesh_build(ofx_ctx* c, const double* x, const double* y, const double* z, const int* fnc,
-               const int* fnn, const int* lcIn, const int* rcIn, const int* bct) {
+               const int* fnn, const int* lcIn, const int* rcIn, const int* bct, MeshLists& lists) {
     DevMesh& m = c->m;
     const int C = m.C, F = m.F, B = m.B, T = m.T;
     // face -> node CSR, orientation fix (codes/geometry/src/UnsGrid.cpp:160-170), NormalizeBc
@@ -755,11 +755,11 @@ int mesh_build(ofx_ctx* c, const double* x, const double* y, const double* z, co
     }
     k_face_vis_static<<<(F + TB - 1) / TB, TB, 0, c->stream>>>(m);
     OFX_HIP(hipGetLastError());
-    OFX_TRY(sweep_build(c, off, c2n, cinv, lev, levU));
     // the wall distance is computed on first use (ensure_dist): a mesh that
     // is declared as several zones next searches each zone's walls only
     c->dist_valid = false;
     OFX_HIP(hipStreamSynchronize(c->stream));
+    lists = {std::move(off), std::move(c2n), std::move(cinv), std::move(lev), std::move(levU)};
     return 0;
 }
 

@@ -46,6 +46,7 @@
 #include <algorithm>
 #include <memory>
 #include <new>
+#include <vector>
 
 #include "ofx_lusgs.h"
 #include "ofx_sweep.h"
@@ -120,6 +121,12 @@ struct SweepSet {
     int* ticket = nullptr;
     int NE = 0;  // records per stream cell, both directions
     size_t lds[2][2] = {{0, 0}, {0, 0}};  // [solver][direction]
+    hipStream_t stream = nullptr;
+    std::vector<void*> allocs;
+    ~SweepSet() {
+        if (!allocs.empty()) (void)hipStreamSynchronize(stream);
+        for (void* p : allocs) (void)hipFree(p);
+    }
 };
 
 namespace {
@@ -628,17 +635,25 @@ int pipelined_lusgs_sa(ofx_ctx* c) {
 // few levels stay with their launches (the first is fused into the residual).
 static bool use_pipeline(int C, int nlev) { return nlev > 8 && C / nlev < 3000; }
 
-// Build the pipelined schedule of a mesh that profits from it (at the mesh
-// upload; c->sweep stays empty otherwise and the level kernels run).  id: grid
-// id of each storage cell; lev, levU: levels by grid id.
-int sweep_build(ofx_ctx* c, const std::vector<int>& off, const std::vector<int>& nb, const std::vector<int>& id,
-                const std::vector<int>& lev, const std::vector<int>& levU) {
-    sweep_free(c);  // of a mesh whose upload failed later on
+// Device memory of the schedule; OFX_ENOMEM leaves no error behind.
+static int sweep_alloc(ofx_ctx* c, SweepSet& s, void** p, size_t bytes) {
+    s.allocs.push_back(nullptr);
+    if (hipMalloc(p, std::max<size_t>(bytes, 8)) != hipSuccess) {
+        (void)hipGetLastError();
+        return OFX_ENOMEM;
+    }
+    s.allocs.back() = *p;
+    OFX_HIP(hipMemsetAsync(*p, 0, std::max<size_t>(bytes, 8), c->stream));
+    return 0;
+}
+
+static int build_set(ofx_ctx* c, const MeshLists& lists) {
+    const std::vector<int>&off = lists.off, &nb = lists.nb, &id = lists.id;
     const int C = c->m.C;
     const int nlev = std::max(c->m.nLevLo, c->m.nLevUp);
     if (!use_pipeline(C, nlev) || c->m.maxFacesPerCell > 16) return 0;
     std::vector<int> level[2] = {std::vector<int>(C), std::vector<int>(C)};  // by storage cell
-    for (int sc = 0; sc < C; ++sc) { level[0][sc] = lev[id[sc]]; level[1][sc] = levU[id[sc]]; }
+    for (int sc = 0; sc < C; ++sc) { level[0][sc] = lists.lev[id[sc]]; level[1][sc] = lists.levU[id[sc]]; }
     // dependencies per cell in either direction, which size the ring
     int ne = 1;
     for (int sc = 0; sc < C; ++sc) {
@@ -671,9 +686,10 @@ int sweep_build(ofx_ctx* c, const std::vector<int>& off, const std::vector<int>&
                     lds_limit<1, 2>() && lds_limit<1, 3>() && lds_limit<1, 4>() && lds_limit<1, SW_MAXNE>();
     if (!ok) return 0;
     std::unique_ptr<SweepSet> s(new (std::nothrow) SweepSet());
-    if (!s) { set_error("out of host memory"); return OFX_ENOMEM; }
+    if (!s) return OFX_ENOMEM;
     s->NE = NE;
-    auto A = [&](void** p, size_t bytes) { return alloc_bytes(c, p, bytes); };
+    s->stream = c->stream;
+    auto A = [&](void** p, size_t bytes) { return sweep_alloc(c, *s, p, bytes); };
     for (int k = 0; k < 2; ++k) {
         SweepDev& d = s->d[k];
         const SweepPlan& p = P[k];
@@ -686,7 +702,7 @@ int sweep_build(ofx_ctx* c, const std::vector<int>& off, const std::vector<int>&
         OFX_TRY(A((void**)&d.exch[0], sizeof(double) * 5 * (size_t)std::max(1, p.nX)));
         OFX_TRY(A((void**)&d.exch[1], sizeof(double) * (size_t)std::max(1, p.nX)));
         auto put = [&](void** dst, const void* src, size_t bytes) -> int {
-            OFX_TRY(A(dst, std::max<size_t>(bytes, 8)));
+            OFX_TRY(A(dst, bytes));
             return upload(c, *dst, src, bytes);
         };
         OFX_TRY(put((void**)&d.posOf, p.posOf.data(), sizeof(int) * p.posOf.size()));
@@ -707,6 +723,22 @@ int sweep_build(ofx_ctx* c, const std::vector<int>& off, const std::vector<int>&
     OFX_TRY(A((void**)&s->ticket, 2 * sizeof(int)));
     c->sweep = s.release();
     return 0;
+}
+
+// Build the pipelined schedule of a mesh that profits from it (at the mesh
+// upload, once everything else is allocated; c->sweep stays empty otherwise and
+// the level kernels run).  Its streams take 0.7 to 1.9 KB per cell (two to six
+// dependencies); a mesh that leaves no memory for them is swept level by level,
+// and they are given back when a later allocation needs the room (alloc_bytes).
+int sweep_build(ofx_ctx* c, const MeshLists& lists) {
+    sweep_free(c);  // of a mesh whose upload failed later on
+    int rc;
+    try {
+        rc = build_set(c, lists);
+    } catch (const std::bad_alloc&) {
+        rc = OFX_ENOMEM;
+    }
+    return rc == OFX_ENOMEM ? 0 : rc;
 }
 
 void sweep_free(ofx_ctx* c) {

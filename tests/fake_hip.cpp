@@ -57,6 +57,7 @@ int take(void** p, size_t n, const char* fn) {
     return 0;
 }
 int give(void* p) {
+    if (!p) return 0;
     std::lock_guard<std::recursive_mutex> l(mu);
     auto it = live.find(static_cast<char*>(p));
     if (it == live.end()) return last_error = INVALID;

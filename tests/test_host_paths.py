@@ -75,17 +75,62 @@ def retried_upload(fake):
     mesh: its sweeps are its own."""
     L, h = context(fake)
     assert upload(L, h, mesh("chain")) == 0
-    n = len(lines(fake, "hipMalloc"))
+    calls = {b"hipMalloc": len(lines(fake, "hipMalloc")), b"hipStreamSynchronize": len(lines(fake, "sync"))}
     assert any("k_sweep_pipe" in k for k in sweep_kernels(fake, L, h))
     for other in ("coloured", "chain"):
-        for k in range(n - 3, n + 1):  # the upload's last allocations
+        for fn, k in [(fn, n - i) for fn, n in calls.items() for i in range(4)]:  # the upload's last calls
             L, h = context(fake)
-            fake.fake_fail(b"hipMalloc", k)
+            fake.fake_fail(fn, k)
             if upload(L, h, mesh("chain")) == 0:
                 continue
             assert upload(L, h, mesh(other)) == 0
             piped = [s for s in sweep_kernels(fake, L, h) if "k_sweep_pipe" in s]
-            assert bool(piped) == (other == "chain"), (other, k, piped)
+            assert bool(piped) == (other == "chain"), (other, fn, k, piped)
+
+
+@scenario
+def sweeps_without_memory(fake):
+    """A mesh that fits without the pipelined sweeps' streams is accepted and swept
+    level by level, whichever of their allocations fails; streams that are there
+    give way to a later allocation."""
+    L, h = context(fake)
+    assert upload(L, h, mesh("chain")) == 0
+    n, full = len(lines(fake, "hipMalloc")), fake.fake_held()
+    L.ofx_ctx_destroy(h)
+    assert fake.fake_held() == 0
+    fake.fake_capacity(full - 1)
+    L, h = context(fake)
+    assert upload(L, h, mesh("chain")) == 0, L.ofx_last_error()
+    need = fake.fake_held()  # without the streams
+    assert need < full
+    kernels = sweep_kernels(fake, L, h)
+    assert kernels and not any("k_sweep_pipe" in k for k in kernels)
+    L.ofx_ctx_destroy(h)
+    fake.fake_capacity(need)
+    L, h = context(fake)
+    assert upload(L, h, mesh("chain")) == 0, L.ofx_last_error()
+    L.ofx_ctx_destroy(h)
+    fake.fake_capacity(2 * full)
+    piped = []
+    for k in range(1, n + 1):
+        L, h = context(fake)
+        fake.fake_fail(b"hipMalloc", k)
+        if upload(L, h, mesh("chain")) == 0:
+            piped.append(any("k_sweep_pipe" in s for s in sweep_kernels(fake, L, h)))
+        fake.fake_fail(b"hipMalloc", 0)
+        L.ofx_ctx_destroy(h)
+        assert fake.fake_held() == 0
+    assert len(piped) > 10 and not any(piped)
+    # zones declared later: their arrays take the streams' place, and the sweeps go level by level
+    L, h = context(fake)
+    assert upload(L, h, mesh("chain")) == 0
+    assert any("k_sweep_pipe" in k for k in sweep_kernels(fake, L, h))
+    fake.fake_capacity(full)
+    cfg, start = config().to_c(), (ctypes.c_int * 2)
+    assert L.ofx_zones_set(h, 1, start(0, 300), start(0, 602), ctypes.byref(cfg)) == 0, L.ofx_last_error()
+    assert not any("k_sweep_pipe" in k for k in sweep_kernels(fake, L, h))
+    L.ofx_ctx_destroy(h)
+    assert fake.fake_held() == 0
 
 
 @pytest.mark.parametrize("name", list(SCENARIOS))
