@@ -81,6 +81,17 @@ inline SweepGroups sweep_groups(const SweepPlan& P, int cpg, int nw) {
     return G;
 }
 
+// Polls after which a wave's waits over a whole range give up, the guard against a
+// fault of the schedule (its order by itself ends every wait).  A wait may
+// rightly last as long as the sweep, at worst every range after the one before it:
+// 1 us per group and 2 us per range (measured 0.3 to 1 and 2).  A poll is at least an
+// LDS round trip of 64 cycles, 25 ns; ten times the polls that fit, and 4 million for
+// kernels beside this one.  0: more than a counter holds (a chain of seconds).
+inline int sweep_polls(const SweepPlan& P, const SweepGroups& G) {
+    const double us = (double)G.g.size() + 2.0 * P.W, n = 10.0 * us / 0.025 + (1 << 22);
+    return n < 2e9 ? (int)n : 0;
+}
+
 constexpr int SW_RMIN = 64;  // a range takes at least this many cells
 
 // off / nb: faces of each storage cell (CSR) and the neighbour of each (>= C:

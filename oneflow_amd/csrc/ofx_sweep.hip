@@ -28,9 +28,9 @@
 // value itself.  Workgroups take their range by a ticket drawn when they
 // start, so a range's predecessors have always started before it: the first
 // unfinished range never waits, whatever the dispatch order or the number of
-// resident workgroups, and every wait ends.  As a guard each wait also gives
-// up after SPIN_MAX polls and leaves a NaN increment, which the residual
-// norms report.
+// resident workgroups, and every wait ends.  As a guard a wave's waits also give
+// up after sweep_polls polls, many times the longest chain, and leave a NaN
+// increment, which the residual norms report.
 //
 // The arithmetic is the level kernels' operation for operation.
 //
@@ -59,7 +59,6 @@ typedef int sw_int4 __attribute__((ext_vector_type(4)));
 typedef int sw_int2 __attribute__((ext_vector_type(2)));
 
 constexpr unsigned long long SW_EMPTY = 0x7FF0A5A5DEADBEEFull;  // a signalling NaN: never a result of arithmetic
-constexpr int SPIN_MAX = 1 << 22;
 constexpr int SW_LDS = 160 * 1024;
 // Most cells of a range, and cells per level it may hold.  Narrow ranges keep a
 // level to one round of the compute waves; wide ones spare the chain handovers
@@ -114,6 +113,7 @@ struct SweepDev {
     SweepMeta* meta = nullptr;
     int* slot = nullptr;
     int C = 0, R = 0, W = 0, NE = 0, nX = 0, maxHalo = 0;
+    int polls[2] = {0, 0};  // NS, SA: sweep_polls
 };
 
 struct SweepSet {
@@ -307,7 +307,7 @@ struct Group {
 // the upper sweep's stream.  VISC: the NS face terms hold a viscous radius.
 template <int NEQ, int NE, bool UPPER, bool VISC>
 __global__ void __launch_bounds__(Shape<NEQ>::WAVES * 64) k_sweep_pipe(SweepDev s, char* stream2, double* dq, int T,
-                                                                      double gama, int* ticket) {
+                                                                      double gama, int polls, int* ticket) {
     using S = Shape<NEQ>;
     constexpr int SV = NEQ == 5 ? 0 : 1;
     constexpr int NW = S::NW, NL = S::NL, CH = S::CH, NCH = S::NCH, RC = S::RC, IST = S::IST;
@@ -348,19 +348,19 @@ __global__ void __launch_bounds__(Shape<NEQ>::WAVES * 64) k_sweep_pipe(SweepDev 
     if (w > NW) {  // ---- loaders: chunk c = CH cells of the stream, contiguous
         constexpr int U = CH * st / 1024;  // 16-byte vectors per lane
         static_assert(CH * st % 1024 == 0, "whole vectors");
-        int spin = 0;  // (past SPIN_MAX nothing waits any more)
+        int spin = 0;  // (past `polls` nothing waits any more)
         for (int c = w - NW - 1; c * CH < n; c += NL) {
             const sw_int4* a = reinterpret_cast<const sw_int4*>(src + (size_t)c * CH * st);
             sw_int4 v[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) v[u] = a[u * 64 + lane];
             // the chunk's ring slot is free once chunk c - NCH is consumed
-            while (read_counters().done < (c - NCH + 1) * CH && ++spin < SPIN_MAX) __builtin_amdgcn_s_sleep(1);
+            while (read_counters().done < (c - NCH + 1) * CH && ++spin < polls) __builtin_amdgcn_s_sleep(1);
             sw_int4* o = reinterpret_cast<sw_int4*>(ring + (size_t)(c % NCH) * CH * st);
 #pragma unroll
             for (int u = 0; u < U; ++u) o[u * 64 + lane] = v[u];
             SW_ORDER();
-            while (read_counters().ring < c * CH && ++spin < SPIN_MAX) {}  // chunks are published in order
+            while (read_counters().ring < c * CH && ++spin < polls) {}  // chunks are published in order
             if (lane == 0) ctr[4] = (uint16_t)((c + 1) * CH);
             SW_ORDER();
         }
@@ -368,11 +368,12 @@ __global__ void __launch_bounds__(Shape<NEQ>::WAVES * 64) k_sweep_pipe(SweepDev 
     }
     if (w == NW) {  // ---- halo receiver: one lane per item, published in order
         const int h0 = s.haloOff[g], nh = s.haloOff[g + 1] - h0;
+        int spin = 0;
         for (int b = 0; b < nh; b += 64) {
             const int it = b + lane;
             bool wait = it < nh;
             const unsigned long long* a = exch + (size_t)(wait ? s.haloX[h0 + it] : 0) * NEQ;
-            int spin = 0, seen = b;
+            int seen = b;
             while (true) {
                 if (wait) {
                     unsigned long long v[NEQ];
@@ -382,7 +383,7 @@ __global__ void __launch_bounds__(Shape<NEQ>::WAVES * 64) k_sweep_pipe(SweepDev 
                         v[e] = __hip_atomic_load(a + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
                     for (int e = 0; e < NEQ; ++e) ok = ok && v[e] != SW_EMPTY;
-                    if (ok || spin > SPIN_MAX) {
+                    if (ok || spin > polls) {
                         for (int e = 0; e < NEQ; ++e)
                             inc[(size_t)(s.R + it) * IST + e] =
                                 ok ? __longlong_as_double((long long)v[e]) : __builtin_nan("");
@@ -448,7 +449,7 @@ __global__ void __launch_bounds__(Shape<NEQ>::WAVES * 64) k_sweep_pipe(SweepDev 
     // into N meanwhile; `loaded` then tells whether the ring held them.
     auto step = [&](Grp& G, Grp& N) {
         if (__builtin_expect(!loaded, 0)) {
-            while (read_counters().ring < pos + cnt && ++spin < SPIN_MAX) {}
+            while (read_counters().ring < pos + cnt && ++spin < polls) {}
             load(G);
         }
         const int nd = G.link & 7;
@@ -473,7 +474,7 @@ __global__ void __launch_bounds__(Shape<NEQ>::WAVES * 64) k_sweep_pipe(SweepDev 
         const Ctr k = counters(kv);
         if (k.done < start || k.halo < need) {
             Ctr q;
-            do { q = read_counters(); } while ((q.done < start || q.halo < need) && ++spin < SPIN_MAX);
+            do { q = read_counters(); } while ((q.done < start || q.halo < need) && ++spin < polls);
             increments();
             SW_ORDER();
         }
@@ -528,7 +529,7 @@ __global__ void __launch_bounds__(Shape<NEQ>::WAVES * 64) k_sweep_pipe(SweepDev 
         double x = ofxm::div_by(num, G.rad, G.y);
         if (__builtin_expect(!__all(ofxm::div_by_ok(num, G.y)), 0)) x = num / G.rad;
         if (UPPER) x = G.val + x;
-        if (lead && c < ncell && spin < SPIN_MAX) {
+        if (lead && c < ncell && spin < polls) {
             inc[(here + c) * IST + e] = x;
             if (UPPER) dq[(size_t)e * T + G.dest] = x;
             else reinterpret_cast<double*>(stream2 + (size_t)G.dest * st)[e] = x;
@@ -550,7 +551,7 @@ __global__ void __launch_bounds__(Shape<NEQ>::WAVES * 64) k_sweep_pipe(SweepDev 
         if (i >= i1) break;
         step(GB, GA);
     }
-    if (lane == 0 && spin >= SPIN_MAX) {  // a wait was given up: a NaN increment reports it
+    if (lane == 0 && spin >= polls) {  // a wait was given up: a NaN increment reports it
         if (UPPER) dq[0] = __builtin_nan("");
         else *reinterpret_cast<double*>(stream2) = __builtin_nan("");
     }
@@ -561,9 +562,9 @@ int sweep_pair(ofx_ctx* c, SweepSet& s, double* dq) {
     using S = Shape<NEQ>;
     constexpr int sv = NEQ == 5 ? 0 : 1;
     k_sweep_pipe<NEQ, NE, false, VISC><<<s.d[0].W, S::WAVES * 64, s.lds[sv][0], c->stream>>>(
-        s.d[0], s.d[1].stream[sv], dq, c->m.T, c->k.gama, s.ticket);
+        s.d[0], s.d[1].stream[sv], dq, c->m.T, c->k.gama, s.d[0].polls[sv], s.ticket);
     k_sweep_pipe<NEQ, NE, true, VISC><<<s.d[1].W, S::WAVES * 64, s.lds[sv][1], c->stream>>>(
-        s.d[1], nullptr, dq, c->m.T, c->k.gama, s.ticket + 1);
+        s.d[1], nullptr, dq, c->m.T, c->k.gama, s.d[1].polls[sv], s.ticket + 1);
     OFX_HIP(hipGetLastError());
     return 0;
 }
@@ -677,7 +678,7 @@ static int build_set(ofx_ctx* c, const MeshLists& lists) {
             fits = Shape<5>::lds(P[k], G[k][0].max, NE) <= (size_t)SW_LDS &&
                    Shape<1>::lds(P[k], G[k][1].max, NE) <= (size_t)SW_LDS;
         }
-        if (!fits) return 0;
+        if (!fits || !sweep_polls(P[k], G[k][0]) || !sweep_polls(P[k], G[k][1])) return 0;
     }
     for (int k = 0; k < 2; ++k)
         for (int p = 0; p < C; ++p) P[k].meta[p].pos2 = P[1 - k].posOf[P[k].meta[p].cell];
@@ -711,6 +712,7 @@ static int build_set(ofx_ctx* c, const MeshLists& lists) {
             OFX_TRY(put((void**)&d.grpOff[v], G[k][v].off.data(), sizeof(int) * G[k][v].off.size()));
             OFX_TRY(put((void**)&d.grp[v], G[k][v].g.data(), sizeof(SweepGroup) * G[k][v].g.size()));
             d.maxGrp[v] = G[k][v].max;
+            d.polls[v] = sweep_polls(p, G[k][v]);
         }
         OFX_TRY(put((void**)&d.haloOff, p.haloOff.data(), sizeof(int) * p.haloOff.size()));
         OFX_TRY(put((void**)&d.haloX, p.haloX.data(), sizeof(int) * p.haloX.size()));

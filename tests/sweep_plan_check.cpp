@@ -6,7 +6,9 @@
 // compute waves must cover each range once.  Then the division by a stored
 // reciprocal (ofx_math.h) against the processor's: the same quotient wherever
 // div_by_ok holds, dense, sparse and extreme significands, products of the
-// divisor and their neighbours among the dividends.
+// divisor and their neighbours among the dividends.  Last the waits' guard:
+// on rows numbered back and forth (as many levels as cells, the longest chain a
+// grid can have) a wave may poll several times as long as the sweep takes.
 // Prints "ok <plans>" or the first failure.
 #include "../oneflow_amd/csrc/ofx_sweep.h"
 
@@ -155,6 +157,36 @@ int main() {
         ofxm::div_reciprocal(NAN) != 0.0 || ofxm::div_by_ok(INFINITY, 1.0) || ofxm::div_by_ok(NAN, 1.0) ||
         ofxm::div_by_ok(1e-200, 1.0) || ofxm::div_by_ok(1.0, 0.0))
         return fail("domain", 0, 0);
+    for (int n : {30, 300, 1000, 1700}) {
+        const int C = n * n;
+        std::vector<int> off(C + 1, 0), nb, id(C), level[2] = {std::vector<int>(C), std::vector<int>(C)};
+        for (int c = 0; c < C; ++c) {  // storage cell (i, j)
+            const int i = c % n, j = c / n;
+            id[c] = j * n + (j & 1 ? n - 1 - i : i);
+            if (i > 0) nb.push_back(c - 1);
+            if (i + 1 < n) nb.push_back(c + 1);
+            if (j > 0) nb.push_back(c - n);
+            if (j + 1 < n) nb.push_back(c + n);
+            off[c + 1] = (int)nb.size();
+            level[0][c] = id[c];
+            level[1][c] = C - 1 - id[c];
+        }
+        for (int up = 0; up < 2; ++up) {
+            SweepPlan P;
+            if (!build_sweep_plan(C, off, nb, id, level[up], up == 1, 1024, 6, P)) return fail("long chain", n, up);
+            for (int cpg : {4, 64}) {  // NS, SA
+                const double chain_us = 0.46 * C + 2.0 * P.W;  // measured per level and per range
+                const double poll_us = 0.025;                  // one LDS round trip, the least it can be
+                const int polls = sweep_polls(P, sweep_groups(P, cpg, cpg == 4 ? 3 : 2));
+                if (polls < 8 * chain_us / poll_us) return fail("polls", n, polls);
+            }
+        }
+    }
+    {  // more than a counter holds: not swept by the pipeline
+        SweepPlan P;
+        P.W = 6000000;
+        if (sweep_polls(P, SweepGroups()) != 0) return fail("poll limit", 0, 0);
+    }
     std::printf("ok %ld\n", plans);
     return 0;
 }
