@@ -679,6 +679,15 @@ int ofx_set_kernel_variant(ofx_ctx* c, int kernel, int variant) {
     return 0;
 }
 
+// Not in ofx.h: for the test that a given-up wait is never silent.
+int ofx_set_sweep_polls(ofx_ctx* c, int polls) {
+    CHECK_CTX(c);
+    if (polls < 0) { set_error("sweep polls must be >= 0"); return OFX_EINVAL; }
+    c->sweep_polls = polls;
+    ++c->gen;
+    return 0;
+}
+
 int ofx_get_kernel_variant(ofx_ctx* c, int kernel, int* variant) {
     CHECK_CTX(c);
     if (!variant || kernel < 0 || kernel > 6) { set_error("kernel variant: kernel 0..6 and non-null out"); return OFX_EINVAL; }

@@ -215,6 +215,7 @@ struct ofx_ctx {
     ofx::DevMesh m;
     ofx::HostSched sched;
     ofx::SweepSet* sweep = nullptr;  // null: the sweeps run level by level
+    int sweep_polls = 0;             // limit of the pipelined sweeps' waits, 0: the schedule's
     ofx::DevFields d;
     std::vector<void*> allocs;
     double* hsum = nullptr;  // pinned host memory the norm and force kernels write: [6 nz]

@@ -29,8 +29,11 @@
 // start, so a range's predecessors have always started before it: the first
 // unfinished range never waits, whatever the dispatch order or the number of
 // resident workgroups, and every wait ends.  As a guard a wave's waits also give
-// up after sweep_polls polls, many times the longest chain, and leave a NaN
-// increment, which the residual norms report.
+// up after sweep_polls polls, many times the longest chain.  No wave goes on as if
+// it had been served: a loader stops (it overwrites nothing and publishes nothing, so
+// that the compute waves give up in turn), the receiver hands out NaN for what it
+// did not get, and a compute wave leaves NaN increments in the cells that it waited
+// for in vain, which all that depend on them inherit and the residual norms report.
 //
 // The arithmetic is the level kernels' operation for operation.
 //
@@ -348,7 +351,7 @@ __global__ void __launch_bounds__(Shape<NEQ>::WAVES * 64) k_sweep_pipe(SweepDev 
     if (w > NW) {  // ---- loaders: chunk c = CH cells of the stream, contiguous
         constexpr int U = CH * st / 1024;  // 16-byte vectors per lane
         static_assert(CH * st % 1024 == 0, "whole vectors");
-        int spin = 0;  // (past `polls` nothing waits any more)
+        int spin = 0;
         for (int c = w - NW - 1; c * CH < n; c += NL) {
             const sw_int4* a = reinterpret_cast<const sw_int4*>(src + (size_t)c * CH * st);
             sw_int4 v[U];
@@ -356,11 +359,13 @@ __global__ void __launch_bounds__(Shape<NEQ>::WAVES * 64) k_sweep_pipe(SweepDev 
             for (int u = 0; u < U; ++u) v[u] = a[u * 64 + lane];
             // the chunk's ring slot is free once chunk c - NCH is consumed
             while (read_counters().done < (c - NCH + 1) * CH && ++spin < polls) __builtin_amdgcn_s_sleep(1);
+            if (spin >= polls) return;
             sw_int4* o = reinterpret_cast<sw_int4*>(ring + (size_t)(c % NCH) * CH * st);
 #pragma unroll
             for (int u = 0; u < U; ++u) o[u * 64 + lane] = v[u];
             SW_ORDER();
             while (read_counters().ring < c * CH && ++spin < polls) {}  // chunks are published in order
+            if (spin >= polls) return;
             if (lane == 0) ctr[4] = (uint16_t)((c + 1) * CH);
             SW_ORDER();
         }
@@ -383,7 +388,7 @@ __global__ void __launch_bounds__(Shape<NEQ>::WAVES * 64) k_sweep_pipe(SweepDev 
                         v[e] = __hip_atomic_load(a + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
                     for (int e = 0; e < NEQ; ++e) ok = ok && v[e] != SW_EMPTY;
-                    if (ok || spin > polls) {
+                    if (ok || spin >= polls) {
                         for (int e = 0; e < NEQ; ++e)
                             inc[(size_t)(s.R + it) * IST + e] =
                                 ok ? __longlong_as_double((long long)v[e]) : __builtin_nan("");
@@ -451,6 +456,12 @@ __global__ void __launch_bounds__(Shape<NEQ>::WAVES * 64) k_sweep_pipe(SweepDev 
         if (__builtin_expect(!loaded, 0)) {
             while (read_counters().ring < pos + cnt && ++spin < polls) {}
             load(G);
+            if (spin >= polls) {  // given up: what the stores below need comes from memory, the value is NaN
+                G.val = __builtin_nan("");
+                const int* h = reinterpret_cast<const int*>(src + (size_t)(pos + min(c, cnt - 1)) * st + S::META);
+                G.dest = h[0];
+                G.link = h[1] & ~7;
+            }
         }
         const int nd = G.link & 7;
         // The increments, once every cell of the earlier levels and the level's
@@ -475,6 +486,7 @@ __global__ void __launch_bounds__(Shape<NEQ>::WAVES * 64) k_sweep_pipe(SweepDev 
         if (k.done < start || k.halo < need) {
             Ctr q;
             do { q = read_counters(); } while ((q.done < start || q.halo < need) && ++spin < polls);
+            if (spin >= polls) G.val = __builtin_nan("");
             increments();
             SW_ORDER();
         }
@@ -529,7 +541,7 @@ __global__ void __launch_bounds__(Shape<NEQ>::WAVES * 64) k_sweep_pipe(SweepDev 
         double x = ofxm::div_by(num, G.rad, G.y);
         if (__builtin_expect(!__all(ofxm::div_by_ok(num, G.y)), 0)) x = num / G.rad;
         if (UPPER) x = G.val + x;
-        if (lead && c < ncell && spin < polls) {
+        if (lead && c < ncell) {
             inc[(here + c) * IST + e] = x;
             if (UPPER) dq[(size_t)e * T + G.dest] = x;
             else reinterpret_cast<double*>(stream2 + (size_t)G.dest * st)[e] = x;
@@ -551,20 +563,17 @@ __global__ void __launch_bounds__(Shape<NEQ>::WAVES * 64) k_sweep_pipe(SweepDev 
         if (i >= i1) break;
         step(GB, GA);
     }
-    if (lane == 0 && spin >= polls) {  // a wait was given up: a NaN increment reports it
-        if (UPPER) dq[0] = __builtin_nan("");
-        else *reinterpret_cast<double*>(stream2) = __builtin_nan("");
-    }
 }
 
 template <int NEQ, int NE, bool VISC>
 int sweep_pair(ofx_ctx* c, SweepSet& s, double* dq) {
     using S = Shape<NEQ>;
     constexpr int sv = NEQ == 5 ? 0 : 1;
+    const int set = c->sweep_polls;
     k_sweep_pipe<NEQ, NE, false, VISC><<<s.d[0].W, S::WAVES * 64, s.lds[sv][0], c->stream>>>(
-        s.d[0], s.d[1].stream[sv], dq, c->m.T, c->k.gama, s.d[0].polls[sv], s.ticket);
+        s.d[0], s.d[1].stream[sv], dq, c->m.T, c->k.gama, set ? set : s.d[0].polls[sv], s.ticket);
     k_sweep_pipe<NEQ, NE, true, VISC><<<s.d[1].W, S::WAVES * 64, s.lds[sv][1], c->stream>>>(
-        s.d[1], nullptr, dq, c->m.T, c->k.gama, s.d[1].polls[sv], s.ticket + 1);
+        s.d[1], nullptr, dq, c->m.T, c->k.gama, set ? set : s.d[1].polls[sv], s.ticket + 1);
     OFX_HIP(hipGetLastError());
     return 0;
 }
