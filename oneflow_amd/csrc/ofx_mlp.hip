@@ -1190,6 +1190,8 @@ int ofx_mlp_create(ofx_mlp** out, int device, unsigned long long seed) {
     }
     if (!rc) rc = refresh_wt(n);
     if (!rc) rc = refresh_frag(n);
+    // (ofx_mlp_forward_noalloc may read them on any stream next)
+    if (!rc && hipStreamSynchronize(n->stream) != hipSuccess) rc = OFX_EHIP;
     if (rc) {
         ofx_mlp_destroy(n);
         return rc;

@@ -133,6 +133,20 @@ def sweeps_without_memory(fake):
     assert fake.fake_held() == 0
 
 
+@scenario
+def network_is_ready(fake):
+    """Whatever ofx_mlp_create launches on the network's stream is finished when it
+    returns: a forward pass may follow on any other stream."""
+    from oneflow_amd.mlp import Mlp
+    m = Mlp(seed=3)
+    work = [s for s in fake.fake_log().decode().splitlines() if s.split()[0] in ("launch", "copy", "sync")]
+    assert any("k_frag" in s for s in work)
+    streams = {s.split()[1] for s in work}
+    for st in streams:
+        assert [s for s in work if s.split()[1] == st][-1] == "sync " + st, (st, work[-8:])
+    del m
+
+
 @pytest.mark.parametrize("name", list(SCENARIOS))
 def test_host_path(name, tmp_path):
     if not shutil.which("g++"):
