@@ -367,10 +367,12 @@ int ofx_mlp_set_forward_variant(ofx_mlp* net, int variant);
  * capture, serving loops).  x_dev [n][9] and y_dev [n][5] are DEVICE pointers
  * owned by the caller; the work is launched on `stream` (a hipStream_t; NULL:
  * the network's own stream) with no host synchronisation, copy, memset or
- * allocation.  n <= 8192; larger n is rejected (OFX_EINVAL).  Under
- * forward variant 0 the work arrays are one fixed 10.25 MiB device array per
- * GPU, held until the process ends and shared by every call on that GPU, so
- * such calls that overlap on one GPU race; variant 1 needs no work array.  Results equal ofx_mlp_forward's bit for bit. */
+ * allocation.  x_dev and y_dev may overlap.  n <= 8192; larger n is rejected
+ * (OFX_EINVAL).  Under forward variant 0, and where x_dev and y_dev overlap,
+ * the work array is one fixed 10.25 MiB device array per GPU, held until the
+ * process ends and shared by every call on that GPU, so such calls that
+ * overlap in time on one GPU race; otherwise variant 1 needs no work array.
+ * Results equal ofx_mlp_forward's bit for bit. */
 int ofx_mlp_forward_noalloc(ofx_mlp* net, const float* x_dev, int n, float* y_dev, void* stream);
 /* Mean-squared-error loss over the 5 outputs and its gradient with respect to
  * every parameter (same layout as the parameter vector); no update. */

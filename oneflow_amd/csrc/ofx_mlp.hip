@@ -340,6 +340,11 @@ __global__ void k_transpose(const bf16* in, int R, int Cc, bf16* out, int Cp) {
     }
 }
 
+__global__ void k_copy_floats(const float* a, int n, float* b) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) b[i] = a[i];
+}
+
 // Inputs fp32 [n][NIN] -> bf16 [Mp][NIN_P] (zero padded).
 __global__ void k_pack_inputs(const float* x, int n, int Mp, bf16* out) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -956,6 +961,13 @@ int forward_fused(const ofx_mlp* n, hipStream_t st, const float* x, int nsamp, f
     return forward_shape<4, 8, 4, true>(n, st, x, nsamp, y);
 }
 
+// Whether inputs x and outputs y of n samples share memory: the one-kernel pass
+// writes rows while it reads others, and the piped one while others are not uploaded.
+bool overlapping(const float* x, const float* y, int n) {
+    const uintptr_t a = reinterpret_cast<uintptr_t>(x), b = reinterpret_cast<uintptr_t>(y);
+    return a < b + sizeof(float) * (size_t)n * NOUT && b < a + sizeof(float) * (size_t)n * NIN;
+}
+
 // A forward pass of many host samples in pieces: this thread copies a piece's
 // inputs and launches its kernel, a second one copies finished pieces' outputs.
 // Copies of ordinary host memory hold the calling thread (1.2 ms in, 1.2 ms out,
@@ -1263,7 +1275,7 @@ int ofx_mlp_forward(ofx_mlp* n, const float* x, int nsamp, float* y) {
     const size_t cnt = (size_t)nsamp * NOUT;
     if (n->fwd_variant == 1) {
         OFX_TRY(io_reserve(n, nsamp));
-        if (nsamp >= PIPE_MIN) {
+        if (nsamp >= PIPE_MIN && !overlapping(x, y, nsamp)) {
             const int rc = forward_piped(n, x, nsamp, y);
             if (rc != OFX_ESTATE) return rc;
         }
@@ -1292,9 +1304,16 @@ int ofx_mlp_forward_noalloc(ofx_mlp* n, const float* x_dev, int nsamp, float* y_
     }
     OFX_HIP(hipSetDevice(n->device));
     hipStream_t st = stream ? static_cast<hipStream_t>(stream) : n->stream;
-    if (n->fwd_variant == 1) return forward_fused(n, st, x_dev, nsamp, y_dev);
+    if (n->fwd_variant == 1 && !overlapping(x_dev, y_dev, nsamp)) return forward_fused(n, st, x_dev, nsamp, y_dev);
     unsigned char* base = nullptr;
     OFX_TRY(scratch_address(n->device, &base));
+    if (n->fwd_variant == 1) {  // y_dev overwrites inputs: from a copy of them
+        static_assert(sizeof(float) * NOALLOC_MAXN * NIN <= NOALLOC_BYTES, "room for the inputs");
+        float* in = reinterpret_cast<float*>(base);
+        k_copy_floats<<<(nsamp * NIN + 255) / 256, 256, 0, st>>>(x_dev, nsamp * NIN, in);
+        OFX_HIP(hipGetLastError());
+        return forward_fused(n, st, in, nsamp, y_dev);
+    }
     bf16* in = reinterpret_cast<bf16*>(base);
     bf16* act[2] = {reinterpret_cast<bf16*>(base + NOALLOC_IN), reinterpret_cast<bf16*>(base + NOALLOC_IN + NOALLOC_ACT)};
     float* yp = reinterpret_cast<float*>(base + NOALLOC_IN + 2 * NOALLOC_ACT);

@@ -147,6 +147,30 @@ def network_is_ready(fake):
     del m
 
 
+@scenario
+def network_buffers_overlap(fake):
+    """Outputs that overwrite inputs: every input is read before the first output
+    is written, on the host (one upload, then one download) and on the device (the
+    forward kernel reads a copy)."""
+    from oneflow_amd.mlp import NIN, NOUT, Mlp, _fp
+    m, n = Mlp(seed=3), 1 << 19
+    buf = np.zeros((NIN + 2 * NOUT) * n, np.float32)
+    x = buf[NOUT * n: (NOUT + NIN) * n]
+    for at, apart in ((0, True), (1, False), (NOUT * n, False), ((NOUT + NIN) * n - 1, False), ((NOUT + NIN) * n, True)):
+        fake.fake_clear()
+        assert m._L.ofx_mlp_forward(m.h, _fp(x), n, _fp(buf[at:])) == 0
+        assert (len(lines(fake, "copy")) > 2) == apart, at
+    n = 1024
+    x = buf[NOUT * n: (NOUT + NIN) * n]
+    dev = lambda a: ctypes.c_void_p(a.ctypes.data)
+    for at, apart in ((0, True), (1, False), (NOUT * n, False), ((NOUT + NIN) * n - 1, False), ((NOUT + NIN) * n, True)):
+        fake.fake_clear()
+        assert m._L.ofx_mlp_forward_noalloc(m.h, dev(x), n, dev(buf[at:]), None) == 0
+        kernels = lines(fake, "launch")
+        assert len(kernels) == (1 if apart else 2) and "k_mlp_forward" in kernels[-1], (at, kernels)
+    del m
+
+
 @pytest.mark.parametrize("name", list(SCENARIOS))
 def test_host_path(name, tmp_path):
     if not shutil.which("g++"):
