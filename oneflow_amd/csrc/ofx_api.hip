@@ -55,14 +55,13 @@ __global__ void k_fill_field(double* p, long n, double v) {
 static int host_sums(ofx_ctx* c, int nz) {
     if (nz <= c->hsum_n) return 0;
     nz = std::max(nz, 64);  // (one page holds 85)
-    if (c->hsum) (void)hipHostFree(c->hsum);
-    c->hsum = nullptr;
-    c->hsum_n = 0;
     void* p = nullptr;
     if (hipHostMalloc(&p, sizeof(double) * 6 * (size_t)nz, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();  // reported here
         set_error("out of pinned host memory");
         return OFX_ENOMEM;
     }
+    if (c->hsum) (void)hipHostFree(c->hsum);
     c->hsum = static_cast<double*>(p);
     c->hsum_n = nz;
     return 0;
@@ -834,40 +833,47 @@ int ofx_zones_set(ofx_ctx* c, int n, const int* cellStart, const int* bfaceStart
         while (w < m.nWall && wall[w] < fz) ++w;
         zwall[z] = w;
     }
-    c->zkh.resize(n);
-    for (int z = 0; z < n; ++z) c->zkh[z] = zone_consts(cfgs[z]);
-    auto A = [&](void** p, size_t bytes) { return alloc_bytes(c, p, bytes); };
-    OFX_TRY(A((void**)&m.zcell, sizeof(int) * T));
-    OFX_TRY(A((void**)&m.zface, sizeof(int) * F));
-    OFX_TRY(A((void**)&m.zwall, sizeof(int) * (n + 1)));
+    std::vector<ZoneK> zkh(n);
+    for (int z = 0; z < n; ++z) zkh[z] = zone_consts(cfgs[z]);
+    // everything new beside what the context works with, which it keeps if anything fails
+    DevMesh nm = m;
+    DevFields nd = c->d;
+    int* zcells = nullptr;
     ZoneK* zk = nullptr;
+    auto A = [&](void** p, size_t bytes) { return alloc_bytes(c, p, bytes); };
+    OFX_TRY(A((void**)&nm.zcell, sizeof(int) * T));
+    OFX_TRY(A((void**)&nm.zface, sizeof(int) * F));
+    OFX_TRY(A((void**)&nm.zwall, sizeof(int) * (n + 1)));
     OFX_TRY(A((void**)&zk, sizeof(ZoneK) * n));
-    OFX_TRY(upload(c, m.zcell, zcell.data(), sizeof(int) * T));
-    OFX_TRY(upload(c, m.zface, zface.data(), sizeof(int) * F));
-    OFX_TRY(upload(c, m.zwall, zwall.data(), sizeof(int) * (n + 1)));
-    OFX_TRY(upload(c, zk, c->zkh.data(), sizeof(ZoneK) * n));
-    OFX_TRY(A((void**)&c->zcells, sizeof(int) * (n + 1)));
-    OFX_TRY(upload(c, c->zcells, cellStart, sizeof(int) * (n + 1)));
-    OFX_TRY(A((void**)&c->d.norms, sizeof(double) * 6 * 512 * (size_t)n));
+    OFX_TRY(upload(c, nm.zcell, zcell.data(), sizeof(int) * T));
+    OFX_TRY(upload(c, nm.zface, zface.data(), sizeof(int) * F));
+    OFX_TRY(upload(c, nm.zwall, zwall.data(), sizeof(int) * (n + 1)));
+    OFX_TRY(upload(c, zk, zkh.data(), sizeof(ZoneK) * n));
+    OFX_TRY(A((void**)&zcells, sizeof(int) * (n + 1)));
+    OFX_TRY(upload(c, zcells, cellStart, sizeof(int) * (n + 1)));
+    OFX_TRY(A((void**)&nd.norms, sizeof(double) * 6 * 512 * (size_t)n));
     OFX_TRY(host_sums(c, n));
-    m.zk = zk;
     // per-zone reduction slots (both parities; the min quantity starts at LARGE) and results
-    DevFields& d = c->d;
-    OFX_TRY(alloc_bytes(c, (void**)&d.slots, sizeof(unsigned long long) * 2 * (size_t)n * RQ_N * NSLOT));
+    OFX_TRY(A((void**)&nd.slots, sizeof(unsigned long long) * 2 * (size_t)n * RQ_N * NSLOT));
     for (int p = 0; p < 2; ++p)
         for (int z = 0; z < n; ++z)
-            k_fill_field<<<1, 64, 0, c->stream>>>(reinterpret_cast<double*>(d.slots) +
+            k_fill_field<<<1, 64, 0, c->stream>>>(reinterpret_cast<double*>(nd.slots) +
                                                       (((size_t)p * n + z) * RQ_N + RQ_DTMIN) * NSLOT, NSLOT, LARGE);
     OFX_HIP(hipGetLastError());
-    OFX_TRY(A((void**)&d.zred, sizeof(double) * (size_t)n * RQ_N));
+    OFX_TRY(A((void**)&nd.zred, sizeof(double) * (size_t)n * RQ_N));
+    OFX_HIP(hipStreamSynchronize(c->stream));
+    nm.zk = zk;
+    nm.nz = n;
+    m = nm;
+    c->d = nd;
+    c->zcells = zcells;
+    c->zkh = std::move(zkh);
     c->par_dt = c->par_lim = c->par_fix = 0;
     c->qext_gen = -1;
-    m.nz = n;
     c->zc.assign(cellStart, cellStart + n + 1);
     c->zb.assign(bfaceStart, bfaceStart + n + 1);
     c->zcfg.assign(cfgs, cfgs + n);
     c->dist_valid = false;  // per-zone walls from now on, computed on first use
-    OFX_HIP(hipStreamSynchronize(c->stream));
     ++c->gen;
     return 0;
 }

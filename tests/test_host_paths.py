@@ -54,6 +54,16 @@ def context(fake):
     return L, h
 
 
+def zones_set(L, h, n, cells, faces):
+    """The return code of declaring n zones of `cells` cells and `faces` boundary faces each."""
+    from oneflow_amd.config import OfxConfig
+    cfgs = (OfxConfig * n)()
+    for z in range(n):
+        cfgs[z] = config().to_c()
+    start = lambda k: (ctypes.c_int * (n + 1))(*[k * z for z in range(n)], k * n)
+    return L.ofx_zones_set(h, n, start(cells), start(faces), cfgs)
+
+
 def lines(fake, word):
     return [s for s in fake.fake_log().decode().splitlines() if s.startswith(word)]
 
@@ -169,6 +179,48 @@ def network_buffers_overlap(fake):
         kernels = lines(fake, "launch")
         assert len(kernels) == (1 if apart else 2) and "k_mlp_forward" in kernels[-1], (at, kernels)
     del m
+
+
+@scenario
+def zones_refused(fake):
+    """ofx_zones_set that fails, at whichever allocation, leaves the context with the
+    zones and the result memory it had: norms and forces still go somewhere."""
+    from oneflow_amd import meshgen
+    from oneflow_amd.solver import OfxNorms
+    parts = 140
+    one = meshgen.box2d(3, 2)
+    g = meshgen.concat_grids([one] * parts)[0]
+    cells, faces = one.n_cells, one.n_bfaces
+    for kernel, arg in (("k_norm_partial", 2), ("k_norm_final", 1), ("k_norm_final", 2), ("k_aero", 3)):
+        fake.fake_watch(kernel.encode(), arg)
+    out, forces = (OfxNorms * parts)(), (ctypes.c_double * (4 * parts))()
+    for before in (1, 2, 70):  # zones when the refused call comes
+        n = {"hipMalloc": 0, "hipHostMalloc": 0}
+        for fn in n:
+            k = 0
+            while True:
+                L, h = context(fake)
+                c = config().to_c()
+                assert upload(L, h, g) == 0 and L.ofx_config_set(h, ctypes.byref(c)) == 0
+                if before > 1:
+                    assert zones_set(L, h, before, cells * parts // before, faces * parts // before) == 0
+                k += 1
+                fake.fake_fail(fn.encode(), k)
+                rc = zones_set(L, h, parts, cells, faces)
+                fake.fake_fail(fn.encode(), 0)
+                fake.fake_clear()
+                assert L.ofx_zones_norms(h, out) == 0 and L.ofx_zones_aero(h, forces) == 0
+                assert L.ofx_init_freestream(h) == 0
+                now = parts if rc == 0 else before
+                sizes = [int(s.split()[1]) for s in lines(fake, "arg")]
+                want = [6 * 512 * 8 * now, 6 * 512 * 8 * now, 6 * 8 * now, 6 * 8 * now]
+                assert len(sizes) == 4 and all(a >= b for a, b in zip(sizes, want)), (before, fn, k, rc, sizes, want)
+                L.ofx_ctx_destroy(h)
+                assert fake.fake_held() == 0
+                if rc == 0:
+                    break
+                n[fn] += 1
+        assert n["hipMalloc"] >= 7 and n["hipHostMalloc"] == 1, n
 
 
 @pytest.mark.parametrize("name", list(SCENARIOS))
