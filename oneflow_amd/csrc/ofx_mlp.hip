@@ -19,7 +19,6 @@
 
 #include <condition_variable>
 #include <mutex>
-#include <system_error>
 #include <thread>
 
 namespace ofx {
@@ -982,11 +981,13 @@ int forward_piped(ofx_mlp* n, const float* x, int nsamp, float* y) {
     const int np = (nsamp + PIPE_PIECE - 1) / PIPE_PIECE;
     if (!n->out_stream && hipStreamCreateWithFlags(&n->out_stream, hipStreamNonBlocking) != hipSuccess) {
         n->out_stream = nullptr;
+        (void)hipGetLastError();  // the caller goes on without
         return OFX_ESTATE;
     }
     for (int p = 0; p < np; ++p)
         if (!n->out_ready[p] && hipEventCreateWithFlags(&n->out_ready[p], hipEventDisableTiming) != hipSuccess) {
             n->out_ready[p] = nullptr;
+            (void)hipGetLastError();
             return OFX_ESTATE;
         }
     std::mutex mu;
@@ -1001,7 +1002,7 @@ int forward_piped(ofx_mlp* n, const float* x, int nsamp, float* y) {
             {
                 std::unique_lock<std::mutex> lock(mu);
                 cv.wait(lock, [&] { return launched > p || failed; });
-                if (launched <= p) return;
+                if (launched <= p) break;
             }
             const size_t o = (size_t)p * PIPE_PIECE * NOUT;
             out = hipStreamWaitEvent(n->out_stream, n->out_ready[p], 0);
@@ -1009,12 +1010,14 @@ int forward_piped(ofx_mlp* n, const float* x, int nsamp, float* y) {
                 out = hipMemcpyAsync(y + o, n->io_y + o, sizeof(float) * (size_t)count(p) * NOUT, hipMemcpyDeviceToHost,
                                      n->out_stream);
         }
-        if (out == hipSuccess) out = hipStreamSynchronize(n->out_stream);
+        const hipError_t done = hipStreamSynchronize(n->out_stream);  // (also after an error: y is the caller's again)
+        if (out == hipSuccess) out = done;
+        (void)hipGetLastError();  // reported by the caller's thread
     };
     std::thread worker;
     try {
         worker = std::thread(outputs);
-    } catch (const std::system_error&) {
+    } catch (...) {  // no thread, or no memory for one
         return OFX_ESTATE;
     }
     int rc = 0;
@@ -1034,7 +1037,10 @@ int forward_piped(ofx_mlp* n, const float* x, int nsamp, float* y) {
     }
     worker.join();
     if (hipStreamSynchronize(n->stream) != hipSuccess || out != hipSuccess) rc = OFX_EHIP;
-    if (rc == OFX_EHIP) set_error("mlp_forward: HIP error");
+    if (rc == OFX_EHIP) {
+        (void)hipGetLastError();  // reported here
+        set_error("mlp_forward: HIP error");
+    }
     return rc;
 }
 

@@ -223,6 +223,30 @@ def zones_refused(fake):
         assert n["hipMalloc"] >= 7 and n["hipHostMalloc"] == 1, n
 
 
+@scenario
+def piped_forward_fails(fake):
+    """The piped forward pass without a second stream, or with a copy that fails
+    midway: it falls back, or reports the error with nothing left in flight to the
+    caller's outputs, and the next call succeeds."""
+    from oneflow_amd.mlp import NIN, NOUT, Mlp, _fp
+    n = 1 << 19
+    x, y = np.zeros((n, NIN), np.float32), np.zeros((n, NOUT), np.float32)
+    m = Mlp(seed=3)
+    fake.fake_fail(b"hipStreamCreateWithFlags", 1)
+    assert m._L.ofx_mlp_forward(m.h, _fp(x), n, _fp(y)) == 0, m._L.ofx_last_error()
+    for k in range(1, 10):
+        fake.fake_clear()
+        fake.fake_fail(b"hipMemcpyAsync", k)
+        rc = m._L.ofx_mlp_forward(m.h, _fp(x), n, _fp(y))
+        fake.fake_fail(b"hipMemcpyAsync", 0)
+        work = [s for s in fake.fake_log().decode().splitlines() if s.split()[0] in ("copy", "sync")]
+        assert (rc != 0) == (k <= 8), (k, rc)
+        for st in {s.split()[1] for s in work}:
+            assert [s for s in work if s.split()[1] == st][-1] == "sync " + st, (k, st, work)
+        assert m._L.ofx_mlp_forward(m.h, _fp(x), n, _fp(y)) == 0, (k, m._L.ofx_last_error())
+    del m
+
+
 @pytest.mark.parametrize("name", list(SCENARIOS))
 def test_host_path(name, tmp_path):
     if not shutil.which("g++"):
