@@ -312,10 +312,13 @@ int ofx_get_kernel_variant(ofx_ctx* ctx, int kernel, int* variant);
 
 /* Autotuner (no counterpart in the reference): times the NS face kernel for
  * each face tile and split, the gather and both gradients for each variant,
- * and the SA residual for each SA face tile and geometry variant on the current state (each the
- * median of five timings of `iters` launches), keeps the fastest, and
- * reports the face tiles in chosen2[0..1] (may be NULL).
- * Leaves res / turbres as one evaluation of the current state. */
+ * and the SA residual for each SA face tile and geometry variant on the
+ * current state (each the median of five timings of `iters` launches), keeps
+ * the fastest, and reports the face tiles in chosen2[0..1] (may be NULL).
+ * Where a full step evaluates both gradients in one kernel (LU-SGS with SA,
+ * cells of at most 4 faces in 2-D, 5 in 3-D) it takes variant 1 of both, which
+ * that kernel needs.  Leaves res / turbres as one evaluation of the current
+ * state. */
 int ofx_autotune(ofx_ctx* ctx, int iters, int* chosen2);
 
 /* Batched cases (the reference solves zones one after another,

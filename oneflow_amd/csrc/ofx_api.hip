@@ -739,25 +739,26 @@ int ofx_autotune(ofx_ctx* c, int iters, int* chosen2) {
         if (ms < best) { best = ms; pick = v; }
     }
     c->gather_variant = pick;
-    // the NS gradient's face terms: by face id or the per-entry copies (part 0)
-    best = 1e300;
-    pick = c->grad_variant;
-    for (int v = 0; v < 2; ++v) {
-        c->grad_variant = v;
-        OFX_TRY(median_ms(c, 0, iters, &ms));
-        if (ms < best) { best = ms; pick = v; }
-    }
-    c->grad_variant = pick;
-    if (c->k.vismodel == 3) {
-        // the same choice for the SA gradient (part 6)
-        best = 1e300;
-        pick = c->sagrad_variant;
+    // The gradients' face terms, by face id or the per-entry copies (parts 0 and 6).
+    // A full LU-SGS step with SA evaluates both gradients in one kernel, which reads
+    // the copies; timed one by one they would miss what that saves.
+    const bool together = c->cfg.time_integral != 1 && c->k.vismodel == 3 &&
+                          c->m.maxFacesPerCell <= sa_early_faces(c->m.dim);
+    auto gradient = [&](int& variant, int part) -> int {
+        if (together) { variant = 1; return 0; }
+        double best = 1e300;
+        int pick = variant;
         for (int v = 0; v < 2; ++v) {
-            c->sagrad_variant = v;
-            OFX_TRY(median_ms(c, 6, iters, &ms));
+            variant = v;
+            OFX_TRY(median_ms(c, part, iters, &ms));
             if (ms < best) { best = ms; pick = v; }
         }
-        c->sagrad_variant = pick;
+        variant = pick;
+        return 0;
+    };
+    OFX_TRY(gradient(c->grad_variant, 0));
+    if (c->k.vismodel == 3) {
+        OFX_TRY(gradient(c->sagrad_variant, 6));
         best = 1e300;
         pick = c->saface_tb;
         for (int t : cand) {

@@ -262,9 +262,8 @@ namespace ofx {
 // would not fit the registers (222 of 256 without it in 3-D).
 constexpr int sa_early_faces(int dim) { return dim == 2 ? 4 : 5; }
 inline bool sa_early_ok(const ofx_ctx* c) {
-    const int mf = c->m.maxFacesPerCell;
     return c->k.vismodel == 3 && c->grad_variant == 1 && c->sagrad_variant == 1 &&
-           (c->m.dim == 2 ? mf <= 4 : mf <= 5);
+           c->m.maxFacesPerCell <= sa_early_faces(c->m.dim);
 }
 // Threads per block of a face kernel over F faces.  256 unless that leaves
 // fewer than two blocks per CU: 64 then spreads the faces over all of them

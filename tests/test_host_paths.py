@@ -247,6 +247,32 @@ def piped_forward_fails(fake):
     del m
 
 
+@scenario
+def autotune_keeps_the_fused_gradients(fake):
+    """Gradient kernels timed one by one, the form by face id a little faster: a full
+    LU-SGS step keeps the form that evaluates both gradients in one kernel, which no
+    such timing covers; a multi-stage run, which has no such kernel, takes the
+    faster ones."""
+    for k in (b"k_ns_gradILi2ELi4ELin1ELb0", b"k_ns_gradILi2ELi4ELi0ELb0", b"k_sa_gradILi2ELi4ELb0"):
+        fake.fake_cost(k, 1.0)
+    for k in (b"k_ns_grad", b"k_sa_grad"):
+        fake.fake_cost(k, 1.01)
+    for kw, fused in ((dict(), True), (dict(time_integral=1, rk_stage=3), False), (dict(vismodel=1), False)):
+        L, h = context(fake)
+        c = config(**kw).to_c()
+        assert upload(L, h, mesh("coloured")) == 0 and L.ofx_config_set(h, ctypes.byref(c)) == 0
+        assert L.ofx_autotune(h, 1, None) == 0
+        v = [ctypes.c_int() for _ in range(2)]
+        for x, kernel in zip(v, (0, 5)):
+            assert L.ofx_get_kernel_variant(h, kernel, ctypes.byref(x)) == 0
+        sa = kw.get("vismodel", 3) == 3
+        assert [x.value for x in v] == [int(fused), int(fused or not sa)], (kw, [x.value for x in v])
+        fake.fake_clear()
+        assert L.ofx_iterate(h, 1, 1, None) == 0
+        assert any("k_sa_grad_boundary" in s for s in lines(fake, "launch")) == fused
+        L.ofx_ctx_destroy(h)
+
+
 @pytest.mark.parametrize("name", list(SCENARIOS))
 def test_host_path(name, tmp_path):
     if not shutil.which("g++"):
