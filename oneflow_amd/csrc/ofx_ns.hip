@@ -1340,9 +1340,8 @@ int norms(ofx_ctx* c, ofx_norms* out, bool zones) {
     return 0;
 }
 
-// CalcAeroForce per wall face (codes/force/src/AeroForceTask.cpp:186-440), the
-// sum in face order on one thread as the reference loops.
-// Pressure and viscous force of wall face f and its pressure coefficient
+// CalcAeroForce (codes/force/src/AeroForceTask.cpp:186-440):
+// pressure and viscous force of wall face f and its pressure coefficient
 // (CalcAeroForce's face loop, codes/force/src/AeroForceTask.cpp:365-424, with
 // Stress::CalcForce, codes/solver/src/Stress.cpp).  bcdq* = owner gradient.
 __device__ __forceinline__ void wall_face_force(const DevMesh& m, const DevFields& d, const Consts& k, int f,
