@@ -42,10 +42,10 @@
 // operations, the division), 0.6-1 us where levels are wider than a round or
 // cells have three dependencies, and ~2 us per range the chain crosses.
 // Measured, lower + upper sweep with the preparation, NS / SA in us:
-//   RAE2822, 23,552 cells, 431 levels:      585 / 351 (one 1024-thread workgroup
+//   RAE2822, 23,552 cells, 431 levels:      577 / 352 (one 1024-thread workgroup
 //     walking all levels with a barrier between them: 9564 / 1188)
-//   O-grid, 120,832 cells, 747 levels:     1380 / 656 (18645 / 2661)
-//   plate, 960 cells, 63 levels:             82 / 58 (a launch per level: 862 / 474)
+//   O-grid, 120,832 cells, 747 levels:     1355 / 655 (18645 / 2661)
+//   plate, 960 cells, 63 levels:             80 / 58 (a launch per level: 862 / 474)
 #include <algorithm>
 #include <memory>
 #include <new>
