@@ -45,7 +45,7 @@
 //   RAE2822, 23,552 cells, 431 levels:      577 / 352 (one 1024-thread workgroup
 //     walking all levels with a barrier between them: 9564 / 1188)
 //   O-grid, 120,832 cells, 747 levels:     1355 / 655 (18645 / 2661)
-//   plate, 960 cells, 63 levels:             80 / 58 (a launch per level: 862 / 474)
+//   plate, 960 cells, 63 levels:             80 (a launch per level: 862)
 #include <algorithm>
 #include <memory>
 #include <new>
